@@ -13,7 +13,7 @@ namespace emc {
 
 // Lanes along pixels (neighbouring pixels hit neighbouring voxels), transpose through LDS,
 // store with lanes along orientations (coalesced rows of logW). u_r (max_prob.c:36-38) sums W
-// over mask < 1. The FP64 model is interpolated as slice_gen3d does (slice_value_flat); the
+// over mask < 1. The FP64 model is interpolated as slice_gen3d does (slice_value); the
 // FP32 copy (halo bricks, copy_f32_brick_kernel) in FP32 from an FP32 rotation
 // (slice_value_f32h).
 // elements of one mode's volume: size^3 for the FP64 model, the brick grid for the FP32 copy
@@ -76,7 +76,7 @@ __device__ __forceinline__ void expand_block(
                         slice_value_f32h(mdl, (int)size, nb, &sh.rot[rr * 9], qf0, qf1, qf2, crf, (float)center);
                     sh.tile[lane][rr] = sh.pad[rr] ? 1.f : v;
                 } else {
-                    const double v = slice_value_flat(mdl, size, &sh.rot[rr * 9], q0, q1, q2, cr, center);
+                    const double v = slice_value(mdl, size, &sh.rot[rr * 9], q0, q1, q2, cr, center);
                     sh.tile[lane][rr] = sh.pad[rr] ? 1. : v;
                 }
             }

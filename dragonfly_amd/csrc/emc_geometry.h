@@ -36,49 +36,31 @@ __device__ __forceinline__ bool locate(const double *rot, double q0, double q1, 
     return true;
 }
 
-// Interpolated model value times corr, DBL_MIN outside the grid (model.c:35-57).
+// Two neighbouring voxels along z, read with one 16-byte load from any 8-byte boundary.
+typedef double VoxelPair __attribute__((ext_vector_type(2), aligned(8)));
+
+// Interpolated model value times corr, DBL_MIN outside the grid (model.c:35-57). No branch
+// around the loads: a pixel outside the grid reads the corners of cell (0, 0, 0) and returns
+// DBL_MIN, so the loads of several calls can be in flight at once. The reference wraps the far
+// corner, (x + 1) % size, but cells stop at size - 2, so the wrap never happens: the far
+// corners are at fixed distances from the near one and the two corners of each z edge are one
+// 16-byte load. Without the three 64-bit remainders and four of the eight loads the FP64
+// expand of 25,680 orientations x 66,820 pixels on 251^3 takes 16.0 ms instead of 19.4.
 __device__ __forceinline__ double slice_value(const double *__restrict__ model, long size,
                                               const double *rot, double q0, double q1, double q2,
                                               double corr, double center) {
-    Cell c;
-    if (!locate(rot, q0, q1, q2, center, size, c)) return DBL_MIN;
-    const long s2 = size * size;
-    const long x1 = (c.x + 1) % size, y1 = (c.y + 1) % size, z1 = (c.z + 1) % size;
-    const long cx0 = c.x, cy0 = c.y, cz0 = c.z;
-    const double cx = 1. - c.fx, cy = 1. - c.fy, cz = 1. - c.fz;
-    const double fx = c.fx, fy = c.fy, fz = c.fz;
-    double v = cx * cy * cz * model[cx0 * s2 + cy0 * size + cz0] +
-               cx * cy * fz * model[cx0 * s2 + cy0 * size + z1] +
-               cx * fy * cz * model[cx0 * s2 + y1 * size + cz0] +
-               cx * fy * fz * model[cx0 * s2 + y1 * size + z1] +
-               fx * cy * cz * model[x1 * s2 + cy0 * size + cz0] +
-               fx * cy * fz * model[x1 * s2 + cy0 * size + z1] +
-               fx * fy * cz * model[x1 * s2 + y1 * size + cz0] +
-               fx * fy * fz * model[x1 * s2 + y1 * size + z1];
-    return v * corr;
-}
-
-// slice_value without a branch around the loads: a pixel outside the grid reads the corners of
-// cell (0, 0, 0) and returns DBL_MIN, so the eight loads of several calls can be in flight at
-// once. The value is the same as slice_value's.
-__device__ __forceinline__ double slice_value_flat(const double *__restrict__ model, long size,
-                                                   const double *rot, double q0, double q1, double q2,
-                                                   double corr, double center) {
+    if (size < 2) return DBL_MIN;  // no cell at all
     Cell c{0, 0, 0, 0., 0., 0.};
     const bool ok = locate(rot, q0, q1, q2, center, size, c);
-    const long s2 = size * size;
-    const long cx0 = ok ? c.x : 0, cy0 = ok ? c.y : 0, cz0 = ok ? c.z : 0;
-    const long x1 = (cx0 + 1) % size, y1 = (cy0 + 1) % size, z1 = (cz0 + 1) % size;
+    const int sz = (int)size;
+    const double *__restrict__ m = model + (ok ? (long)(c.x * sz + c.y) * sz + c.z : 0);
+    const long s2 = (long)sz * sz;
+    const VoxelPair m00 = *(const VoxelPair *)m, m01 = *(const VoxelPair *)(m + sz);
+    const VoxelPair m10 = *(const VoxelPair *)(m + s2), m11 = *(const VoxelPair *)(m + s2 + sz);
     const double cx = 1. - c.fx, cy = 1. - c.fy, cz = 1. - c.fz;
     const double fx = c.fx, fy = c.fy, fz = c.fz;
-    const double v = cx * cy * cz * model[cx0 * s2 + cy0 * size + cz0] +
-                     cx * cy * fz * model[cx0 * s2 + cy0 * size + z1] +
-                     cx * fy * cz * model[cx0 * s2 + y1 * size + cz0] +
-                     cx * fy * fz * model[cx0 * s2 + y1 * size + z1] +
-                     fx * cy * cz * model[x1 * s2 + cy0 * size + cz0] +
-                     fx * cy * fz * model[x1 * s2 + cy0 * size + z1] +
-                     fx * fy * cz * model[x1 * s2 + y1 * size + cz0] +
-                     fx * fy * fz * model[x1 * s2 + y1 * size + z1];
+    const double v = cx * cy * cz * m00.x + cx * cy * fz * m00.y + cx * fy * cz * m01.x + cx * fy * fz * m01.y +
+                     fx * cy * cz * m10.x + fx * cy * fz * m10.y + fx * fy * cz * m11.x + fx * fy * fz * m11.y;
     return ok ? v * corr : DBL_MIN;
 }
 
