@@ -753,7 +753,6 @@ int merge_chunk(const emc_engine *e, const emc_engine::BrickChunk &bc, const dou
     if ((view32 || nzmask) && (!do_model || do_weight))
         return fail(EMC_E_STATE, "internal: an FP32 or masked view merges the model only");
     if (view32) {
-        // an FP32 view: FP32 brick sums
         emc::launch_merge_model_f32(e->stream, bc.units.p, bc.num_units, bc.list.p, bc.lmask.p, rots, bc.r0, num_valid,
                                     view32, psum, all_on, e->qvals.p, e->corr.p, e->mask.p, e->num_pix, e->size,
                                     (e->num_pix + 63) / 64, nbx, e->model2.p, nzmask);
@@ -763,7 +762,7 @@ int merge_chunk(const emc_engine *e, const emc_engine::BrickChunk &bc, const dou
                              view, psum,
                              all_on, e->qvals.p, e->corr.p, e->mask.p, e->num_pix, e->size,
                              (e->num_pix + 63) / 64, nbx, e->model2.p, e->weight.p, do_model, do_weight,
-                             e->precision != 0, gate, nzmask);  // reduced-precision modes sum bricks in FP32
+                             gate, nzmask);
     return 0;
 }
 
