@@ -2756,7 +2756,7 @@ int emc_maximize(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *stats
                 return fail(EMC_E_STATE, "likelihood product: shape does not fit the tiles");
         } else if (g32) {
             emc::launch_likelihood(s, e->logw32.p, Cc, P, e->lik_off.p, e->lik_pix.p, e->lik_cnt.p,
-                                   e->blacklist.p, N, e->R.p, r0, e->lik_tiles, e->lik_unroll);
+                                   e->blacklist.p, N, e->R.p, r0, e->lik_unroll, e->lik_xcd);
         } else if (bgp) {
             emc::launch_likelihood_bg(s, e->logw.p, Cc, P, e->lik_off.p, e->lik_pix.p, e->lik_cnt.p, e->blacklist.p,
                                       N, e->scale.p, e->bgscale.p, e->bg.p, e->R.p, r0);

@@ -25,7 +25,7 @@ void launch_copy_f32_brick(hipStream_t s, const double *in, long size, int modes
 void launch_to_f32(hipStream_t s, const double *P, int num_data, int r0, int C, float *out);
 void launch_likelihood(hipStream_t s, const float *logw, int C, int num_pix, const long *off,
                        const int *pix, const double *cnt, const uint8_t *blacklist, int num_data,
-                       double *G, int r0, int tiles, int unroll);
+                       double *G, int r0, int unroll, int xcd_order);
 // Likelihood over X pixel ranges (lists split per range, off8[d * (X + 1) + x]) into partials
 // part[X][C / 64][num_data][64], then added in range order into the chunk's tiles of G.
 void launch_likelihood_split(hipStream_t s, const double *logw, int C, int num_pix, const long *off8, int X,

@@ -17,6 +17,7 @@
 
 #include "emc_common.h"
 #include "emc_expand.h"
+#include "emc_gather.h"
 #include "emc_geometry.h"
 #include "emc_kernels.h"
 
@@ -104,40 +105,72 @@ __global__ __launch_bounds__(kBlock) void rescale_kernel(const double *__restric
     if (threadIdx.x == 0) scalars[0] = mean_count / s[0] * modes;
 }
 
+// Frame group and orientation tile of a block in the XCD-aware 1-D order: workgroups go
+// round-robin to the kNumXcd XCDs, which form groups of G (1, 2, 4 or 8); group g takes
+// orientation tiles g, g + kNumXcd / G, ... one at a time, its G members splitting the nfg frame
+// groups, so each L2 sees the rows of one log W tile and kNumXcd / G tiles are live chip-wide.
+__device__ __forceinline__ void xcd_tile(int G, int nfg, int &fg, int &tb) {
+    const int ngrp = kNumXcd / G, nfgG = (nfg + G - 1) / G;
+    const int x = blockIdx.x % kNumXcd, j = blockIdx.x / kNumXcd;
+    tb = x / G + ngrp * (j / nfgG);
+    fg = (j % nfgG) * G + x % G;
+}
+
 // ---- likelihood: G_dr = sum_t K_dt log W_rt over one frame's photons (mask < 1) ------------
-// One wavefront = one frame x NT*64 orientations; the frame's (pixel, count) list is read
-// with scalar loads (wave-uniform) and each photon costs NT 512-byte row reads of logW.
-// Row loads of several photons are issued before the additions, which stay in list order.
-template <int NT, int U, typename T>
-__global__ __launch_bounds__(kBlock) void likelihood_kernel(
-    const T *__restrict__ logw, int C, size_t tsW, const long *__restrict__ off,
-    const int *__restrict__ pix, const double *__restrict__ cnt,
-    const uint8_t *__restrict__ blacklist, int num_data, double *__restrict__ G, size_t tsG,
-    int r0, const int *__restrict__ fmap, int xcd_order) {
+// One wavefront = one frame x one log W tile of kW orientations (64 FP64, 128 FP32: 512-byte
+// rows), gathered 16 bytes a lane and two photons at a time (emc_gather.h); writes the 64-wide
+// tile-major G of orientations < C. fmap (nullable): the frame whose photons row d holds.
+template <typename T, int kW, int U>
+__global__ __launch_bounds__(kBlock) void likelihood_rows_kernel(
+    const T *__restrict__ logw, int C, size_t tsW, const long *__restrict__ off, const int *__restrict__ pix,
+    const double *__restrict__ cnt, const uint8_t *__restrict__ blacklist, int num_data, double *__restrict__ G,
+    size_t tsG, int r0, const int *__restrict__ fmap, int xcd_order) {
+    constexpr int n = RowVec<T>::n, LR = kW / n;
+    __shared__ RowEntry s_list[kWavesPerBlock][64];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     int fg = blockIdx.x, tb = blockIdx.y;
     if (xcd_order) {
-        // 1-D grid, XCD-aware: workgroups go round-robin to the kNumXcd XCDs. The XCDs form
-        // groups of G = xcd_order (1, 2, 4 or 8); group g takes orientation tiles
-        // g, g + kNumXcd / G, ... one at a time, its G members splitting the frames, so each
-        // L2 sees the rows of one log W tile and kNumXcd / G tiles are live chip-wide
-        const int G = xcd_order, ngrp = kNumXcd / G;
-        const int nfg = (num_data + kWavesPerBlock - 1) / kWavesPerBlock, nfgG = (nfg + G - 1) / G;
-        const int x = blockIdx.x % kNumXcd, j = blockIdx.x / kNumXcd;
-        tb = x / G + ngrp * (j / nfgG);
-        fg = (j % nfgG) * G + x % G;
+        const int nfg = (num_data + kWavesPerBlock - 1) / kWavesPerBlock;
+        xcd_tile(xcd_order, nfg, fg, tb);
+        if ((long)tb * kW >= C || fg >= nfg) return;
+    }
+    const int d = fg * kWavesPerBlock + wave;
+    if (d >= num_data) return;
+    const int fd = fmap ? fmap[d] : d;
+    if (blacklist[fd]) return;
+    double acc[n] = {};
+    gather_rows<T, kW, LR, U>(logw + (size_t)tb * tsW + (lane % LR) * n, pix, cnt, off[fd], off[fd + 1], s_list[wave],
+                              lane, acc);
+    const int c = tb * kW + lane * n;
+    if (lane < LR && c < C)
+        store_sums<n>(G + (size_t)((r0 + c) / kRTile) * tsG + (size_t)d * kRTile + (c % kRTile), acc);
+}
+
+// The same with NT (2 or 4) 64-orientation tiles per wavefront (option lik_tiles): the frame's
+// (pixel, count) list is read with scalar loads and each photon costs NT 512-byte row reads.
+template <int NT, int U>
+__global__ __launch_bounds__(kBlock) void likelihood_kernel(
+    const double *__restrict__ logw, int C, size_t tsW, const long *__restrict__ off,
+    const int *__restrict__ pix, const double *__restrict__ cnt,
+    const uint8_t *__restrict__ blacklist, int num_data, double *__restrict__ G, size_t tsG,
+    int r0, int xcd_order) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    int fg = blockIdx.x, tb = blockIdx.y;
+    if (xcd_order) {
+        const int nfg = (num_data + kWavesPerBlock - 1) / kWavesPerBlock;
+        xcd_tile(xcd_order, nfg, fg, tb);
         if (tb * (kRTile * NT) >= C || fg >= nfg) return;
     }
     const int d = fg * kWavesPerBlock + wave;
     if (d >= num_data) return;
-    const int fd = fmap ? fmap[d] : d;  // frame whose photons row d holds
-    if (blacklist[fd]) return;
+    if (blacklist[d]) return;
     const int c0 = tb * (kRTile * NT);
     const int nt = min(NT, (C - c0) / kRTile);
-    const T *__restrict__ col = logw + (size_t)(c0 >> 6) * tsW + lane;
-    const long k1 = off[fd + 1];
-    long k = off[fd];
+    const double *__restrict__ col = logw + (size_t)(c0 >> 6) * tsW + lane;
+    const long k1 = off[d + 1];
+    long k = off[d];
     double acc[NT];
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[j] = 0.;
@@ -147,7 +180,7 @@ __global__ __launch_bounds__(kBlock) void likelihood_kernel(
         for (int u = 0; u < U; ++u) {
             const size_t row = (size_t)pix[k + u] * kRTile;
 #pragma unroll
-            for (int j = 0; j < NT; ++j) v[u][j] = (j < nt) ? (double)col[row + tsW * j] : 0.;
+            for (int j = 0; j < NT; ++j) v[u][j] = (j < nt) ? col[row + tsW * j] : 0.;
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -158,7 +191,7 @@ __global__ __launch_bounds__(kBlock) void likelihood_kernel(
         const size_t row = (size_t)pix[k] * kRTile;
 #pragma unroll
         for (int j = 0; j < NT; ++j)
-            if (j < nt) acc[j] += cnt[k] * (double)col[row + tsW * j];
+            if (j < nt) acc[j] += cnt[k] * col[row + tsW * j];
     }
 #pragma unroll
     for (int j = 0; j < NT; ++j)
@@ -1127,47 +1160,6 @@ void launch_to_f32(hipStream_t s, const double *P, int num_data, int r0, int C, 
     to_f32_w128_kernel<<<grid_cap(cdiv(n, 256)), 256, 0, s>>>(P, num_data, r0, C, out);
 }
 
-// Likelihood with FP32 log W in 128-wide tiles: one wavefront = one frame x 128 orientations,
-// every lane reads two neighbouring orientations (one 8-byte load, 512 bytes per row) and
-// keeps two FP64 sums; writes the 64-wide tile-major G of orientations < C.
-template <int U>
-__global__ __launch_bounds__(kBlock) void likelihood_w128_kernel(
-    const float *__restrict__ logw, int C, size_t tsW, const long *__restrict__ off,
-    const int *__restrict__ pix, const double *__restrict__ cnt, const uint8_t *__restrict__ blacklist,
-    int num_data, double *__restrict__ G, size_t tsG, int r0, const int *__restrict__ fmap) {
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    const int d = blockIdx.x * kWavesPerBlock + wave;
-    if (d >= num_data) return;
-    const int fd = fmap ? fmap[d] : d;  // frame whose photons row d holds
-    if (blacklist[fd]) return;
-    const int tile = blockIdx.y;
-    const float2 *__restrict__ col = reinterpret_cast<const float2 *>(logw + (size_t)tile * tsW) + lane;
-    const long k1 = off[fd + 1];
-    long k = off[fd];
-    double a0 = 0., a1 = 0.;
-    for (; k + U <= k1; k += U) {
-        float2 v[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = col[(size_t)pix[k + u] * 64];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            a0 += cnt[k + u] * (double)v[u].x;
-            a1 += cnt[k + u] * (double)v[u].y;
-        }
-    }
-    for (; k < k1; ++k) {
-        const float2 v = col[(size_t)pix[k] * 64];
-        a0 += cnt[k] * (double)v.x;
-        a1 += cnt[k] * (double)v.y;
-    }
-    const int c = tile * 128 + 2 * lane;
-    if (c < C) {
-        double2 *dst = reinterpret_cast<double2 *>(G + (size_t)((r0 + c) / kRTile) * tsG + (size_t)d * kRTile + (c % kRTile));
-        *dst = make_double2(a0, a1);
-    }
-}
-
 // Frame-partitioned tomogram over an FP32 posterior in 128-wide tiles (see to_f32_w128_kernel):
 // each lane gathers two orientations per photon; partial sums in FP64, written in the 64-wide
 // tile-major partial layout of tomogram_part_kernel.
@@ -1221,38 +1213,50 @@ void launch_rescale(hipStream_t s, const double *quats, const double *u, int num
     rescale_kernel<<<1, kBlock, 0, s>>>(quats, u, num_rot, mean_count, (double)modes, scalars);
 }
 
-template <typename T>
-static void likelihood_launch(hipStream_t s, const T *logw, int C, int num_pix, const long *off,
-                              const int *pix, const double *cnt, const uint8_t *blacklist, int num_data,
-                              double *G, int r0, int tiles, int unroll, const int *fmap = nullptr,
-                              int xcd_order = 0) {
+// 1-D XCD-aware grid of a likelihood launch over gy column tiles (xcd: XCDs sharing a tile, 1,
+// 2, 4 or 8; 0, or more work-items than a grid size holds: the plain 2-D grid, xcd becomes 0)
+static dim3 likelihood_grid(int num_data, size_t gy, int &xcd) {
     const unsigned gx = cdiv(num_data, kWavesPerBlock);
-    const size_t tsW = (size_t)num_pix * kRTile, tsG = (size_t)num_data * kRTile;
-    /* XCDs sharing a tile in the 1-D order: 1, 2, 4 or 8 (0: 2-D grid) */
-    const int xg = xcd_order >= 8 ? 8 : xcd_order >= 4 ? 4 : xcd_order >= 2 ? 2 : (xcd_order > 0 ? 1 : 0);
-#define EMC_LIK(NT, U)                                                                           \
-    do {                                                                                         \
-        const size_t gy = cdiv(C, kRTile * NT);                                                  \
-        const size_t nblk = xg ? (size_t)kNumXcd * cdiv(gx, xg) * cdiv(gy, kNumXcd / xg) : 0;    \
-        /* the 1-D order needs its work-item count to fit the 32-bit grid size */                \
-        const int xo = xg && nblk * kBlock < ((size_t)1 << 32);                                  \
-        const dim3 grid = xo ? dim3((unsigned)nblk) : dim3(gx, (unsigned)gy);                    \
-        likelihood_kernel<NT, U, T><<<grid, kBlock, 0, s>>>(logw, C, tsW, off, pix, cnt, blacklist, num_data, G, \
-                                                            tsG, r0, fmap, xo ? xg : 0);        \
-    } while (0)
-    if (tiles >= 4) EMC_LIK(4, 2);
-    else if (tiles == 2) EMC_LIK(2, 4);
-    else if (unroll >= 16) EMC_LIK(1, 16);
-    else if (unroll == 4) EMC_LIK(1, 4);
-    else EMC_LIK(1, 8);
+    xcd = xcd >= 8 ? 8 : xcd >= 4 ? 4 : xcd >= 2 ? 2 : (xcd > 0 ? 1 : 0);
+    const size_t nblk = xcd ? (size_t)kNumXcd * cdiv(gx, xcd) * cdiv(gy, kNumXcd / xcd) : 0;
+    if (xcd && nblk * kBlock < ((size_t)1 << 32)) return dim3((unsigned)nblk);
+    xcd = 0;
+    return dim3(gx, (unsigned)gy);
+}
+
+// unroll: photon rows in flight per wavefront (4, 8 or 16), two of them per load instruction
+template <typename T, int kW>
+static void likelihood_rows_launch(hipStream_t s, const T *logw, int C, int num_pix, const long *off, const int *pix,
+                                   const double *cnt, const uint8_t *blacklist, int num_data, double *G, int r0,
+                                   int unroll, const int *fmap, int xcd) {
+    const size_t tsW = (size_t)num_pix * kW, tsG = (size_t)num_data * kRTile;
+    const dim3 grid = likelihood_grid(num_data, cdiv(C, kW), xcd);
+#define EMC_LIK(U)                                                                                                  \
+    likelihood_rows_kernel<T, kW, U><<<grid, kBlock, 0, s>>>(logw, C, tsW, off, pix, cnt, blacklist, num_data, G,  \
+                                                             tsG, r0, fmap, xcd)
+    if (unroll >= 16) EMC_LIK(8);
+    else if (unroll == 4) EMC_LIK(2);
+    else EMC_LIK(4);
 #undef EMC_LIK
 }
 
 void launch_likelihood(hipStream_t s, const double *logw, int C, int num_pix, const long *off,
                        const int *pix, const double *cnt, const uint8_t *blacklist, int num_data,
                        double *G, int r0, int tiles, int unroll, int xcd_order) {
-    likelihood_launch(s, logw, C, num_pix, off, pix, cnt, blacklist, num_data, G, r0, tiles, unroll, nullptr,
-                      xcd_order);
+    if (tiles < 2) {
+        likelihood_rows_launch<double, kRTile>(s, logw, C, num_pix, off, pix, cnt, blacklist, num_data, G, r0, unroll,
+                                               nullptr, xcd_order);
+        return;
+    }
+    const size_t tsW = (size_t)num_pix * kRTile, tsG = (size_t)num_data * kRTile;
+    const int nt = tiles >= 4 ? 4 : 2;
+    const dim3 grid = likelihood_grid(num_data, cdiv(C, (size_t)kRTile * nt), xcd_order);
+    if (nt == 4)
+        likelihood_kernel<4, 2><<<grid, kBlock, 0, s>>>(logw, C, tsW, off, pix, cnt, blacklist, num_data, G, tsG, r0,
+                                                        xcd_order);
+    else
+        likelihood_kernel<2, 4><<<grid, kBlock, 0, s>>>(logw, C, tsW, off, pix, cnt, blacklist, num_data, G, tsG, r0,
+                                                        xcd_order);
 }
 
 void launch_likelihood_split(hipStream_t s, const double *logw, int C, int num_pix, const long *off8, int X,
@@ -1274,34 +1278,24 @@ void launch_likelihood_split(hipStream_t s, const double *logw, int C, int num_p
 void launch_likelihood_mapped(hipStream_t s, const double *logw, int C, int num_pix, const long *off,
                               const int *pix, const double *cnt, const uint8_t *blacklist, const int *fmap,
                               int num_rows, double *G, int r0) {
-    if (num_rows > 0) likelihood_launch(s, logw, C, num_pix, off, pix, cnt, blacklist, num_rows, G, r0, 1, 8, fmap);
-}
-
-static void likelihood_w128_launch(hipStream_t s, const float *logw, int C, int num_pix, const long *off,
-                                   const int *pix, const double *cnt, const uint8_t *blacklist, int num_data,
-                                   double *G, int r0, int unroll, const int *fmap) {
-    const unsigned gx = cdiv(num_data, kWavesPerBlock);
-    const size_t tsW = (size_t)num_pix * 128, tsG = (size_t)num_data * kRTile;
-    const dim3 grid(gx, cdiv(C, 128));
-    if (unroll >= 16)
-        likelihood_w128_kernel<16><<<grid, kBlock, 0, s>>>(logw, C, tsW, off, pix, cnt, blacklist, num_data, G, tsG, r0,
-                                                           fmap);
-    else
-        likelihood_w128_kernel<8><<<grid, kBlock, 0, s>>>(logw, C, tsW, off, pix, cnt, blacklist, num_data, G, tsG, r0,
-                                                          fmap);
+    if (num_rows > 0)
+        likelihood_rows_launch<double, kRTile>(s, logw, C, num_pix, off, pix, cnt, blacklist, num_rows, G, r0, 8, fmap,
+                                               1);
 }
 
 void launch_likelihood(hipStream_t s, const float *logw, int C, int num_pix, const long *off,
                        const int *pix, const double *cnt, const uint8_t *blacklist, int num_data,
-                       double *G, int r0, int tiles, int unroll) {
-    (void)tiles;
-    likelihood_w128_launch(s, logw, C, num_pix, off, pix, cnt, blacklist, num_data, G, r0, unroll, nullptr);
+                       double *G, int r0, int unroll, int xcd_order) {
+    likelihood_rows_launch<float, 2 * kRTile>(s, logw, C, num_pix, off, pix, cnt, blacklist, num_data, G, r0, unroll,
+                                              nullptr, xcd_order);
 }
 
 void launch_likelihood_mapped(hipStream_t s, const float *logw, int C, int num_pix, const long *off,
                               const int *pix, const double *cnt, const uint8_t *blacklist, const int *fmap,
                               int num_rows, double *G, int r0) {
-    if (num_rows > 0) likelihood_w128_launch(s, logw, C, num_pix, off, pix, cnt, blacklist, num_rows, G, r0, 16, fmap);
+    if (num_rows > 0)
+        likelihood_rows_launch<float, 2 * kRTile>(s, logw, C, num_pix, off, pix, cnt, blacklist, num_rows, G, r0, 8,
+                                                  fmap, 1);
 }
 
 void launch_frame_max(hipStream_t s, double *R, int num_rot, int num_data,

@@ -23,6 +23,7 @@
 
 #include "emc_common.h"
 #include "emc_expand.h"
+#include "emc_gather.h"
 #include "emc_kernels.h"
 
 namespace emc {
@@ -66,38 +67,41 @@ __device__ __forceinline__ FrameRows frame_rows(double *R, const long *pair_off,
 
 }  // namespace
 
-// G[k][lane] = sum over the frame's photons of count * logW[tile - t0][pix][lane] for the
-// partial-frame pairs of tiles [t0, t1). Pairs are walked tile-major (tile_off / tile_pair), so
-// the waves resident at one time read rows of the same log W tile. log W is chunk-local and
-// tile-major with kW-wide tiles of type TW (64 x f64, or 128 x f32: two 64-slot tiles per row).
+// One (frame, tile) pair's 64 sums over the frame's photons of count * log W: log W tiles of
+// kW orientations (64 x f64, or 128 x f32: two 64-slot tiles per row; lt counts 64-slot tiles).
+// Called by a whole wavefront.
+template <typename T, int kW, int U>
+__device__ __forceinline__ void pair_sums(const T *__restrict__ logw, size_t tsW, int lt, const int *__restrict__ pix,
+                                          const double *__restrict__ cnt, long q0, long q1, RowEntry *s_list, int lane,
+                                          double *__restrict__ G) {
+    constexpr int n = RowVec<T>::n, LR = kRTile / n, kSub = kW / kRTile;
+    double acc[n] = {};
+    gather_rows<T, kW, LR, U>(logw + (size_t)(lt / kSub) * tsW + (lt % kSub) * kRTile + (lane % LR) * n, pix, cnt, q0, q1,
+                              s_list, lane, acc);
+    if (lane < LR) store_sums<n>(G + lane * n, acc);
+}
+
+// G[k][0..64) for the partial-frame pairs of tiles [t0, t1). Pairs are walked tile-major
+// (tile_off / tile_pair), each XCD (workgroups go to them round-robin) over its own contiguous
+// eighth of the list, so the waves resident on an XCD read rows of one log W tile through its L2
+// and no two XCDs fetch the same tile.
 template <int U, typename TW, int kW>
 __global__ __launch_bounds__(kBlock) void pair_likelihood_kernel(
     const TW *__restrict__ logw, size_t tsW, const long *__restrict__ off,
     const int *__restrict__ pix, const double *__restrict__ cnt, const int *__restrict__ pair_frame,
     const int *__restrict__ pair_tile, const long *__restrict__ tile_off, const int *__restrict__ tile_pair,
     int t0, int t1, double *__restrict__ G) {
-    constexpr int kSub = kW / kRTile;
+    __shared__ RowEntry s_list[kWavesPerBlock][64];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    const long j1 = tile_off[t1];
-    const long stride = (long)gridDim.x * kWavesPerBlock;
-    for (long j = tile_off[t0] + (long)blockIdx.x * kWavesPerBlock + wave; j < j1; j += stride) {
+    const long j0 = tile_off[t0], per = (tile_off[t1] - j0 + kNumXcd - 1) / kNumXcd;
+    const long first = j0 + (blockIdx.x % kNumXcd) * per, last = min(first + per, tile_off[t1]);
+    const long stride = (long)(gridDim.x / kNumXcd) * kWavesPerBlock;
+    for (long j = first + (long)(blockIdx.x / kNumXcd) * kWavesPerBlock + wave; j < last; j += stride) {
         const int k = tile_pair[j];
         const int d = pair_frame[k];
-        const int lt = pair_tile[k] - t0;
-        const TW *__restrict__ col = logw + (size_t)(lt / kSub) * tsW + (lt % kSub) * kRTile + lane;
-        long q = off[d];
-        const long q1 = off[d + 1];
-        double acc = 0.;
-        for (; q + U <= q1; q += U) {
-            double v[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) v[u] = (double)col[(size_t)pix[q + u] * kW];
-#pragma unroll
-            for (int u = 0; u < U; ++u) acc += cnt[q + u] * v[u];
-        }
-        for (; q < q1; ++q) acc += cnt[q] * (double)col[(size_t)pix[q] * kW];
-        G[(size_t)k * kRTile + lane] = acc;
+        pair_sums<TW, kW, U>(logw, tsW, pair_tile[k] - t0, pix, cnt, off[d], off[d + 1], s_list[wave], lane,
+                             G + (size_t)k * kRTile);
     }
 }
 
@@ -880,8 +884,8 @@ __global__ __launch_bounds__(kBlock) void fused_expand_likelihood_kernel(
     const double *__restrict__ cnt, const int *__restrict__ pair_frame, const int *__restrict__ pair_tile,
     const long *__restrict__ tile_off, const int *__restrict__ tile_pair, int t0, int ntiles,
     unsigned *__restrict__ counter, double *__restrict__ G) {
-    constexpr int kSub = kW / kRTile;
     __shared__ ExpandShared<MT> sh;
+    __shared__ RowEntry s_list[kWavesPerBlock][64];
     __shared__ int s_tile;
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -902,19 +906,8 @@ __global__ __launch_bounds__(kBlock) void fused_expand_likelihood_kernel(
         for (long j = tile_off[t0 + lt] + wave; j < j1; j += kWavesPerBlock) {
             const int kp = tile_pair[j];
             const int d = pair_frame[kp];
-            const T *__restrict__ col = logw + (size_t)(lt / kSub) * tsW + (lt % kSub) * kRTile + lane;
-            long q = off[d];
-            const long q1 = off[d + 1];
-            double acc = 0.;
-            for (; q + U <= q1; q += U) {
-                double v[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) v[u] = (double)col[(size_t)pix[q + u] * kW];
-#pragma unroll
-                for (int u = 0; u < U; ++u) acc += cnt[q + u] * v[u];
-            }
-            for (; q < q1; ++q) acc += cnt[q] * (double)col[(size_t)pix[q] * kW];
-            G[(size_t)kp * kRTile + lane] = acc;
+            pair_sums<T, kW, U>(logw, tsW, lt, pix, cnt, off[d], off[d + 1], s_list[wave], lane,
+                                G + (size_t)kp * kRTile);
         }
     }
 }
@@ -933,13 +926,13 @@ static void fused_launch(hipStream_t s, const double *rots, const MT *model, lon
         int dev = 0, cus = 0, per_cu = 0;
         (void)hipGetDevice(&dev);
         (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fused_expand_likelihood_kernel<8, T, kW, MT>,
+        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fused_expand_likelihood_kernel<4, T, kW, MT>,
                                                            kBlock, 0);
         resident = std::max(1, cus * std::max(per_cu, 1));
     }
     const unsigned grid = (unsigned)std::min(ntiles, resident);
     const int ngroups = (num_pix + pix_per_group - 1) / pix_per_group;
-    fused_expand_likelihood_kernel<8, T, kW, MT><<<grid, kBlock, 0, s>>>(
+    fused_expand_likelihood_kernel<4, T, kW, MT><<<grid, kBlock, 0, s>>>(
         rots, model, size, qvals, corr, mask, num_pix, r0, C, pix_per_group, ngroups, logw, upart, ubad, slot_rot, off,
         pix, cnt, pair_frame, pair_tile, tile_off, tile_pair, t0, ntiles, counter, G);
 }
@@ -966,12 +959,17 @@ void launch_fused_expand_likelihood(hipStream_t s, const double *rots, const flo
                                            tile_pair, t0, counter, G);
 }
 
+// grid of pair_likelihood_kernel: kNumXcd eighths of the pairs, a wave per pair (or strided)
+static unsigned pair_grid(long num_pairs) {
+    const long per = (num_pairs + kNumXcd - 1) / kNumXcd;
+    return kNumXcd * (unsigned)std::min<long>((per + kWavesPerBlock - 1) / kWavesPerBlock, kMaxStrideBlocks / kNumXcd);
+}
+
 void launch_pair_likelihood(hipStream_t s, const double *logw, int num_pix, const long *off, const int *pix,
                             const double *cnt, const int *pair_frame, const int *pair_tile, const long *tile_off,
                             const int *tile_pair, long num_pairs, int t0, int t1, double *G) {
-    const unsigned grid = stride_grid((num_pairs + kWavesPerBlock - 1) / kWavesPerBlock);
-    if (grid == 0) return;
-    pair_likelihood_kernel<8, double, kRTile><<<grid, kBlock, 0, s>>>(logw, (size_t)num_pix * kRTile, off, pix, cnt,
+    if (num_pairs <= 0) return;
+    pair_likelihood_kernel<4, double, kRTile><<<pair_grid(num_pairs), kBlock, 0, s>>>(logw, (size_t)num_pix * kRTile, off, pix, cnt,
                                                                       pair_frame, pair_tile, tile_off, tile_pair, t0,
                                                                       t1, G);
 }
@@ -979,9 +977,8 @@ void launch_pair_likelihood(hipStream_t s, const double *logw, int num_pix, cons
 void launch_pair_likelihood(hipStream_t s, const float *logw, int num_pix, const long *off, const int *pix,
                             const double *cnt, const int *pair_frame, const int *pair_tile, const long *tile_off,
                             const int *tile_pair, long num_pairs, int t0, int t1, double *G) {
-    const unsigned grid = stride_grid((num_pairs + kWavesPerBlock - 1) / kWavesPerBlock);
-    if (grid == 0) return;
-    pair_likelihood_kernel<8, float, 2 * kRTile><<<grid, kBlock, 0, s>>>(logw, (size_t)num_pix * 2 * kRTile, off, pix,
+    if (num_pairs <= 0) return;
+    pair_likelihood_kernel<4, float, 2 * kRTile><<<pair_grid(num_pairs), kBlock, 0, s>>>(logw, (size_t)num_pix * 2 * kRTile, off, pix,
                                                                          cnt, pair_frame, pair_tile, tile_off,
                                                                          tile_pair, t0, t1, G);
 }

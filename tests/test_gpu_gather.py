@@ -1,0 +1,87 @@
+"""Photon gathers at the sizes where their lists are cut: frames of every photon count around the
+64-entry stage, the two (FP32: two, and four for pairs) photon streams of a wavefront and the
+rows in flight; frame counts that leave a block's wavefronts idle; orientation counts that end
+inside a tile. Checked against the oracle: FP64 to 1e-9 as the other parity tests, FP32 log W to
+the FP32-gather tests' bars (average log-likelihood 1e-6)."""
+import numpy as np
+import pytest
+import torch  # noqa: F401  (its HIP runtime is loaded before the engine's library)
+
+import problems as P
+from dragonfly_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+COUNTS = (0, 1, 2, 3, 7, 8, 9, 15, 16, 17, 31, 33, 63, 64, 65, 66, 71, 72, 73, 127, 128, 129, 191, 200)
+
+
+def counted_problem(counts, num_rot, seed=7):
+    """The tiny geometry with frames of exactly counts[d] photon pixels (every fifth of them a
+    multi-photon pixel), and the first num_rot orientations of the num_div 2 sampling."""
+    p = P.build(P.tiny_config(num_data=len(counts)), quats=_lib.quat_gen(2)[:num_rot])
+    rng = np.random.default_rng(seed)
+    mask = p['det']['mask']
+    good = np.flatnonzero(mask < 1)
+    ones, multi, po, pm, cm = [], [], [], [], []
+    for n in counts:
+        px = rng.permutation(good)[:n]
+        m = n // 5
+        ones.append(n - m)
+        multi.append(m)
+        po.append(px[m:])
+        pm.append(px[:m])
+        cm.append(rng.integers(2, 9, m))
+    f = dict(ones=np.array(ones, 'i4'), multi=np.array(multi, 'i4'), place_ones=np.concatenate(po).astype('i4'),
+             place_multi=np.concatenate(pm).astype('i4'), count_multi=np.concatenate(cm).astype('i4'))
+    f['ones_accum'] = np.concatenate([[0], np.cumsum(ones)[:-1]]).astype('i8')
+    f['multi_accum'] = np.concatenate([[0], np.cumsum(multi)[:-1]]).astype('i8')
+    p['frames'] = f
+    fp = p['fparams']
+    fp['fcounts'] = P.frame_counts(f['ones'], f['multi'], f['place_ones'], f['place_multi'], f['count_multi'], mask)
+    fp['sum_fact'] = P.sum_log_factorials(f['multi'], f['place_multi'], f['count_multi'], mask)
+    fp['mean_count'] = fp['fcounts'].astype('f8').mean()
+    fp['beta'] = np.full(len(counts), 0.05)
+    return p
+
+
+@pytest.mark.parametrize('num_rot', (63, 129, 420))
+@pytest.mark.parametrize('unroll', (4, 8, 16))
+def test_likelihood_photon_counts(num_rot, unroll):
+    p = counted_problem(COUNTS[:len(COUNTS) - (unroll == 8)], num_rot)
+    o = P.run_oracle(p, dict(iteration=1))
+    eng = P.engine_for(p)
+    eng.set_option('lik_unroll', unroll)
+    g = P.run_engine(eng, dict(iteration=1))
+    for k in ('max_exp', 'p_norm', 'likelihood', 'prob', 'model2'):
+        assert P.rel_err(g[k], o[k]) <= 1e-9, k
+    # a frame without photons has R = log w - phi u alone, and the flat detector's two-fold symmetry
+    # gives orientations 0 and 5 the same u to rounding: its arg-max is a tie
+    seen = np.array(COUNTS[:len(g['rmax'])]) > 0
+    assert np.array_equal(g['rmax'][seen], o['rmax'][seen])
+    eng.set_precision(3)
+    h = P.run_engine(eng, dict(iteration=1))
+    assert abs(h['avg_likelihood'] / o['avg_likelihood'] - 1.) <= 1e-6
+    assert P.rel_err(h['max_exp'], o['max_exp']) <= 1e-6
+    eng.close()
+
+
+@pytest.mark.parametrize('precision', (0, 3))
+def test_pair_likelihood_photon_counts(precision):
+    """The same lists on refinement subsets (pairs of frames and 64-slot tiles) against the
+    masked full search of the engine."""
+    p = counted_problem(COUNTS, 420)
+    qc = _lib.quat_gen(1)
+    cells = _lib.voronoi_subset(qc, p['quats'])
+    rng = np.random.default_rng(3)
+    sets = [np.sort(rng.permutation(len(qc))[:1 + d % 9]).astype('i4') for d in range(len(COUNTS))]
+    off = np.concatenate([[0], np.cumsum([len(s) for s in sets])]).astype('i8')
+    out = []
+    for subset in (1, 0):
+        eng = P.engine_for(p)
+        eng.set_precision(precision)
+        eng.set_option('subset', subset)
+        eng.set_refine(len(qc), cells, off, np.concatenate(sets))
+        out.append(P.run_engine(eng, dict(iteration=1)))
+        eng.close()
+    for k in ('max_exp', 'p_norm', 'likelihood', 'prob'):
+        assert P.rel_err(out[0][k], out[1][k]) <= (1e-9 if precision == 0 else 1e-6), k
