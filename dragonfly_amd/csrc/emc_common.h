@@ -16,6 +16,7 @@ constexpr int kWavesPerBlock = kBlock / 64;
 // MI355X dispatches consecutive workgroups of a launch round-robin over its 8 XCDs, each with
 // its own L2.
 constexpr int kNumXcd = 8;
+constexpr int kNumCus = 256;
 
 // Mixed-precision product tiles (emc_mp.hip): block tile kGemmBM x kGemmBN, kGemmBK halves
 // of K per step, 8 waves; kGemmGroupM m-tiles per panel of the block order.

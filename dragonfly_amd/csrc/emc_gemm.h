@@ -243,4 +243,76 @@ __device__ __forceinline__ void gemm_for_each(size_t m0, size_t n0, const floatx
         }
 }
 
+// ---- small block tile -----------------------------------------------------------------------
+// The same product in block tiles of 64 x 64 (4 waves, one 32 x 32 MFMA tile each, two LDS
+// stages of kSmallBK elements of K), for outputs too small to give every CU a 256 x 256 tile: each
+// accumulator element sums the same products in the same order, so the values are the same.
+constexpr int kSmallTile = 64;
+constexpr int kSmallBK = 128;
+constexpr int kSmallRow = kSmallBK + kGemmLdsPad;
+constexpr size_t kSmallLdsElems = 2 * (size_t)(2 * kSmallTile) * kSmallRow;
+
+__device__ __forceinline__ GemmTile gemm_small_tile(int n_tiles) {
+    return GemmTile{(size_t)(blockIdx.x / n_tiles) * kSmallTile, (size_t)(blockIdx.x % n_tiles) * kSmallTile, true};
+}
+
+template <typename T>
+__device__ __forceinline__ void gemm_small_mainloop(const T *__restrict__ A, size_t lda, const T *__restrict__ B,
+                                                    size_t ldb, int K, size_t m0, size_t n0, T *smem,
+                                                    floatx16 &acc) {
+    typedef typename Mfma<T>::vec8 vec8;
+    constexpr int kStage = 2 * kSmallTile * kSmallRow;
+    constexpr int kChunks = kSmallBK / 8, kRowsPerPass = kBlock / kChunks, kLoads = kSmallTile / kRowsPerPass;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lrow = tid / kChunks, lchunk = (tid % kChunks) * 8;
+    vec8 ra[kLoads], rb[kLoads];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) {
+            ra[j] = *reinterpret_cast<const vec8 *>(A + (m0 + lrow + kRowsPerPass * j) * lda + k0 + lchunk);
+            rb[j] = *reinterpret_cast<const vec8 *>(B + (n0 + lrow + kRowsPerPass * j) * ldb + k0 + lchunk);
+        }
+    };
+    auto store = [&](T *sA) {
+        T *sB = sA + kSmallTile * kSmallRow;
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) {
+            *reinterpret_cast<vec8 *>(sA + (lrow + kRowsPerPass * j) * kSmallRow + lchunk) = ra[j];
+            *reinterpret_cast<vec8 *>(sB + (lrow + kRowsPerPass * j) * kSmallRow + lchunk) = rb[j];
+        }
+    };
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+    const int frag_k = (lane >> 5) * 8;
+    const int fa = ((wave & 1) * 32 + (lane & 31)) * kSmallRow + frag_k;
+    const int fb = (kSmallTile + (wave >> 1) * 32 + (lane & 31)) * kSmallRow + frag_k;
+    load(0);
+    store(smem);
+    __syncthreads();
+    int stage = 0;
+    for (int k0 = 0; k0 < K; k0 += kSmallBK) {
+        const bool more = k0 + kSmallBK < K;
+        if (more) load(k0 + kSmallBK);
+        const T *sm = smem + stage * kStage;
+#pragma unroll
+        for (int kk = 0; kk < kSmallBK; kk += 16)
+            acc = Mfma<T>::run(*reinterpret_cast<const vec8 *>(sm + fa + kk),
+                               *reinterpret_cast<const vec8 *>(sm + fb + kk), acc);
+        // the other stage was last read by the previous step, which every wave finished
+        // before the previous barrier
+        if (more) store(smem + (stage ^ 1) * kStage);
+        __syncthreads();
+        stage ^= 1;
+    }
+}
+
+template <typename F>
+__device__ __forceinline__ void gemm_small_for_each(size_t m0, size_t n0, const floatx16 &acc, F f) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const size_t n = n0 + (wave >> 1) * 32 + (lane & 31);
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+        f(m0 + (wave & 1) * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3), n, acc[v]);
+}
+
 }  // namespace emc

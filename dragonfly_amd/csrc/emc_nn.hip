@@ -23,19 +23,45 @@ typedef __bf16 bf16;
 
 // ---- products ------------------------------------------------------------------------------
 
+// The product of a block's tile passed to the epilogue f(m, n, value). kSmall: 64 x 64 tiles of 4
+// waves, else 256 x 256 tiles of 8 waves (K advances 64 elements a step through two LDS stages
+// where K allows, as the mixed-precision EMC products do, else 32).
+enum class NnTile { kSmall, kLarge64, kLarge32 };
+
+template <NnTile kTile>
+constexpr int nn_threads() {
+    return kTile == NnTile::kSmall ? kBlock : kGemmThreads;
+}
+
+template <NnTile kTile, typename F>
+__device__ __forceinline__ void nn_product(const bf16 *__restrict__ A, size_t lda, const bf16 *__restrict__ B,
+                                           size_t ldb, int K, int m_tiles, int n_tiles, bf16 *smem, F f) {
+    if constexpr (kTile == NnTile::kSmall) {
+        const GemmTile tile = gemm_small_tile(n_tiles);
+        floatx16 acc;
+        gemm_small_mainloop<bf16>(A, lda, B, ldb, K, tile.m0, tile.n0, smem, acc);
+        gemm_small_for_each(tile.m0, tile.n0, acc, f);
+    } else {
+        const GemmTile tile = gemm_block_tile(m_tiles, n_tiles);
+        if (!tile.valid) return;
+        floatx16 acc[2][4];
+        if constexpr (kTile == NnTile::kLarge64)
+            gemm_mainloop<bf16, 1, kMpGemmBK, true, true>(A, lda, B, nullptr, ldb, K, tile.m0, tile.n0, smem, acc);
+        else
+            gemm_mainloop<bf16, 1>(A, lda, B, nullptr, ldb, K, tile.m0, tile.n0, smem, acc);
+        gemm_for_each(tile.m0, tile.n0, acc, f);
+    }
+}
+
 // Y[m][n] (m < M_valid, n < N_valid) = act(sum_k X[m][k] W[n][k] + bias[n]); out_f32 selects
 // FP32 output (logits) instead of BF16; relu applies max(0, .).
-template <bool kF32Out>
-__global__ __launch_bounds__(kGemmThreads) void nn_fwd_kernel(
+template <NnTile kTile, bool kF32Out>
+__global__ __launch_bounds__(nn_threads<kTile>()) void nn_fwd_kernel(
     const bf16 *__restrict__ X, size_t ldx, const bf16 *__restrict__ W, size_t ldw, int K,
     int m_tiles, int n_tiles, int M_valid, int N_valid, const float *__restrict__ bias, int relu,
     void *__restrict__ out, size_t ldo) {
     extern __shared__ bf16 nn_smem[];
-    const GemmTile tile = gemm_block_tile(m_tiles, n_tiles);
-    if (!tile.valid) return;
-    floatx16 acc[2][4];
-    gemm_mainloop<bf16, 1>(X, ldx, W, nullptr, ldw, K, tile.m0, tile.n0, nn_smem, acc);
-    gemm_for_each(tile.m0, tile.n0, acc, [&](size_t m, size_t n, float a) {
+    nn_product<kTile>(X, ldx, W, ldw, K, m_tiles, n_tiles, nn_smem, [&](size_t m, size_t n, float a) {
         if (m >= (size_t)M_valid || n >= (size_t)N_valid) return;
         float y = a + bias[n];
         if (relu) y = y > 0.f ? y : 0.f;
@@ -45,16 +71,13 @@ __global__ __launch_bounds__(kGemmThreads) void nn_fwd_kernel(
 }
 
 // dX[m][n] = (sum_k dY[m][k] Wt[n][k]) * (H[m][n] > 0) (H null: no mask), BF16.
-__global__ __launch_bounds__(kGemmThreads) void nn_bwd_data_kernel(
+template <NnTile kTile>
+__global__ __launch_bounds__(nn_threads<kTile>()) void nn_bwd_data_kernel(
     const bf16 *__restrict__ dY, size_t ldy, const bf16 *__restrict__ Wt, size_t ldwt, int K,
     int m_tiles, int n_tiles, int M_valid, int N_valid, const bf16 *__restrict__ H, size_t ldh,
     bf16 *__restrict__ dX, size_t ldx) {
     extern __shared__ bf16 nn_smem[];
-    const GemmTile tile = gemm_block_tile(m_tiles, n_tiles);
-    if (!tile.valid) return;
-    floatx16 acc[2][4];
-    gemm_mainloop<bf16, 1>(dY, ldy, Wt, nullptr, ldwt, K, tile.m0, tile.n0, nn_smem, acc);
-    gemm_for_each(tile.m0, tile.n0, acc, [&](size_t m, size_t n, float a) {
+    nn_product<kTile>(dY, ldy, Wt, ldwt, K, m_tiles, n_tiles, nn_smem, [&](size_t m, size_t n, float a) {
         if (m >= (size_t)M_valid || n >= (size_t)N_valid) return;
         if (H && !((float)H[m * ldh + n] > 0.f)) a = 0.f;
         dX[m * ldx + n] = (bf16)a;
@@ -62,15 +85,12 @@ __global__ __launch_bounds__(kGemmThreads) void nn_bwd_data_kernel(
 }
 
 // dW[m][n] = sum_k dYt[m][k] Xt[n][k] (FP32).
-__global__ __launch_bounds__(kGemmThreads) void nn_bwd_weight_kernel(
+template <NnTile kTile>
+__global__ __launch_bounds__(nn_threads<kTile>()) void nn_bwd_weight_kernel(
     const bf16 *__restrict__ dYt, size_t lda, const bf16 *__restrict__ Xt, size_t ldb, int K,
     int m_tiles, int n_tiles, int M_valid, int N_valid, float *__restrict__ dW, size_t ldo) {
     extern __shared__ bf16 nn_smem[];
-    const GemmTile tile = gemm_block_tile(m_tiles, n_tiles);
-    if (!tile.valid) return;
-    floatx16 acc[2][4];
-    gemm_mainloop<bf16, 1>(dYt, lda, Xt, nullptr, ldb, K, tile.m0, tile.n0, nn_smem, acc);
-    gemm_for_each(tile.m0, tile.n0, acc, [&](size_t m, size_t n, float a) {
+    nn_product<kTile>(dYt, lda, Xt, ldb, K, m_tiles, n_tiles, nn_smem, [&](size_t m, size_t n, float a) {
         if (m >= (size_t)M_valid || n >= (size_t)N_valid) return;
         dW[m * ldo + n] = a;
     });
@@ -288,35 +308,71 @@ bool tiles_ok(int M, int N, int K, size_t lda, size_t ldb) {
 }
 }  // namespace
 
+// Tile of a product: 256 x 256 where its blocks give every CU one, else 64 x 64 (K a multiple of
+// its step): a minibatch of 1024 rows by 1024 outputs makes 16 large blocks or 256 small ones.
+// Loss and gradients of 1024 rows through 4096-1024-1024-1024-3240: 910 -> 344 us.
+struct NnLaunch {
+    NnTile tile;
+    int mt, nt;
+    unsigned grid;
+    size_t lds;
+};
+
+static NnLaunch nn_launch(int M, int N, int K) {
+    const long large = (long)(M / kGemmBM) * (N / kGemmBN);
+    if (large < kNumCus && K % kSmallBK == 0) {
+        const int mt = M / kSmallTile, nt = N / kSmallTile;
+        return {NnTile::kSmall, mt, nt, (unsigned)(mt * nt), kSmallLdsElems * sizeof(bf16)};
+    }
+    const int mt = M / kGemmBM, nt = N / kGemmBN;
+    const unsigned grid = (unsigned)gemm_grid(mt, nt);
+    if (K % kMpGemmBK == 0)
+        return {NnTile::kLarge64, mt, nt, grid, gemm_lds_elems<bf16>(1, kMpGemmBK, 2) * sizeof(bf16)};
+    return {NnTile::kLarge32, mt, nt, grid, gemm_lds_elems<bf16>(1) * sizeof(bf16)};
+}
+
+#define EMC_NN_LAUNCH(l, s, call, ...)                                                                             \
+    do {                                                                                                          \
+        if (l.tile == NnTile::kSmall)                                                                             \
+            call(NnTile::kSmall)<<<l.grid, nn_threads<NnTile::kSmall>(), l.lds, s>>>(__VA_ARGS__);                \
+        else if (l.tile == NnTile::kLarge64)                                                                      \
+            call(NnTile::kLarge64)<<<l.grid, nn_threads<NnTile::kLarge64>(), l.lds, s>>>(__VA_ARGS__);            \
+        else                                                                                                      \
+            call(NnTile::kLarge32)<<<l.grid, nn_threads<NnTile::kLarge32>(), l.lds, s>>>(__VA_ARGS__);            \
+    } while (0)
+
 int launch_nn_fwd(hipStream_t s, const bf16 *X, size_t ldx, const bf16 *W, size_t ldw, int M, int N, int K,
                   int M_valid, int N_valid, const float *bias, int relu, int out_f32, void *out, size_t ldo) {
     if (!tiles_ok(M, N, K, ldx, ldw)) return -1;
-    const int mt = M / kGemmBM, nt = N / kGemmBN;
-    const size_t lds = gemm_lds_elems<bf16>(1) * sizeof(bf16);
+    const NnLaunch l = nn_launch(M, N, K);
+#define EMC_FWD32(t) nn_fwd_kernel<t, true>
+#define EMC_FWD16(t) nn_fwd_kernel<t, false>
     if (out_f32)
-        nn_fwd_kernel<true><<<gemm_grid(mt, nt), kGemmThreads, lds, s>>>(X, ldx, W, ldw, K, mt, nt, M_valid,
-                                                                         N_valid, bias, relu, out, ldo);
+        EMC_NN_LAUNCH(l, s, EMC_FWD32, X, ldx, W, ldw, K, l.mt, l.nt, M_valid, N_valid, bias, relu, out, ldo);
     else
-        nn_fwd_kernel<false><<<gemm_grid(mt, nt), kGemmThreads, lds, s>>>(X, ldx, W, ldw, K, mt, nt, M_valid,
-                                                                          N_valid, bias, relu, out, ldo);
+        EMC_NN_LAUNCH(l, s, EMC_FWD16, X, ldx, W, ldw, K, l.mt, l.nt, M_valid, N_valid, bias, relu, out, ldo);
+#undef EMC_FWD32
+#undef EMC_FWD16
     return 0;
 }
 
 int launch_nn_bwd_data(hipStream_t s, const bf16 *dY, size_t ldy, const bf16 *Wt, size_t ldwt, int M, int N,
                        int K, int M_valid, int N_valid, const bf16 *H, size_t ldh, bf16 *dX, size_t ldx) {
     if (!tiles_ok(M, N, K, ldy, ldwt)) return -1;
-    const int mt = M / kGemmBM, nt = N / kGemmBN;
-    nn_bwd_data_kernel<<<gemm_grid(mt, nt), kGemmThreads, gemm_lds_elems<bf16>(1) * sizeof(bf16), s>>>(
-        dY, ldy, Wt, ldwt, K, mt, nt, M_valid, N_valid, H, ldh, dX, ldx);
+    const NnLaunch l = nn_launch(M, N, K);
+#define EMC_BWD(t) nn_bwd_data_kernel<t>
+    EMC_NN_LAUNCH(l, s, EMC_BWD, dY, ldy, Wt, ldwt, K, l.mt, l.nt, M_valid, N_valid, H, ldh, dX, ldx);
+#undef EMC_BWD
     return 0;
 }
 
 int launch_nn_bwd_weight(hipStream_t s, const bf16 *dYt, size_t lda, const bf16 *Xt, size_t ldb, int M, int N,
                          int K, int M_valid, int N_valid, float *dW, size_t ldo) {
     if (!tiles_ok(M, N, K, lda, ldb)) return -1;
-    const int mt = M / kGemmBM, nt = N / kGemmBN;
-    nn_bwd_weight_kernel<<<gemm_grid(mt, nt), kGemmThreads, gemm_lds_elems<bf16>(1) * sizeof(bf16), s>>>(
-        dYt, lda, Xt, ldb, K, mt, nt, M_valid, N_valid, dW, ldo);
+    const NnLaunch l = nn_launch(M, N, K);
+#define EMC_BWD(t) nn_bwd_weight_kernel<t>
+    EMC_NN_LAUNCH(l, s, EMC_BWD, dYt, lda, Xt, ldb, K, l.mt, l.nt, M_valid, N_valid, dW, ldo);
+#undef EMC_BWD
     return 0;
 }
 
