@@ -17,9 +17,7 @@ PLAIN_SPACE = (
     ('lik_xcd', (1, 2, 0), ('likelihood',)),
     ('lik_unroll', (8, 16, 4), ('likelihood',)),
     ('lik_tiles', (1, 2), ('likelihood',)),
-    ('tomo_unroll', (16, 8), ('tomogram',)),
-    ('tomo_parts', (8, 16, 4), ('tomogram', 'reduce')),
-    ('tomo_width32', (0, 1), ('tomogram', 'reduce')),
+    ('tomo_parts', (8, 16, 4), ('tomogram',)),
 )
 
 

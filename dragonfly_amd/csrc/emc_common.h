@@ -35,6 +35,12 @@ constexpr int kUnitItems = 2048;
 // Sparse subsets: pixels per LDS range of the pair tomogram.
 constexpr int kPairRange = 64;
 
+// Tomogram rows (emc_tomogram.hip): bytes of one frame's row of a tile, and frames of one launch
+// (2 MB of rows, half an XCD's L2)
+constexpr int kTomoRowBytes = 128;
+constexpr int kFramesPerTomoRange = 16384;
+constexpr int kTomoUnitEntries = 8192;  // photons of one block's pixels, about
+
 // Reference constants (dragonfly/src/max_internal.h:6-8).
 constexpr double kProbMin = 1.e-6;
 constexpr double kPdiffThresh = 14.;

@@ -161,6 +161,7 @@ int parallel_ranges(long n, int nparts, F &&fn) {
         // no further thread to be had: this one takes the parts left
     }
     run(0);
+    for (; next < nparts; ++next) run(next);
     for (auto &th : pool) th.join();
     return failed ? fail(EMC_E_NOMEM, "host memory ran out while building lists") : 0;
 }
@@ -282,8 +283,13 @@ struct emc_engine {
     DevBuf<long> lik_off, tom_off;
     DevBuf<int> lik_pix, tom_frame;
     DevBuf<double> lik_cnt, tom_cnt;
-    // per (pixel, frame range) offsets into the tomogram list for the frame-partitioned form
-    DevBuf<long> tom_off2;
+    // the tomogram list of every (frame range, pixel), ranges one after another: pixel t of range
+    // x at tp_off[x * num_pix + t] (one range: the tomogram list itself)
+    int tp_ranges = 1;
+    DevBuf<int2> tp_units;  // the tomogram's pixel units (tomo_units)
+    DevBuf<long> tp_off;
+    DevBuf<int> tp_frame;
+    DevBuf<double> tp_cnt;
     // host copies of the per-pixel photon lists (tom_off / tom_frame / tom_cnt)
     std::vector<long> h_tom_off;
     std::vector<int> h_tom_frame;
@@ -297,11 +303,12 @@ struct emc_engine {
     DevBuf<long> lik8_off;
     DevBuf<int> lik8_pix;
     DevBuf<double> lik8_cnt, lik_part;
-    int tom_parts = 8, tomo_width32 = 0;
+    int tom_parts = 8, tomo_width32 = 0;  // most frame ranges of the tomogram
     // upper bound on the orientation chunk width (0: memory decides)
     int max_chunk_cols = 0;
-    DevBuf<double> tom_partial;
-    DevBuf<float> tom_partial32;  // FP32 partial views of the full frames (subset path, FP32 gathers)
+    DevBuf<double> tom_rows;      // the chunk's posterior as the tomogram reads it (128-byte rows)
+    DevBuf<double> tom_partial;   // subset path: the full frames' sums of a chunk
+    DevBuf<float> tom_partial32;  // the same in FP32 (FP32 gathers)
     // log W of every slot (one orientation chunk), left by an expectation step of the subset
     // path with the current model and geometry and not written over since: a later expectation
     // step (a second pass over new lists) skips the expand. Cleared by every change of model,
@@ -336,14 +343,15 @@ struct emc_engine {
 
     bool have_results = false;
     int last_unmerged = -1;
+    PinnedBuf<char> h_stage;  // kCopyThreads pieces of large results on their way to the host
     // orientation tiles (of 64) per wavefront in the two photon-gather kernels; tomogram
-    // form (2: frame-partitioned gather, 1: pixel-tile LDS accumulation, 0: per-pixel gather)
+    // form (2: row tiles, emc_tomogram.hip; 1: pixel-tile LDS accumulation; 0: per-pixel gather).
+    // tomo_width32, tomo_unroll and tomo_seq chose among kernels that are gone; still accepted.
     int lik_tiles = 1, tomo_tiles = 1, tomo_tile_mode = 2;
     int lik_unroll = 8, tomo_unroll = 16, tomo_seq = 0, lik_xcd = 1;
 
     // mixed-precision dense-frame path (0: plain FP64; 1: FP16 log W; 2: FP16 hi + lo log W)
     int precision = 0;
-    PinnedBuf<char> h_stage;  // kCopyThreads pieces of large results on their way to the host
     int max_count = 0;                  // largest photon count in the frames
     size_t mp_ldp = 0, mp_ldd = 0;      // padded pixel / frame counts (K of the two products)
     size_t mp_rows_d = 0, mp_rows_t = 0, mp_rows_c = 0;
@@ -417,6 +425,7 @@ struct emc_engine {
     std::vector<int> h_fidx;
     DevBuf<int> fidx, ffull, ftom_frame;
     DevBuf<long> ftom_off2;
+    DevBuf<int2> ftom_units;
     DevBuf<double> ftom_cnt, RF, scale_full, psum_full, psum_full_part;
     DevBuf<int> d_fof, d_fcounts;   // full index of every frame (-1: partial) and list counts
     DevBuf<uint8_t> blacklist_full;
@@ -465,15 +474,6 @@ struct emc_engine {
 
 namespace {
 
-// FP32 copy of model1 (every mode) for the FP32-gather expand, refreshed after model1 changed.
-int ensure_model32(emc_engine *e) {
-    if (e->model32_valid) return 0;
-    int rc;
-    if ((rc = e->model32.alloc(emc::model_brick_elems(e->size, e->num_modes)))) return rc;
-    emc::launch_copy_f32_brick(e->stream, e->model1.p, e->size, e->num_modes, e->model32.p);
-    HIP_TRY(hipGetLastError());
-    e->model32_valid = true;
-    return 0;
 // n bytes of device memory to the caller's (pageable) buffer, complete on return. Large results
 // (volumes) go through page-locked pieces that several host threads copy out, each taking every
 // kCopyThreads-th piece: hipMemcpy into fresh pageable memory runs at 10.7 GB/s here (one thread
@@ -515,6 +515,15 @@ int copy_to_host(emc_engine *e, void *dst, const void *src, size_t n) {
     return 0;
 }
 
+// FP32 copy of model1 (every mode) for the FP32-gather expand, refreshed after model1 changed.
+int ensure_model32(emc_engine *e) {
+    if (e->model32_valid) return 0;
+    int rc;
+    if ((rc = e->model32.alloc(emc::model_brick_elems(e->size, e->num_modes)))) return rc;
+    emc::launch_copy_f32_brick(e->stream, e->model1.p, e->size, e->num_modes, e->model32.p);
+    HIP_TRY(hipGetLastError());
+    e->model32_valid = true;
+    return 0;
 }
 
 // precision modes of the dense-frame products: 1, 2 FP16 log W (one term, hi + lo); 4, 5 the
@@ -584,18 +593,32 @@ int build_lists(emc_engine *e) {
             if (mask[p] < 2) { tframe[tfill[q]] = d; tcnt[tfill[q]] = c; ++tfill[q]; }
         }
     }
-    // frame-range offsets: toff2[t * nparts + x] = first photon of pixel t in frame range x
-    const int nparts = e->tom_parts;
-    std::vector<long> toff2((size_t)P * nparts + 1);
-    for (int t = 0; t < P; ++t) {
-        long k = tcount[t];
+    // frame ranges of about kFramesPerTomoRange frames (at most tom_parts): range x holds the
+    // frames N x / nparts <= d < N (x + 1) / nparts; its lists, pixel after pixel
+    const int nparts = std::max(1, std::min(e->tom_parts, (N + emc::kFramesPerTomoRange - 1) / emc::kFramesPerTomoRange));
+    std::vector<long> poff;
+    std::vector<int> pframe;
+    std::vector<double> pcnt;
+    if (nparts > 1) {
+        poff.resize((size_t)P * nparts + 1);
+        pframe.resize(tframe.size());
+        pcnt.resize(tcnt.size());
+        std::vector<long> next(tcount.begin(), tcount.end() - 1);
+        long at = 0;
         for (int x = 0; x < nparts; ++x) {
-            const long lo = (long)N * x / nparts;
-            while (k < tcount[t + 1] && tframe[k] < lo) ++k;
-            toff2[(size_t)t * nparts + x] = k;
+            const long hi = (long)N * (x + 1) / nparts;
+            for (int t = 0; t < P; ++t) {
+                poff[(size_t)x * P + t] = at;
+                long k = next[t];
+                for (; k < tcount[t + 1] && tframe[k] < hi; ++k, ++at) {
+                    pframe[at] = tframe[k];
+                    pcnt[at] = tcnt[k];
+                }
+                next[t] = k;
+            }
         }
+        poff[(size_t)P * nparts] = at;
     }
-    toff2[(size_t)P * nparts] = tcount[P];
 
     // tile form: photons of mask < 2 pixels grouped by 128-pixel tile, then frame
     const int ntiles = (P + 127) / 128;
@@ -649,7 +672,18 @@ int build_lists(emc_engine *e) {
     e->tile_entries = ne;
 
     int rc;
-    if ((rc = e->tom_off2.upload(toff2.data(), toff2.size(), e->stream))) return rc;
+    e->tp_ranges = nparts;
+    const std::vector<int2> units = emc::tomo_units(nparts > 1 ? poff.data() : tcount.data(), nparts, P);
+    if ((rc = e->tp_units.upload(units.data(), units.size(), e->stream))) return rc;
+    if (nparts > 1) {
+        if ((rc = e->tp_off.upload(poff.data(), poff.size(), e->stream))) return rc;
+        if ((rc = e->tp_frame.upload(pframe.data(), pframe.size(), e->stream))) return rc;
+        if ((rc = e->tp_cnt.upload(pcnt.data(), pcnt.size(), e->stream))) return rc;
+    } else {
+        e->tp_off.release();
+        e->tp_frame.release();
+        e->tp_cnt.release();
+    }
     e->any_dense = false;
     for (uint8_t v : e->h_dense) e->any_dense |= (v != 0);
     if ((rc = e->dense.upload(e->h_dense.data(), e->h_dense.size(), e->stream))) return rc;
@@ -1067,8 +1101,7 @@ int build_subset(emc_engine *e, int num_coarse, const int *qmap, const long *rel
 // Per-pixel photon lists (mask < 2) restricted to the full frames, frame index f, with the
 // offsets of tom_parts ranges of f: the plain path's partitioned tomogram lists for RF.
 int build_full_lists(emc_engine *e) {
-    // frame ranges of about kFramesPerTomoPart frames (at most tom_parts): fewer full frames
-    // share fewer partial views, whose writes and reads would otherwise dominate
+    // frame ranges of about full_part_frames frames (at most tom_parts): one tomogram launch each
     const int P = e->num_pix, nF = e->num_full, N = e->num_data;
     const int per = e->full_part_frames;
     const int nparts = std::max(1, std::min(std::min(e->tom_parts, 64), (nF + per - 1) / per));
@@ -1097,6 +1130,8 @@ int build_full_lists(emc_engine *e) {
     }
     off2[ncell] = total;
     if ((rc = e->ftom_off2.upload(off2.data(), off2.size(), s))) return rc;
+    const std::vector<int2> units = emc::tomo_units(off2.data(), nparts, P);
+    if ((rc = e->ftom_units.upload(units.data(), units.size(), s))) return rc;
     if ((rc = e->ftom_frame.alloc((size_t)std::max(total, 1L)))) return rc;
     if ((rc = e->ftom_cnt.alloc((size_t)std::max(total, 1L)))) return rc;
     emc::launch_full_lists(s, 1, e->tom_off.p, e->tom_frame.p, e->tom_cnt.p, e->d_fof.p, P, std::max(nF, 1), nparts,
@@ -1208,7 +1243,7 @@ int ensure_work(emc_engine *e) {
     size_t budget = freeb > reserve ? freeb - reserve : 0;
     const size_t cap = (size_t)120 << 30;
     budget += e->logw.cap * sizeof(double);
-    budget += e->tom_partial.cap * sizeof(double);
+    budget += e->tom_rows.cap * sizeof(double);
     budget += (e->lw_hi.cap + e->lw_lo.cap + e->p16.cap) * sizeof(_Float16);
     const bool mp = mp_mode(e);
     const bool g32 = e->precision == 3;
@@ -1223,15 +1258,16 @@ int ensure_work(emc_engine *e) {
         budget = budget + have > kbytes ? budget + have - kbytes : 0;
     }
     if (budget > cap) budget = cap;
-    // per orientation column: log W / view, plus the partial views of the partitioned
-    // tomogram (plain path) or the FP16 log W rows and posterior column (mixed path)
+    // per orientation column: log W / view, plus the posterior as the tomogram reads it (plain
+    // path) or the FP16 log W rows and posterior column (mixed path)
     const bool split = !mp && !g32 && e->lik_split > 1;
     budget += e->lik_part.cap * sizeof(double);
     if (!split) e->lik_part.release();  // before the chunk buffers grow into its room
     const size_t per_col = mp ? P * sizeof(double) + (mp_two(e) ? 2 : 1) * e->mp_ldp * sizeof(_Float16) +
                                     e->mp_ldd * sizeof(_Float16)
-                              : P * sizeof(double) * (1 + (e->tomo_tile_mode == 2 ? e->tom_parts : 0)) +
-                                    (g32 ? P * sizeof(float) + N * sizeof(float) : 0) +
+                              : P * sizeof(double) +
+                                    (g32 ? P * sizeof(float) + N * sizeof(float)
+                                         : (e->tomo_tile_mode == 2 ? N * sizeof(double) : 0)) +
                                     (split ? (size_t)e->lik_split * N * sizeof(double) : 0);
     size_t cmax = budget / per_col;
     if (e->max_chunk_cols > 0 && cmax > (size_t)e->max_chunk_cols) cmax = e->max_chunk_cols;
@@ -1241,7 +1277,7 @@ int ensure_work(emc_engine *e) {
     if (C != e->C || !e->logw.p) {
         // exact sizes: the budget above counted these buffers as free
         e->bricks_valid = false;
-        e->tom_partial.release();
+        e->tom_rows.release();
         e->logw.release();
         e->lik_part.release();
         e->logw32.release();
@@ -1249,8 +1285,9 @@ int ensure_work(emc_engine *e) {
         if ((rc = e->logw.alloc(P * (size_t)C))) return rc;
         e->C = C;
     }
+    e->tom_partial.release();  // the subset path's
+    if (mp || g32 || e->tomo_tile_mode != 2) e->tom_rows.release();
     if (mp) {
-        e->tom_partial.release();
         const size_t rows_c = round_up((size_t)e->C, emc::kGemmBN);
         if (rows_c != e->mp_rows_c || !e->lw_hi.p || mp_two(e) != (e->lw_lo.p != nullptr)) {
             e->lw_hi.release();
@@ -1286,7 +1323,7 @@ int ensure_work(emc_engine *e) {
         e->ktom.release();
         e->mp_built = false;
         e->mp_rows_c = 0;
-        if (e->tomo_tile_mode == 2 && (rc = e->tom_partial.alloc((size_t)e->tom_parts * P * (size_t)C))) return rc;
+        if (!g32 && e->tomo_tile_mode == 2 && (rc = e->tom_rows.alloc(N * (size_t)C))) return rc;
     }
     if (split) {
         if (e->split_built != e->lik_split && (rc = build_lik_split(e, e->lik_split))) return rc;
@@ -1296,7 +1333,7 @@ int ensure_work(emc_engine *e) {
         // 128-wide tiles: room for the chunk rounded up to 128 orientations
         const size_t C128 = round_up((size_t)e->C, 128);
         if ((rc = e->logw32.alloc(P * C128))) return rc;
-        if ((rc = e->p32.alloc(N * C128))) return rc;
+        if ((rc = e->p32.alloc(N * (size_t)e->C))) return rc;
     } else {
         e->logw32.release();
         e->p32.release();
@@ -1331,7 +1368,8 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
     const size_t vol = (size_t)e->size * e->size * e->size;
     if (!e->fsort_valid && (rc = build_fsort(e))) return rc;
     if (nF > 0 && !e->full_lists_valid && (rc = build_full_lists(e))) return rc;
-    const int nparts = e->full_parts;
+    const emc::TomoLists flists{e->ftom_off2.p, e->ftom_frame.p, e->ftom_cnt.p, e->full_parts, e->ftom_units.p,
+                                (int)e->ftom_units.n};
     // memory: the plain path's rows are not needed here
     e->R.release();
     const size_t rsub_need = (size_t)std::max<long>(e->num_pairs, 1) * emc::kRTile;
@@ -1352,6 +1390,7 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
             e->logw32.release();
             e->logw_resident = false;
         }
+        e->tom_rows.release();
         e->tom_partial.release();
         e->tom_partial32.release();
         e->p32.release();
@@ -1387,15 +1426,14 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
     // full frames: else they keep their room for the next lists that have some)
     size_t budget = (freeb > reserve ? freeb - reserve : 0) + e->logw.cap * sizeof(double) +
                     e->logw32.cap * sizeof(float) +
-                    (nF > 0 ? e->tom_partial.cap * sizeof(double) + (e->p32.cap + e->tom_partial32.cap) * sizeof(float)
+                    (nF > 0 ? (e->tom_rows.cap + e->tom_partial.cap) * sizeof(double) +
+                                  (e->p32.cap + e->tom_partial32.cap) * sizeof(float)
                             : 0);
     budget = std::min(budget, (size_t)120 << 30);
-    // per slot column: log W / view and the full frames' partial views (FP64; with FP32 gathers
-    // all FP32, log W and the view sharing one buffer, plus the full frames' FP32 posterior
-    // column), and the view's nonzero masks
-    const size_t parts_col = nF > 0 ? (size_t)nparts : 0;
-    const size_t per_col = (g32 ? (size_t)P * sizeof(float) * (1 + parts_col) + (size_t)nF * sizeof(float)
-                                : (size_t)P * sizeof(double) * (1 + parts_col)) +
+    // per slot column: log W / view, the full frames' sums and their posterior column (FP64; with
+    // FP32 gathers all FP32), and the view's nonzero masks
+    const size_t parts_col = nF > 0 ? 1 : 0;
+    const size_t per_col = ((size_t)P * (1 + parts_col) + (size_t)nF) * (g32 ? sizeof(float) : sizeof(double)) +
                            (size_t)((P + 63) / 64) * sizeof(unsigned long long);
     size_t cmax = budget / per_col;
     if (e->max_chunk_cols > 0) cmax = std::min(cmax, (size_t)e->max_chunk_cols);
@@ -1425,9 +1463,9 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
     }
     if (g32 && e->logw32.cap > (size_t)P * C128) e->logw_resident = false;  // released below
     if (g32) {
-        const size_t n_part = nF > 0 ? (size_t)nparts * P * (size_t)C : 0, n_logw = (size_t)P * C128,
-                     n_p32 = nF > 0 ? (size_t)nF * C128 : 0;
+        const size_t n_part = nF > 0 ? (size_t)P * C : 0, n_logw = (size_t)P * C128, n_p32 = (size_t)nF * C;
         e->tom_partial.release();
+        e->tom_rows.release();
         shrink(e->logw32, n_logw);
         shrink(e->tom_partial32, n_part);
         shrink(e->p32, n_p32);
@@ -1437,9 +1475,10 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
         e->tom_partial32.release();
         e->logw32.release();
         e->p32.release();
-        const size_t n_part = nF > 0 ? (size_t)nparts * P * (size_t)C : 0;
+        const size_t n_part = nF > 0 ? (size_t)P * C : 0, n_rows = (size_t)nF * C;
         shrink(e->tom_partial, n_part);
-        if ((rc = fit(e->tom_partial, n_part))) return rc;
+        shrink(e->tom_rows, n_rows);
+        if ((rc = fit(e->tom_partial, n_part)) || (rc = fit(e->tom_rows, n_rows))) return rc;
     }
     const int ngroups = (P + kPixPerGroup - 1) / kPixPerGroup;
     if ((rc = e->upart.alloc((size_t)ngroups * C))) return rc;
@@ -1721,14 +1760,12 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
             const int t0 = bc.r0 / emc::kRTile, t1 = (bc.r0 + bc.Cc) / emc::kRTile;
             if (parts && (rc = timed(6, [&] {
                                if (g32) {
-                                   emc::launch_to_f32(s, e->RF.p, nF, bc.r0, bc.Cc, e->p32.p);
-                                   emc::launch_tomogram_parts_f32(s, e->p32.p, nF, bc.Cc, e->ftom_off2.p, nparts,
-                                                                  e->ftom_frame.p, e->ftom_cnt.p, P,
-                                                                  e->tom_partial32.p);
+                                   emc::launch_posterior_rows(s, e->RF.p, nF, bc.r0, bc.Cc, S, e->p32.p);
+                                   emc::launch_tomogram_rows(s, e->p32.p, nF, bc.Cc, flists, P, e->tom_partial32.p);
                                } else {
-                                   emc::launch_tomogram_parts(s, e->RF.p, nF, bc.r0, bc.Cc, e->ftom_off2.p, nparts,
-                                                              e->ftom_frame.p, e->ftom_cnt.p, nullptr, S, P,
-                                                              e->tom_partial.p, e->logw.p, 0, 16, 0);
+                                   emc::launch_posterior_rows(s, e->RF.p, nF, bc.r0, bc.Cc, S, e->tom_rows.p);
+                                   emc::launch_tomogram_rows(s, e->tom_rows.p, nF, bc.Cc, flists, P, nullptr, 0,
+                                                             e->tom_partial.p, false);
                                }
                                return 0;
                            })))
@@ -1742,13 +1779,13 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
                          emc::launch_pair_tomogram(s, e->Rsub32.p, e->tile_off.p, e->sig_pair.p, e->sig_frame.p,
                                                    e->sig_cnt.p, e->fsort_off.p, e->fsort_roff.p, e->nranges,
                                                    e->fsort_pix.p, e->fsort_cnt.p, e->psum_slot.p, t0, t1 - t0, P,
-                                                   parts ? e->tom_partial32.p : nullptr, nparts, e->logw32.p, nz,
+                                                   parts ? e->tom_partial32.p : nullptr, e->logw32.p, nz,
                                                    frows, bkv);
                      else
                          emc::launch_pair_tomogram(s, e->Rsub.p, e->tile_off.p, e->sig_pair.p, e->sig_frame.p,
                                                    e->sig_cnt.p, e->fsort_off.p, e->fsort_roff.p, e->nranges,
                                                    e->fsort_pix.p, e->fsort_cnt.p, e->psum_slot.p, t0, t1 - t0, P,
-                                                   parts ? e->tom_partial.p : nullptr, nparts, e->logw.p, nz,
+                                                   parts ? e->tom_partial.p : nullptr, e->logw.p, nz,
                                                    frows, bkv);
                      return 0;
                  })))
@@ -2005,7 +2042,11 @@ void emc_destroy(emc_engine *e) {
     e->blacklist.release();
     e->lik_off.release();
     e->tom_off.release();
-    e->tom_off2.release();
+    e->tp_units.release();
+    e->tp_off.release();
+    e->tp_frame.release();
+    e->tp_cnt.release();
+    e->tom_rows.release();
     e->tom_partial.release();
     e->ft_off.release();
     e->fe_off.release();
@@ -2935,6 +2976,9 @@ int emc_maximize(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *stats
     }
 
     // tomogram + merge, chunk by chunk
+    const bool ranges = e->tp_ranges > 1;
+    const emc::TomoLists lists{ranges ? e->tp_off.p : e->tom_off.p, ranges ? e->tp_frame.p : e->tom_frame.p,
+                               ranges ? e->tp_cnt.p : e->tom_cnt.p, e->tp_ranges, e->tp_units.p, (int)e->tp_units.n};
     for (int r0 = 0; r0 < e->Rp; r0 += C) {
         const int Cc = (e->Rp - r0 < C) ? (e->Rp - r0) : C;
         float a = 0.f, b = 0.f, c = 0.f;
@@ -2959,14 +3003,12 @@ int emc_maximize(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *stats
                                     1. / pscale))
                 return fail(EMC_E_STATE, "tomogram product: shape does not fit the tiles");
         } else if (g32) {
-            emc::launch_to_f32(s, e->R.p, N, r0, Cc, e->p32.p);
-            emc::launch_tomogram_parts_f32(s, e->p32.p, N, Cc, e->tom_off2.p, e->tom_parts, e->tom_frame.p,
-                                           e->tom_cnt.p, P, e->tom_partial.p);
-        } else if (parts)
-            emc::launch_tomogram_parts(s, e->R.p, N, r0, Cc, e->tom_off2.p, e->tom_parts,
-                                       e->tom_frame.p, e->tom_cnt.p, e->psum_r.p, Rn, P,
-                                       e->tom_partial.p, e->logw.p, e->tomo_width32,
-                                       e->tomo_unroll, e->tomo_seq);
+            emc::launch_posterior_rows(s, e->R.p, N, r0, Cc, Rn, e->p32.p);
+            emc::launch_tomogram_rows(s, e->p32.p, N, Cc, lists, P, e->psum_r.p + r0, Rn - r0, e->logw.p, bricks);
+        } else if (parts) {
+            emc::launch_posterior_rows(s, e->R.p, N, r0, Cc, Rn, e->tom_rows.p);
+            emc::launch_tomogram_rows(s, e->tom_rows.p, N, Cc, lists, P, e->psum_r.p + r0, Rn - r0, e->logw.p, bricks);
+        }
         else if (e->tomo_tile_mode == 1)
             emc::launch_tomogram_tiles(s, e->R.p, N, r0, Cc, e->ft_off.p, e->ft_frame.p,
                                        e->fe_off.p, e->fe_code.p, e->psum_r.p, Rn, P, e->logw.p);
@@ -2974,12 +3016,6 @@ int emc_maximize(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *stats
             emc::launch_tomogram(s, e->R.p, N, r0, Cc, e->tom_off.p, e->tom_frame.p,
                                  e->tom_cnt.p, e->psum_r.p, Rn, P, e->logw.p, e->tomo_tiles);
         HIP_TRY(hipEventRecord(e->ev[1], s));
-        if (parts && bricks)
-            emc::launch_tomogram_reduce_rmajor(s, e->tom_partial.p, e->tom_parts, r0, Cc, e->psum_r.p,
-                                               Rn, P, e->logw.p);
-        else if (parts)
-            emc::launch_tomogram_reduce(s, e->tom_partial.p, e->tom_parts, r0, Cc, e->psum_r.p,
-                                        Rn, P, e->logw.p);
         HIP_TRY(hipEventRecord(e->ev[2], s));
         if (bricks) {
             if ((rc = merge_chunk(e, r0 / C, e->logw.p, false, true, !cached_weight))) return rc;

@@ -5,6 +5,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <vector>
 
 namespace emc {
 
@@ -22,7 +23,6 @@ void launch_copy_f32(hipStream_t s, const double *in, size_t n, float *out);
 // FP32 copy of `modes` volumes in 4^3-voxel bricks (the FP32-gather expand's model)
 size_t model_brick_elems(long size, int modes);
 void launch_copy_f32_brick(hipStream_t s, const double *in, long size, int modes, float *out);
-void launch_to_f32(hipStream_t s, const double *P, int num_data, int r0, int C, float *out);
 void launch_likelihood(hipStream_t s, const float *logw, int C, int num_pix, const long *off,
                        const int *pix, const double *cnt, const uint8_t *blacklist, int num_data,
                        double *G, int r0, int unroll, int xcd_order);
@@ -38,13 +38,6 @@ void launch_likelihood_mapped(hipStream_t s, const double *logw, int C, int num_
 void launch_likelihood_mapped(hipStream_t s, const float *logw, int C, int num_pix, const long *off,
                               const int *pix, const double *cnt, const uint8_t *blacklist, const int *fmap,
                               int num_rows, double *G, int r0);
-void launch_tomogram_parts_f32(hipStream_t s, const float *P32, int num_data, int C, const long *toff2,
-                               int nparts, const int *tframe, const double *tcnt, int num_pix,
-                               double *partial);
-// the same with FP32 partial sums (each the FP64 sum rounded once)
-void launch_tomogram_parts_f32(hipStream_t s, const float *P32, int num_data, int C, const long *toff2,
-                               int nparts, const int *tframe, const double *tcnt, int num_pix,
-                               float *partial);
 void launch_u_reduce(hipStream_t s, const double *upart, const int *ubad, int ngroups, int C,
                      int r0, int num_rot, double *u, int *rbad);
 void launch_rescale(hipStream_t s, const double *quats, const double *u, int num_rot,
@@ -135,14 +128,31 @@ void launch_tomogram_tiles(hipStream_t s, const double *P, int num_data, int r0,
                            const long *ft_off, const int *ft_frame, const long *fe_off,
                            const int *fe_code, const double *psum_r, int num_rot, int num_pix,
                            double *view);
-void launch_tomogram_parts(hipStream_t s, const double *P, int num_data, int r0, int C,
-                           const long *toff2, int nparts, const int *tframe, const double *tcnt,
-                           const double *psum_r, int num_rot, int num_pix, double *partial,
-                           double *view, int width32, int unroll, int seq);
-void launch_tomogram_reduce(hipStream_t s, const double *partial, int nparts, int r0, int C,
-                            const double *psum_r, int num_rot, int num_pix, double *view);
-void launch_tomogram_reduce_rmajor(hipStream_t s, const double *partial, int nparts, int r0, int C,
-                                   const double *psum_r, int num_rot, int num_pix, double *view);
+// ---- tomogram (emc_tomogram.hip) ----
+// rows of the chunk's posterior in tiles of kTomoRowBytes rows (C a multiple of 64 columns from
+// orientation r0; P <= 1e-6 and columns past num_rot are 0): num_data * C elements
+void launch_posterior_rows(hipStream_t s, const double *P, int num_data, int r0, int C, int num_rot, double *rows);
+void launch_posterior_rows(hipStream_t s, const double *P, int num_data, int r0, int C, int num_rot, float *rows);
+// photon lists of nparts frame ranges (range x, pixel t: entries off[x * num_pix + t] up to the
+// next offset; frame, count), and the pixel units (first, number) the blocks take
+struct TomoLists {
+    const long *off;
+    const int *frame;
+    const double *cnt;
+    int nparts;
+    const int2 *units;
+    int num_units;
+};
+std::vector<int2> tomo_units(const long *off, int nparts, int num_pix);
+// the chunk's view from those rows and lists, divided by psum (of the chunk's columns; num_psum of
+// them are orientations; null: sums only); orientation-major or tile-major
+void launch_tomogram_rows(hipStream_t s, const double *rows, int num_data, int C, const TomoLists &l, int num_pix,
+                          const double *psum, int num_psum, double *view, bool rmajor);
+void launch_tomogram_rows(hipStream_t s, const float *rows, int num_data, int C, const TomoLists &l, int num_pix,
+                          const double *psum, int num_psum, double *view, bool rmajor);
+// tile-major FP32 sums (each the FP64 sum rounded once per frame range)
+void launch_tomogram_rows(hipStream_t s, const float *rows, int num_data, int C, const TomoLists &l, int num_pix,
+                          float *sums);
 // ---- brick merge (emc_merge.hip) ----
 // per-brick item lists: pass 0 counts, pass 1 writes the item ids and, beside each, the mask of
 // the item's pixels with a trilinear corner inside the brick
@@ -277,13 +287,13 @@ void launch_sig_full_rows(hipStream_t s, const double *RF, int nF, int num_tiles
 void launch_pair_tomogram(hipStream_t s, const double *P, const long *tile_off, const int *sig_pair,
                           const int *sig_frame, const int *sig_cnt, const long *foff, const int *roff, int nranges,
                           const int *fpix, const double *fcnt, const double *psum_slot, int t0, int ntiles,
-                          int num_pix, const double *partial, int nparts, double *view,
+                          int num_pix, const double *partial, double *view,
                           unsigned long long *nzmask, const SigFullRows &fr = SigFullRows(),
                           const PairBuckets &bk = PairBuckets());
 void launch_pair_tomogram(hipStream_t s, const float *P, const long *tile_off, const int *sig_pair,
                           const int *sig_frame, const int *sig_cnt, const long *foff, const int *roff, int nranges,
                           const int *fpix, const double *fcnt, const double *psum_slot, int t0, int ntiles,
-                          int num_pix, const float *partial, int nparts, float *view, unsigned long long *nzmask,
+                          int num_pix, const float *partial, float *view, unsigned long long *nzmask,
                           const SigFullRows &fr = SigFullRows(), const PairBuckets &bk = PairBuckets());
 // pairs with some P > 1e-6 in their row, per tile in the tile's order (flag: num_pairs bytes;
 // sig_pair / sig_frame: tile_off layout; sig_cnt: per tile)
@@ -301,7 +311,7 @@ void launch_full_scatter(hipStream_t s, const double *RF, int nF, int num_tiles,
                          const int *slot_rot, int num_rot, double *out, int f0 = 0, int f1 = -1, int d0 = 0);
 void launch_slot_gather(hipStream_t s, const double *in, const int *rot_slot, int num_rot, double *out);
 // Full-frame photon lists per engine pixel in nparts ranges of full-frame index (nparts <= 64):
-// pass 0 writes counts[t * nparts + x]; pass 1 fills out_frame / out_cnt from off2 (the
+// pass 0 writes counts[x * num_pix + t]; pass 1 fills out_frame / out_cnt from off2 (the
 // exclusive scan of the counts). fof[d] is frame d's full index or -1.
 void launch_full_lists(hipStream_t s, int pass, const long *tom_off, const int *tom_frame, const double *tom_cnt,
                        const int *fof, int num_pix, int nF, int nparts, int *counts, const long *off2,

@@ -552,143 +552,6 @@ __global__ __launch_bounds__(kBlock) void tomogram_kernel(
     }
 }
 
-// Frame-partitioned form of the tomogram. Frames are split into nparts contiguous ranges and
-// block b works on range b % nparts: with blocks dispatched round-robin over the 8 XCDs
-// (nparts a multiple of 8), each XCD's L2 holds only its own frames' P slab of the
-// orientation tile. Each range writes a partial view; tomogram_reduce_kernel adds the
-// partials in range order and divides by psum_r. toff2[t * nparts + x] is the first photon of
-// pixel t with a frame in range x (the per-pixel list is frame-ascending).
-//
-// kSeq orders the blocks so that each XCD walks its ranges one after another (all pixels of
-// range x, then of range x + 8, ...) instead of interleaving them, which keeps one range's
-// P slab in that XCD's L2 at a time; nparts is then a multiple of 8.
-template <int U, bool kSeq, typename T>
-__global__ __launch_bounds__(kBlock) void tomogram_part_kernel(
-    const T *__restrict__ P, size_t tsP, int r0, int C, const long *__restrict__ toff2,
-    int nparts, const int *__restrict__ tframe, const double *__restrict__ tcnt, int num_pix,
-    int ngroups, double *__restrict__ partial) {
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    int part, group;
-    if (kSeq) {
-        const int seq = blockIdx.x / kNumXcd;
-        part = (seq / ngroups) * kNumXcd + blockIdx.x % kNumXcd;
-        group = seq % ngroups;
-    } else {
-        part = blockIdx.x % nparts;
-        group = blockIdx.x / nparts;
-    }
-    const int t = group * kWavesPerBlock + wave;
-    if (t >= num_pix) return;
-    const int c0 = blockIdx.y * kRTile;
-    const T *__restrict__ col = P + (size_t)((r0 + c0) >> 6) * tsP + lane;
-    const size_t at = (size_t)t * nparts + part;
-    long k = toff2[at];
-    const long k1 = toff2[at + 1];
-    double acc = 0.;
-    for (; k + U <= k1; k += U) {
-        double v[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = (double)col[(size_t)tframe[k + u] * kRTile];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (v[u] > kProbMin) acc += tcnt[k + u] * v[u];
-    }
-    for (; k < k1; ++k) {
-        const double p = (double)col[(size_t)tframe[k] * kRTile];
-        if (p > kProbMin) acc += tcnt[k] * p;
-    }
-    const size_t tsW = (size_t)num_pix * kRTile, tsPart = tsW * (C / kRTile);
-    partial[part * tsPart + (size_t)(c0 >> 6) * tsW + (size_t)t * kRTile + lane] = acc;
-}
-
-// Same as tomogram_part_kernel with a wavefront covering 32 orientations: lanes 0-31 take the
-// even photons of the pixel's list and lanes 32-63 the odd ones (two 256-byte P segments per
-// load instruction); the halves are added at the end. The L2 slab of one frame range for one
-// 32-orientation block is half as large.
-__global__ __launch_bounds__(kBlock) void tomogram_part32_kernel(
-    const double *__restrict__ P, size_t tsP, int r0, int C, const long *__restrict__ toff2,
-    int nparts, const int *__restrict__ tframe, const double *__restrict__ tcnt, int num_pix,
-    double *__restrict__ partial) {
-    constexpr int U = 8;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63, half = lane >> 5;
-    const int part = blockIdx.x % nparts;
-    const int t = (blockIdx.x / nparts) * kWavesPerBlock + wave;
-    if (t >= num_pix) return;
-    const int c0 = blockIdx.y * (kRTile / 2);          // chunk-local first orientation (multiple of 32)
-    const int rg = r0 + c0;                             // global first orientation
-    const double *__restrict__ col = P + (size_t)(rg >> 6) * tsP + (rg & 63) + (lane & 31);
-    const size_t at = (size_t)t * nparts + part;
-    long k = toff2[at];
-    const long k1 = toff2[at + 1];
-    double acc = 0.;
-    for (; k + 2 * U <= k1; k += 2 * U) {
-        double v[U], c[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const long kk = k + 2 * u + half;
-            v[u] = col[(size_t)tframe[kk] * kRTile];
-            c[u] = tcnt[kk];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (v[u] > kProbMin) acc += c[u] * v[u];
-    }
-    for (; k < k1; k += 2) {
-        const long kk = k + half;
-        if (kk < k1) {
-            const double p = col[(size_t)tframe[kk] * kRTile];
-            if (p > kProbMin) acc += tcnt[kk] * p;
-        }
-    }
-    acc += __shfl_down(acc, 32);
-    if (half == 0) {
-        const size_t tsW = (size_t)num_pix * kRTile, tsPart = tsW * (C / kRTile);
-        partial[part * tsPart + (size_t)(c0 >> 6) * tsW + (size_t)t * kRTile + (c0 & 63) + lane] = acc;
-    }
-}
-
-// Same sum, written orientation-major (view[c][t], c chunk-local) through an LDS transpose:
-// block = 64 pixels x 64 orientations.
-__global__ __launch_bounds__(kBlock) void tomogram_reduce_rmajor_kernel(
-    const double *__restrict__ partial, int nparts, int r0, int C, int num_pix,
-    const double *__restrict__ psum_r, int num_rot, double *__restrict__ view) {
-    __shared__ double s[64][kRTile + 1];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int t0 = blockIdx.x * 64, c0 = blockIdx.y * kRTile;
-    const size_t tsW = (size_t)num_pix * kRTile, tsPart = tsW * (C / kRTile);
-    const int r = r0 + c0 + lane;
-    const double ps = (psum_r && r < num_rot) ? psum_r[r] : 0.;  // no psum: sums only
-    for (int k = wave; k < 64; k += kWavesPerBlock) {
-        const int t = t0 + k;
-        if (t >= num_pix) break;
-        const size_t i = (size_t)(c0 >> 6) * tsW + (size_t)t * kRTile + lane;
-        double acc = 0.;
-        for (int x = 0; x < nparts; ++x) acc += partial[x * tsPart + i];
-        s[k][lane] = (ps > 0.) ? acc / ps : acc;
-    }
-    __syncthreads();
-    const int t = t0 + lane;
-    if (t < num_pix)
-        for (int k = wave; k < kRTile; k += kWavesPerBlock)
-            view[(size_t)(c0 + k) * num_pix + t] = s[lane][k];
-}
-
-__global__ void tomogram_reduce_kernel(const double *__restrict__ partial, int nparts, int r0,
-                                       int C, int num_pix, const double *__restrict__ psum_r,
-                                       int num_rot, double *__restrict__ view) {
-    const size_t tsW = (size_t)num_pix * kRTile, n = tsW * (C / kRTile);
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x) {
-        double acc = 0.;
-        for (int x = 0; x < nparts; ++x) acc += partial[x * n + i];
-        const int r = r0 + (int)(i / tsW) * kRTile + (int)(i % kRTile);
-        const double ps = (r < num_rot) ? psum_r[r] : 0.;
-        view[i] = (ps > 0.) ? acc / ps : acc;
-    }
-}
-
 // Tile form of the tomogram. Engine pixels are grouped in tiles of kTomoTile consecutive
 // pixels (compact detector patches, Morton order). For a tile the photons are listed frame by
 // frame: ft_off[tile]..ft_off[tile+1] index the tile's distinct frames (ft_frame), and
@@ -1139,70 +1002,6 @@ void launch_copy_f32_brick(hipStream_t s, const double *in, long size, int modes
     copy_f32_brick_kernel<<<grid_cap(cdiv(n, 256)), 256, 0, s>>>(in, size, modes, out);
 }
 
-// FP32 copy of one orientation chunk of the tile-major posterior in 128-wide tiles:
-// out[(c / 128) * N * 128 + d * 128 + c % 128] = P[((r0 + c) / 64) * N * 64 + d * 64 + c % 64]
-// for chunk orientations c < C (r0 a multiple of 64; columns of the last tile past C are 0).
-__global__ void to_f32_w128_kernel(const double *__restrict__ P, int num_data, int r0, int C,
-                                   float *__restrict__ out) {
-    const size_t n = (size_t)num_data * ((C + 127) / 128) * 128;
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const int cw = (int)(i % 128);
-        const size_t rest = i / 128;
-        const int d = (int)(rest % num_data);
-        const int c = (int)(rest / num_data) * 128 + cw;
-        out[i] = c < C ? (float)P[(size_t)((r0 + c) / kRTile) * num_data * kRTile + (size_t)d * kRTile + (c % kRTile)]
-                       : 0.f;
-    }
-}
-
-void launch_to_f32(hipStream_t s, const double *P, int num_data, int r0, int C, float *out) {
-    const size_t n = (size_t)num_data * ((C + 127) / 128) * 128;
-    to_f32_w128_kernel<<<grid_cap(cdiv(n, 256)), 256, 0, s>>>(P, num_data, r0, C, out);
-}
-
-// Frame-partitioned tomogram over an FP32 posterior in 128-wide tiles (see to_f32_w128_kernel):
-// each lane gathers two orientations per photon; partial sums in FP64, written in the 64-wide
-// tile-major partial layout of tomogram_part_kernel.
-template <int U, typename OT>
-__global__ __launch_bounds__(kBlock) void tomogram_part_w128_kernel(
-    const float *__restrict__ P32, size_t tsP, int C, const long *__restrict__ toff2, int nparts,
-    const int *__restrict__ tframe, const double *__restrict__ tcnt, int num_pix, OT *__restrict__ partial) {
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    const int part = blockIdx.x % nparts;
-    const int t = (blockIdx.x / nparts) * kWavesPerBlock + wave;
-    if (t >= num_pix) return;
-    const int tile = blockIdx.y;
-    const float2 *__restrict__ col = reinterpret_cast<const float2 *>(P32 + (size_t)tile * tsP) + lane;
-    const size_t at = (size_t)t * nparts + part;
-    long k = toff2[at];
-    const long k1 = toff2[at + 1];
-    double a0 = 0., a1 = 0.;
-    for (; k + U <= k1; k += U) {
-        float2 v[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = col[(size_t)tframe[k + u] * 64];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const double c = tcnt[k + u];
-            if ((double)v[u].x > kProbMin) a0 += c * (double)v[u].x;
-            if ((double)v[u].y > kProbMin) a1 += c * (double)v[u].y;
-        }
-    }
-    for (; k < k1; ++k) {
-        const float2 v = col[(size_t)tframe[k] * 64];
-        if ((double)v.x > kProbMin) a0 += tcnt[k] * (double)v.x;
-        if ((double)v.y > kProbMin) a1 += tcnt[k] * (double)v.y;
-    }
-    const int c = tile * 128 + 2 * lane;
-    if (c < C) {
-        const size_t tsW = (size_t)num_pix * kRTile, tsPart = tsW * (C / kRTile);
-        OT *dst = partial + part * tsPart + (size_t)(c / kRTile) * tsW + (size_t)t * kRTile + (c % kRTile);
-        dst[0] = (OT)a0;
-        dst[1] = (OT)a1;
-    }
-}
-
 void launch_u_reduce(hipStream_t s, const double *upart, const int *ubad, int ngroups, int C,
                      int r0, int num_rot, double *u, int *rbad) {
     u_reduce_kernel<<<cdiv(C, 256), 256, 0, s>>>(upart, ubad, ngroups, C, r0, num_rot, u, rbad);
@@ -1611,62 +1410,6 @@ void launch_tomogram_tiles(hipStream_t s, const double *P, int num_data, int r0,
     tomogram_tile_kernel<<<grid, kBlock, 0, s>>>(P, (size_t)num_data * kRTile, r0, C,
                                                  (size_t)num_pix * kRTile, ft_off, ft_frame, fe_off,
                                                  fe_code, psum_r, num_rot, num_pix, view);
-}
-
-void launch_tomogram_parts(hipStream_t s, const double *P, int num_data, int r0, int C,
-                           const long *toff2, int nparts, const int *tframe, const double *tcnt,
-                           const double *psum_r, int num_rot, int num_pix, double *partial,
-                           double *view, int width32, int unroll, int seq) {
-    if (width32) {
-        dim3 grid(cdiv(num_pix, kWavesPerBlock) * nparts, C / (kRTile / 2));
-        tomogram_part32_kernel<<<grid, kBlock, 0, s>>>(P, (size_t)num_data * kRTile, r0, C, toff2,
-                                                       nparts, tframe, tcnt, num_pix, partial);
-    } else {
-        const int ngroups = (int)cdiv(num_pix, kWavesPerBlock);
-        dim3 grid(ngroups * nparts, C / kRTile);
-        const bool sq = seq && nparts % kNumXcd == 0;
-#define EMC_TP(U, SQ)                                                                            \
-    tomogram_part_kernel<U, SQ, double><<<grid, kBlock, 0, s>>>(P, (size_t)num_data * kRTile, r0, C, toff2, \
-                                                                nparts, tframe, tcnt, num_pix, ngroups, partial)
-        if (sq) {
-            if (unroll >= 16) EMC_TP(16, true); else EMC_TP(8, true);
-        } else {
-            if (unroll >= 16) EMC_TP(16, false); else EMC_TP(8, false);
-        }
-#undef EMC_TP
-    }
-}
-
-// FP32 posterior of one orientation chunk (128-wide tiles, to_f32_w128_kernel), FP64 sums.
-void launch_tomogram_parts_f32(hipStream_t s, const float *P32, int num_data, int C, const long *toff2,
-                               int nparts, const int *tframe, const double *tcnt, int num_pix,
-                               double *partial) {
-    const int ngroups = (int)cdiv(num_pix, kWavesPerBlock);
-    dim3 grid(ngroups * nparts, cdiv(C, 128));
-    tomogram_part_w128_kernel<16, double><<<grid, kBlock, 0, s>>>(P32, (size_t)num_data * 128, C, toff2, nparts,
-                                                                  tframe, tcnt, num_pix, partial);
-}
-
-void launch_tomogram_parts_f32(hipStream_t s, const float *P32, int num_data, int C, const long *toff2,
-                               int nparts, const int *tframe, const double *tcnt, int num_pix, float *partial) {
-    const int ngroups = (int)cdiv(num_pix, kWavesPerBlock);
-    dim3 grid(ngroups * nparts, cdiv(C, 128));
-    tomogram_part_w128_kernel<16, float><<<grid, kBlock, 0, s>>>(P32, (size_t)num_data * 128, C, toff2, nparts,
-                                                                 tframe, tcnt, num_pix, partial);
-}
-
-void launch_tomogram_reduce_rmajor(hipStream_t s, const double *partial, int nparts, int r0, int C,
-                                   const double *psum_r, int num_rot, int num_pix, double *view) {
-    dim3 grid(cdiv(num_pix, 64), C / kRTile);
-    tomogram_reduce_rmajor_kernel<<<grid, kBlock, 0, s>>>(partial, nparts, r0, C, num_pix, psum_r, num_rot,
-                                                          view);
-}
-
-void launch_tomogram_reduce(hipStream_t s, const double *partial, int nparts, int r0, int C,
-                            const double *psum_r, int num_rot, int num_pix, double *view) {
-    const size_t n = (size_t)num_pix * C;
-    tomogram_reduce_kernel<<<grid_cap(cdiv(n, 256)), 256, 0, s>>>(partial, nparts, r0, C, num_pix,
-                                                                  psum_r, num_rot, view);
 }
 
 void launch_merge(hipStream_t s, const double *rots, int r0, int C, int num_rot, const double *view,

@@ -553,8 +553,7 @@ void launch_pair_buckets(hipStream_t s, int num_tiles, const long *tile_off, con
 }
 
 // Tomogram of the chunk's tiles [t0, t0 + ntiles) over pixel ranges of kPairRange pixels:
-// block (tile, range) starts from the full frames' partial sums (tomogram_part_kernel
-// layout partial[x][tile][t][64], added over the nparts frame ranges in order) or from zero,
+// block (tile, range) starts from the full frames' sums partial[tile][t][64] or from zero,
 // adds K * P (P > 1e-6) of the tile's significant partial-frame pairs (sig_pair, sig_cnt)
 // and, with RF, of its significant full-frame rows (sigF_*: rows RF[T][f][64], in place of the
 // partial sums) into LDS rows of the range's pixels (frame photon lists sorted by pixel, range
@@ -568,7 +567,7 @@ __global__ __launch_bounds__(kBlock) void pair_tomogram_kernel(
     const int *__restrict__ tile_frame, const int *__restrict__ sig_cnt, const long *__restrict__ foff,
     const int *__restrict__ roff, int nranges, const int *__restrict__ fpix, const double *__restrict__ fcnt,
     const double *__restrict__ psum_slot, int t0, int ntiles, int num_pix,
-    const PT *__restrict__ partial, int nparts, VT *__restrict__ view,
+    const PT *__restrict__ partial, VT *__restrict__ view,
     unsigned long long *__restrict__ nzmask, const double *__restrict__ RF, int nF,
     const int *__restrict__ sigF_row, const int *__restrict__ sigF_frame, const int *__restrict__ sigF_cnt,
     const PairBuckets bk) {
@@ -612,13 +611,12 @@ __global__ __launch_bounds__(kBlock) void pair_tomogram_kernel(
     const size_t frow0 = (size_t)T * nF;
     const int p0 = rg * kPairRange;
     if (partial) {
-        const size_t tsW = (size_t)num_pix * kRTile, tsPart = tsW * ntiles;
+        const size_t tsW = (size_t)num_pix * kRTile;
         for (int i = wave; i < kPairRange; i += kWavesPerBlock) {
             const int t = p0 + i;
             double a = 0.;
             if (t < num_pix) {
-                const size_t at = (size_t)lt * tsW + (size_t)t * kRTile + lane;
-                for (int x = 0; x < nparts; ++x) a += (double)partial[x * tsPart + at];
+                a = (double)partial[(size_t)lt * tsW + (size_t)t * kRTile + lane];
             }
             acc[i][lane] = (A)a;
         }
@@ -804,8 +802,8 @@ __global__ __launch_bounds__(kBlock) void cell_posterior_kernel(
 // ---- full-frame photon lists ----------------------------------------------------------------
 // Per engine pixel, the photons (mask < 2) of the full frames in frame order, split into
 // nparts ranges of full-frame index f (range x holds f with nF * x / nparts <= f). One wave
-// per pixel. Pass 0 counts the photons of every (pixel, range); pass 1 writes them from the
-// pixel's first output slot off2[t * nparts], keeping the pixel's frame order.
+// per pixel. Pass 0 counts the photons of every (range, pixel), counts[x * num_pix + t]; pass 1
+// writes them from off2[x * num_pix + t], keeping the pixel's frame order.
 __device__ __forceinline__ int full_part_of(int f, int nF, int nparts) {
     int x = (int)(((long)f * nparts) / nF);  // then the largest x with nF * x / nparts <= f
     while (x + 1 < nparts && (long)nF * (x + 1) / nparts <= f) ++x;
@@ -822,28 +820,24 @@ __global__ __launch_bounds__(kBlock) void full_lists_kernel(
     const int t = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
     if (t >= num_pix) return;
     const long k0 = tom_off[t], k1 = tom_off[t + 1];
-    long at = pass ? off2[(size_t)t * nparts] : 0;
-    int cnt_lane = 0;  // pass 0: lane x < nparts counts range x
+    // lane x < nparts: entries of range x so far (pass 0), its next position (pass 1)
+    long at = pass && lane < nparts ? off2[(size_t)lane * num_pix + t] : 0;
     for (long kb = k0; kb < k1; kb += 64) {
         const long k = kb + lane;
         const int f = k < k1 ? fof[tom_frame[k]] : -1;
-        const unsigned long long keep = __ballot(f >= 0);
-        if (pass == 0) {
-            const int x = f >= 0 ? full_part_of(f, nF, nparts) : -1;
-            for (int y = 0; y < nparts; ++y) {
-                const int n = __popcll(__ballot(x == y));
-                if (lane == y) cnt_lane += n;
-            }
-        } else {
-            if (f >= 0) {
-                const long pos = at + __popcll(keep & ((1ull << lane) - 1ull));
+        const int x = f >= 0 ? full_part_of(f, nF, nparts) : -1;
+        for (int y = 0; y < nparts; ++y) {
+            const unsigned long long in = __ballot(x == y);
+            const long next = __shfl(at, y);
+            if (pass && x == y) {
+                const long pos = next + __popcll(in & ((1ull << lane) - 1ull));
                 out_frame[pos] = f;
                 out_cnt[pos] = tom_cnt[k];
             }
-            at += __popcll(keep);
+            if (lane == y) at += __popcll(in);
         }
     }
-    if (pass == 0 && lane < nparts) counts[(size_t)t * nparts + lane] = cnt_lane;
+    if (pass == 0 && lane < nparts) counts[(size_t)lane * num_pix + t] = (int)at;
 }
 
 // ---- launchers -----------------------------------------------------------------------------
@@ -1023,32 +1017,32 @@ template <typename TP, typename VT, typename PT>
 static void pair_tomogram_launch(hipStream_t s, const TP *P, const long *tile_off, const int *sig_pair,
                                  const int *sig_frame, const int *sig_cnt, const long *foff, const int *roff,
                                  int nranges, const int *fpix, const double *fcnt, const double *psum_slot, int t0,
-                                 int ntiles, int num_pix, const PT *partial, int nparts, VT *view,
+                                 int ntiles, int num_pix, const PT *partial, VT *view,
                                  unsigned long long *nzmask, const SigFullRows &fr, const PairBuckets &bk) {
     if (ntiles <= 0) return;
     const unsigned grid = (unsigned)((ntiles + kNumXcd - 1) / kNumXcd * kNumXcd) * (unsigned)nranges;
     pair_tomogram_kernel<TP, VT, PT><<<grid, kBlock, 0, s>>>(P, tile_off, sig_pair, sig_frame, sig_cnt, foff, roff,
                                                              nranges, fpix, fcnt, psum_slot, t0, ntiles, num_pix,
-                                                             partial, nparts, view, nzmask, fr.RF, fr.nF, fr.row,
+                                                             partial, view, nzmask, fr.RF, fr.nF, fr.row,
                                                              fr.frame, fr.cnt, bk);
 }
 
 void launch_pair_tomogram(hipStream_t s, const double *P, const long *tile_off, const int *sig_pair,
                           const int *sig_frame, const int *sig_cnt, const long *foff, const int *roff, int nranges,
                           const int *fpix, const double *fcnt, const double *psum_slot, int t0, int ntiles,
-                          int num_pix, const double *partial, int nparts, double *view,
+                          int num_pix, const double *partial, double *view,
                           unsigned long long *nzmask, const SigFullRows &fr, const PairBuckets &bk) {
     pair_tomogram_launch(s, P, tile_off, sig_pair, sig_frame, sig_cnt, foff, roff, nranges, fpix, fcnt, psum_slot,
-                         t0, ntiles, num_pix, partial, nparts, view, nzmask, fr, bk);
+                         t0, ntiles, num_pix, partial, view, nzmask, fr, bk);
 }
 
 void launch_pair_tomogram(hipStream_t s, const float *P, const long *tile_off, const int *sig_pair,
                           const int *sig_frame, const int *sig_cnt, const long *foff, const int *roff, int nranges,
                           const int *fpix, const double *fcnt, const double *psum_slot, int t0, int ntiles,
-                          int num_pix, const float *partial, int nparts, float *view,
+                          int num_pix, const float *partial, float *view,
                           unsigned long long *nzmask, const SigFullRows &fr, const PairBuckets &bk) {
     pair_tomogram_launch(s, P, tile_off, sig_pair, sig_frame, sig_cnt, foff, roff, nranges, fpix, fcnt, psum_slot,
-                         t0, ntiles, num_pix, partial, nparts, view, nzmask, fr, bk);
+                         t0, ntiles, num_pix, partial, view, nzmask, fr, bk);
 }
 
 template <typename TP>

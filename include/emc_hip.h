@@ -168,8 +168,8 @@ int emc_set_precision(emc_engine *e, int mode);
  * wave), lik_unroll (4/8/16 rows in flight), lik_xcd (XCD-aware tile order of the
  * likelihood launch: 1, 2, 4 or 8 XCDs share a log W tile; 0 off), lik_split (2-8: photon lists split into pixel ranges, one per XCD
  * group, partial sums added in range order), tomo_tiles, tomo_tile_mode (0 per-pixel gather,
- * 1 LDS tiles, 2 frame-partitioned, default), tomo_parts (frame ranges, 1-64), tomo_width32,
- * tomo_unroll (8/16), tomo_seq, max_chunk_cols (0 = by memory), merge_mode (0 box, 1 brick),
+ * 1 LDS tiles, 2 row tiles, default), tomo_parts (most frame ranges, 1-64), tomo_width32,
+ * tomo_unroll (8/16) and tomo_seq (accepted, without effect), max_chunk_cols (0 = by memory), merge_mode (0 box, 1 brick),
  * subset (1 sparse refinement subsets, 0 masked), slot_pack (1: refinement cells packed
  * back to back along a nearest-neighbour chain, 0: each cell padded to whole 64-orientation
  * tiles; takes effect at the next emc_set_refine), sparse_rows (frames per batch of

@@ -85,3 +85,47 @@ def test_pair_likelihood_photon_counts(precision):
         eng.close()
     for k in ('max_exp', 'p_norm', 'likelihood', 'prob'):
         assert P.rel_err(out[0][k], out[1][k]) <= (1e-9 if precision == 0 else 1e-6), k
+
+
+@pytest.mark.parametrize('frames, num_rot', ((1, 1), (3, 64), (65, 65), (257, 129), (16385, 20), (33000, 33)))
+def test_tomogram_rows(frames, num_rot):
+    """The tomogram's row tiles and frame ranges: one frame, fewer frames than streams, patches
+    with few or no photons, orientation counts that end inside a 16- or 32-wide tile, two and
+    three frame ranges (16,384 frames each). FP64 against the oracle to 1e-9, FP32 gathers to 1e-4
+    (the FP32-gather tests' bars), orientation-major (brick merge) and tile-major (box merge)."""
+    p = P.build(P.tiny_config(num_data=frames, mean_count=25.), quats=_lib.quat_gen(2)[:num_rot], num_ave=200)
+    p['fparams']['beta'] = np.full(frames, 0.1)
+    o = P.run_oracle(p, dict(iteration=1), dense_prob=False)
+    eng = P.engine_for(p)
+    for precision, merge_mode, bar in ((0, 1, 1e-9), (0, 0, 1e-9), (3, 1, 1e-4)):
+        eng.set_precision(precision)
+        eng.set_option('merge_mode', merge_mode)
+        eng.maximize(1, 0, 1, 0)
+        assert P.rel_err(eng.get('model2'), o['model2']) <= bar, (precision, merge_mode)
+        assert P.rel_err(eng.get('inter_weight'), o['inter_weight']) <= 1e-9
+    eng.close()
+
+
+@pytest.mark.parametrize('precision', (0, 3))
+@pytest.mark.parametrize('part_frames', (12500, 7))
+def test_full_frames_tomogram_ranges(precision, part_frames):
+    """Refinement subsets with full frames: their sums (one launch or several frame ranges)
+    taken over by the pair tomogram, against the masked full search."""
+    p = counted_problem(COUNTS, 420)
+    qc = _lib.quat_gen(1)
+    cells = _lib.voronoi_subset(qc, p['quats'])
+    rng = np.random.default_rng(5)
+    sets = [np.array([-1], 'i4') if d % 2 else np.sort(rng.permutation(len(qc))[:5]).astype('i4')
+            for d in range(len(COUNTS))]
+    off = np.concatenate([[0], np.cumsum([len(s) for s in sets])]).astype('i8')
+    out = []
+    for subset in (1, 0):
+        eng = P.engine_for(p)
+        eng.set_precision(precision)
+        eng.set_option('subset', subset)
+        eng.set_option('sig_full_rows', 0)
+        eng.set_option('full_part_frames', part_frames)
+        eng.set_refine(len(qc), cells, off, np.concatenate(sets))
+        out.append(P.run_engine(eng, dict(iteration=1)))
+        eng.close()
+    assert P.rel_err(out[0]['model2'], out[1]['model2']) <= (1e-9 if precision == 0 else 1e-4)
