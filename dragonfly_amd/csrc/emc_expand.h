@@ -27,21 +27,23 @@ constexpr float kLogDblMin = (float)(-1022.0 * 0.693147180559945309417232121458)
 
 // LDS of one expand block. With the FP32 model copy (MT float) the rotations are FP32 and the
 // transposition tile holds W as FP32 (W = DBL_MIN outside the grid as -inf): 21 KB instead of
-// 43 KB a block, so that twice as many blocks share a CU.
+// 38 KB a block, so that more blocks share a CU.
 template <typename MT>
 struct ExpandShared {
     static constexpr bool f32 = sizeof(MT) == sizeof(float);
     using V = typename std::conditional<f32, float, double>::type;
-    V rot[kRTile * 9];
+    V rot[f32 ? kRTile * 9 : 1];
+    double2 logs[f32 ? 1 : kLogTable];
     V tile[64][kRTile + 1];
     double u[kWavesPerBlock][kRTile];
     int bad[kWavesPerBlock][kRTile];
-    int pad[kRTile];
 };
 
 // Tile starting at chunk column c0, pixel group g; called by all kBlock threads of a block.
-// MT: element type of the model read (double, or float for the FP32-gather path's copy)
-template <typename T, int kW, typename MT>
+// MT: element type of the model read (double, or float for the FP32-gather path's copy); kModes: more
+// than one mode. No branch stands between the interpolations of a wave's orientations, so the loads
+// of several are in flight.
+template <typename T, int kW, typename MT, bool kModes>
 __device__ __forceinline__ void expand_block(
     ExpandShared<MT> &sh, int c0, int g, const double *__restrict__ rots, const MT *__restrict__ model, long size,
     const double *__restrict__ qvals, const double *__restrict__ corr, const uint8_t *__restrict__ mask, int num_pix,
@@ -49,13 +51,16 @@ __device__ __forceinline__ void expand_block(
     const int *__restrict__ slot_rot, int modes, int raw) {
     constexpr bool f32 = sizeof(MT) == sizeof(float);
     const int tid = threadIdx.x;
-    for (int i = tid; i < kRTile * 9; i += kBlock) sh.rot[i] = (typename ExpandShared<MT>::V)rots[(size_t)(r0 + c0) * 9 + i];
-    // padding slots of the subset order (slot_rot < 0) get W = 1 without interpolation
-    if (tid < kRTile) sh.pad[tid] = slot_rot != nullptr && slot_rot[r0 + c0 + tid] < 0;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if constexpr (f32)
+        for (int i = tid; i < kRTile * 9; i += kBlock) sh.rot[i] = (float)rots[(size_t)(r0 + c0) * 9 + i];
+    else if (tid < kLogTable)
+        log_table_entry(tid, sh.logs);
     __syncthreads();
+    // padding slots of the subset order (slot_rot < 0) get W = 1; lane = orientation when storing
+    const bool pad = slot_rot != nullptr && slot_rot[r0 + c0 + lane] < 0;
     const double center = (double)(size / 2);
     const int nb = model_bricks(size);
-    const int lane = tid & 63, wave = tid >> 6;
     const int t_begin = g * pix_per_group;
     const int t_end = min(num_pix, t_begin + pix_per_group);
     double uacc = 0.;
@@ -70,15 +75,13 @@ __device__ __forceinline__ void expand_block(
             for (int k = 0; k < kRTile / kWavesPerBlock; ++k) {
                 const int rr = wave + kWavesPerBlock * k;
                 // combined orientation index r = rotation * modes + mode (max_prob.c:80-84)
-                const MT *mdl = modes > 1 ? model + (size_t)((r0 + c0 + rr) % modes) * mode_stride(model, size) : model;
-                if constexpr (f32) {
-                    const float v =
+                const MT *mdl = kModes ? model + (size_t)((r0 + c0 + rr) % modes) * mode_stride(model, size) : model;
+                if constexpr (f32)
+                    sh.tile[lane][rr] =
                         slice_value_f32h(mdl, (int)size, nb, &sh.rot[rr * 9], qf0, qf1, qf2, crf, (float)center);
-                    sh.tile[lane][rr] = sh.pad[rr] ? 1.f : v;
-                } else {
-                    const double v = slice_value(mdl, size, &sh.rot[rr * 9], q0, q1, q2, cr, center);
-                    sh.tile[lane][rr] = sh.pad[rr] ? 1. : v;
-                }
+                else  // a wave's rotation is uniform: scalar loads
+                    sh.tile[lane][rr] =
+                        slice_value(mdl, size, rots + (size_t)(r0 + c0 + rr) * 9, q0, q1, q2, cr, center);
             }
         }
         __syncthreads();
@@ -91,7 +94,7 @@ __device__ __forceinline__ void expand_block(
                 T *dst = logw + (size_t)(c / kW) * ((size_t)num_pix * kW) + (size_t)tt * kW + (c % kW);
                 if constexpr (f32) {
                     // FP32 tile: -inf outside the grid (W = DBL_MIN there: not bad, log W = log(DBL_MIN))
-                    const float Wt = sh.tile[p][lane];
+                    const float Wt = pad ? 1.f : sh.tile[p][lane];
                     const bool outside = Wt == -INFINITY;
                     if (mask[tt] < 1) {
                         uacc += outside ? DBL_MIN : (double)Wt;
@@ -99,13 +102,13 @@ __device__ __forceinline__ void expand_block(
                     }
                     *dst = (T)(outside ? kLogDblMin : (Wt >= FLT_MIN ? __logf(Wt) : logf(Wt)));
                 } else {
-                    const double W = sh.tile[p][lane];
+                    const double W = pad ? 1. : sh.tile[p][lane];
                     if (mask[tt] < 1) {
                         uacc += W;
                         bad |= !(W > 0.);
                     }
                     // raw: W itself (the background-aware likelihood takes log(phi W + b B))
-                    *dst = raw ? (T)W : (T)log(W);
+                    *dst = raw ? (T)W : (T)table_log(W, sh.logs);
                 }
             }
         }

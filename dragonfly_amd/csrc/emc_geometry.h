@@ -28,12 +28,11 @@ __device__ __forceinline__ bool locate(const double *rot, double q0, double q1, 
     c.y = __double2int_rz(p1);
     c.z = __double2int_rz(p2);
     const int hi = (int)size - 2;
-    if (c.x < 0 || c.x > hi || c.y < 0 || c.y > hi || c.z < 0 || c.z > hi)
-        return false;
     c.fx = p0 - c.x;
     c.fy = p1 - c.y;
     c.fz = p2 - c.z;
-    return true;
+    // one unsigned comparison an axis (a negative cell is a large one); hi < 0: no cell
+    return hi >= 0 && (unsigned)c.x <= (unsigned)hi && (unsigned)c.y <= (unsigned)hi && (unsigned)c.z <= (unsigned)hi;
 }
 
 // Two neighbouring voxels along z, read with one 16-byte load from any 8-byte boundary.
@@ -44,16 +43,17 @@ typedef double VoxelPair __attribute__((ext_vector_type(2), aligned(8)));
 // DBL_MIN, so the loads of several calls can be in flight at once. The reference wraps the far
 // corner, (x + 1) % size, but cells stop at size - 2, so the wrap never happens: the far
 // corners are at fixed distances from the near one and the two corners of each z edge are one
-// 16-byte load. Without the three 64-bit remainders and four of the eight loads the FP64
+// 16-byte load. A 1^3 model has no cell: its (unused) loads stay at its one voxel and the spare
+// element that the engine allocates behind a model. Without the three 64-bit remainders and four of the eight loads the FP64
 // expand of 25,680 orientations x 66,820 pixels on 251^3 takes 16.0 ms instead of 19.4.
 __device__ __forceinline__ double slice_value(const double *__restrict__ model, long size,
                                               const double *rot, double q0, double q1, double q2,
                                               double corr, double center) {
-    if (size < 2) return DBL_MIN;  // no cell at all
-    Cell c{0, 0, 0, 0., 0., 0.};
+    Cell c;
     const bool ok = locate(rot, q0, q1, q2, center, size, c);
-    const int sz = (int)size;
-    const double *__restrict__ m = model + (ok ? (long)(c.x * sz + c.y) * sz + c.z : 0);
+    const int sz = size < 2 ? 0 : (int)size;
+    const long at = (long)(int)((unsigned)c.x * (unsigned)sz + (unsigned)c.y) * sz + c.z;
+    const double *__restrict__ m = model + (ok ? at : 0);
     const long s2 = (long)sz * sz;
     const VoxelPair m00 = *(const VoxelPair *)m, m01 = *(const VoxelPair *)(m + sz);
     const VoxelPair m10 = *(const VoxelPair *)(m + s2), m11 = *(const VoxelPair *)(m + s2 + sz);
@@ -62,6 +62,32 @@ __device__ __forceinline__ double slice_value(const double *__restrict__ model, 
     const double v = cx * cy * cz * m00.x + cx * cy * fz * m00.y + cx * fy * cz * m01.x + cx * fy * fz * m01.y +
                      fx * cy * cz * m10.x + fx * cy * fz * m10.y + fx * fy * cz * m11.x + fx * fy * fz * m11.y;
     return ok ? v * corr : DBL_MIN;
+}
+
+// log of a positive normal number by table (P. T. P. Tang's scheme: the mantissa's interval gives 1 / c
+// and log c, and log1p of r = z / c - 1, |r| <= 2^-8, is a polynomial): 15 FP64 operations and one
+// 16-byte LDS read where the device library's log takes 70 operations, within 1 ulp of it
+// (absolute error 1.1e-16 from the table where the result is near 0). Anything else goes to log().
+constexpr int kLogTable = 128;
+__device__ __forceinline__ void log_table_entry(int i, double2 *tab) {
+    const double inv = 1. / __hiloint2double(0x3fe60000 + (i << 13) + (1 << 12), 0);
+    tab[i] = make_double2(inv, -log(inv));
+}
+__device__ __forceinline__ double table_log(double x, const double2 *tab) {
+    const int hi = __double2hiint(x);
+    if ((unsigned)hi - 0x00100000u >= 0x7fe00000u) return log(x);  // 0, subnormal, negative, inf, NaN
+    const int tmp = hi - 0x3fe60000;  // intervals of the mantissa from 0.6875 to 1.375
+    const double2 t = tab[(tmp >> 13) & (kLogTable - 1)];
+    const double z = __hiloint2double(hi - (tmp & (int)0xfff00000), __double2loint(x));
+    const double r = __builtin_fma(z, t.x, -1.), k = (double)(tmp >> 20);
+    const double w = __builtin_fma(k, 0x1.62e42fefa3800p-1, t.y);  // k ln 2: the high part times k is exact
+    const double s = w + r, lo = __builtin_fma(k, 0x1.ef35793c76730p-45, (w - s) + r);
+    double p = __builtin_fma(r, 1. / 7., -1. / 6.);
+    p = __builtin_fma(r, p, 1. / 5.);
+    p = __builtin_fma(r, p, -1. / 4.);
+    p = __builtin_fma(r, p, 1. / 3.);
+    p = __builtin_fma(r, p, -1. / 2.);
+    return s + __builtin_fma(r * r, p, lo);
 }
 
 // FP32 model copy in bricks of 4 x 4 x 4 trilinear cells: brick (X/4, Y/4, Z/4) of an nb^3
@@ -74,7 +100,7 @@ constexpr int kModelBrick = 4;
 constexpr int kHaloBrickFloats = 128;  // 5^3 = 125 corners, padded
 __host__ __device__ __forceinline__ int model_bricks(long size) { return (int)((size - 2) / kModelBrick + 1); }
 __device__ __forceinline__ long halo_index(int nb, int x, int y, int z) {
-    return (((long)(x >> 2) * nb + (y >> 2)) * nb + (z >> 2)) * kHaloBrickFloats + (x & 3) * 25 + (y & 3) * 5 + (z & 3);
+    return ((long)((x >> 2) * nb + (y >> 2)) * nb + (z >> 2)) * kHaloBrickFloats + ((x & 3) * 25 + (y & 3) * 5 + (z & 3));
 }
 
 // Interpolated value of the FP32 brick copy at the rotated position of a pixel times the
@@ -90,9 +116,10 @@ __device__ __forceinline__ float slice_value_f32h(const float *__restrict__ mode
     const float p2 = __builtin_fmaf(rot[6], q0, __builtin_fmaf(rot[7], q1, __builtin_fmaf(rot[8], q2, center)));
     const int x = (int)p0, y = (int)p1, z = (int)p2;  // truncation toward zero
     const int hi = size - 2;
-    const bool ok = x >= 0 && x <= hi && y >= 0 && y <= hi && z >= 0 && z <= hi;
+    const bool ok = hi >= 0 && (unsigned)x <= (unsigned)hi && (unsigned)y <= (unsigned)hi && (unsigned)z <= (unsigned)hi;
     const float fx = p0 - (float)x, fy = p1 - (float)y, fz = p2 - (float)z;
-    const float *b = model + (ok ? halo_index(nb, x, y, z) : 0);
+    // the cell, not the index, is selected: a branch here would serialise the loads of a wave's values
+    const float *b = model + halo_index(nb, ok ? x : 0, ok ? y : 0, ok ? z : 0);
     const float m000 = b[0], m001 = b[1], m010 = b[5], m011 = b[6];
     const float m100 = b[25], m101 = b[26], m110 = b[30], m111 = b[31];
     const float a00 = __builtin_fmaf(fz, m001 - m000, m000), a01 = __builtin_fmaf(fz, m011 - m010, m010);

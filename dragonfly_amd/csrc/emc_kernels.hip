@@ -45,7 +45,7 @@ __device__ __forceinline__ void merge_value(double *__restrict__ model2, double 
 
 // ---- expand: log W for one orientation chunk, plus partial u_r ---------------------------
 // Block = 64 orientations x one pixel group (expand_block, emc_expand.h).
-template <typename T, int kW, typename MT = double>
+template <typename T, int kW, typename MT, bool kModes>
 __global__ __launch_bounds__(kBlock) void expand_kernel(
     const double *__restrict__ rots, const MT *__restrict__ model, long size,
     const double *__restrict__ qvals, const double *__restrict__ corr,
@@ -61,7 +61,7 @@ __global__ __launch_bounds__(kBlock) void expand_kernel(
     const int xcd = blockIdx.x % kNumXcd, b = blockIdx.x / kNumXcd;
     const int tile = xcd * per + b % per, g = b / per;
     if (tile >= ntiles || (long)g * pix_per_group >= num_pix) return;
-    expand_block<T, kW, MT>(sh, tile * kRTile, g, rots, model, size, qvals, corr, mask, num_pix, r0, C, pix_per_group,
+    expand_block<T, kW, MT, kModes>(sh, tile * kRTile, g, rots, model, size, qvals, corr, mask, num_pix, r0, C, pix_per_group,
                             logw, upart, ubad, slot_rot, modes, raw);
 }
 
@@ -935,17 +935,24 @@ void launch_expand(hipStream_t s, const double *rots, const double *model, long 
                    const double *qvals, const double *corr, const uint8_t *mask, int num_pix,
                    int r0, int C, int pix_per_group, double *logw, double *upart, int *ubad,
                    const int *slot_rot, int modes, int raw) {
-    expand_kernel<double, kRTile><<<expand_grid(C, num_pix, pix_per_group), kBlock, 0, s>>>(rots, model, size, qvals, corr, mask, num_pix, r0, C,
-                                                          pix_per_group, logw, upart, ubad, slot_rot, modes, raw);
+#define EMC_EXPAND(M)                                                                                              \
+    expand_kernel<double, kRTile, double, M><<<expand_grid(C, num_pix, pix_per_group), kBlock, 0, s>>>(             \
+        rots, model, size, qvals, corr, mask, num_pix, r0, C, pix_per_group, logw, upart, ubad, slot_rot, modes, raw)
+    if (modes > 1) EMC_EXPAND(true);
+    else EMC_EXPAND(false);
+#undef EMC_EXPAND
 }
 
 void launch_expand(hipStream_t s, const double *rots, const float *model, long size,
                    const double *qvals, const double *corr, const uint8_t *mask, int num_pix,
                    int r0, int C, int pix_per_group, float *logw, double *upart, int *ubad,
                    const int *slot_rot, int modes) {
-    expand_kernel<float, 2 * kRTile, float><<<expand_grid(C, num_pix, pix_per_group), kBlock, 0, s>>>(rots, model, size, qvals, corr, mask, num_pix,
-                                                                    r0, C, pix_per_group, logw, upart, ubad,
-                                                                    slot_rot, modes, 0);
+#define EMC_EXPAND(M)                                                                                              \
+    expand_kernel<float, 2 * kRTile, float, M><<<expand_grid(C, num_pix, pix_per_group), kBlock, 0, s>>>(           \
+        rots, model, size, qvals, corr, mask, num_pix, r0, C, pix_per_group, logw, upart, ubad, slot_rot, modes, 0)
+    if (modes > 1) EMC_EXPAND(true);
+    else EMC_EXPAND(false);
+#undef EMC_EXPAND
 }
 
 __global__ void copy_if_zero_kernel(double *__restrict__ dst, const double *__restrict__ src, size_t n,

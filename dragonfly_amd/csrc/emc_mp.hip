@@ -164,17 +164,17 @@ __global__ __launch_bounds__(kBlock) void expand_mp_kernel(
     const uint8_t *__restrict__ mask, const double *__restrict__ center_t, int num_pix, int r0,
     int C, int pix_per_group, size_t ldp, int two_terms, T *__restrict__ lw_hi,
     T *__restrict__ lw_lo, double *__restrict__ upart, int *__restrict__ ubad) {
-    __shared__ double s_rot[kRTile * 9];
+    __shared__ double2 s_logs[kLogTable];
     __shared__ double s_tile[64][kRTile + 1];
     __shared__ double s_u[kWavesPerBlock][kRTile];
     __shared__ int s_bad[kWavesPerBlock][kRTile];
     const int tid = threadIdx.x;
     const int c0 = blockIdx.x * kRTile;
     const int g = blockIdx.y;
-    for (int i = tid; i < kRTile * 9; i += kBlock) s_rot[i] = rots[(size_t)(r0 + c0) * 9 + i];
+    if (tid < kLogTable) log_table_entry(tid, s_logs);
     __syncthreads();
     const double center = (double)(size / 2);
-    const int lane = tid & 63, wave = tid >> 6;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int t_begin = g * pix_per_group;
     const int t_end = min(num_pix, t_begin + pix_per_group);
     double uacc = 0.;
@@ -185,15 +185,23 @@ __global__ __launch_bounds__(kBlock) void expand_mp_kernel(
             const double q0 = qvals[3 * (size_t)t], q1 = qvals[3 * (size_t)t + 1],
                          q2 = qvals[3 * (size_t)t + 2], cr = corr[t], ct = center_t[t];
             const bool good = mask[t] < 1;
-            for (int k = 0; k < kRTile / kWavesPerBlock; ++k) {
-                const int rr = wave + kWavesPerBlock * k;
-                const double W = slice_value(model, size, &s_rot[rr * 9], q0, q1, q2, cr, center);
-                s_tile[lane][rr] = W;
-                double x = (good && W > 0.) ? log(W) - ct : 0.;
-                const T hi = to_op<T>(x);
-                const size_t at = (size_t)(c0 + rr) * ldp + t;
-                lw_hi[at] = hi;
-                if (two_terms) lw_lo[at] = to_op<T>(x - from_op<T>(hi));
+            // four values a step: their loads are in flight together
+            for (int k0 = 0; k0 < kRTile / kWavesPerBlock; k0 += 4) {
+                double W[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    W[j] = slice_value(model, size, rots + (size_t)(r0 + c0 + wave + kWavesPerBlock * (k0 + j)) * 9, q0,
+                                       q1, q2, cr, center);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int rr = wave + kWavesPerBlock * (k0 + j);
+                    s_tile[lane][rr] = W[j];
+                    const double x = (good && W[j] > 0.) ? table_log(W[j], s_logs) - ct : 0.;
+                    const T hi = to_op<T>(x);
+                    const size_t at = (size_t)(c0 + rr) * ldp + t;
+                    lw_hi[at] = hi;
+                    if (two_terms) lw_lo[at] = to_op<T>(x - from_op<T>(hi));
+                }
             }
         }
         __syncthreads();

@@ -892,7 +892,7 @@ __global__ __launch_bounds__(kBlock) void fused_expand_likelihood_kernel(
         __syncthreads();
         if (lt >= ntiles) break;  // every block leaves here once the tiles run out
         for (int g = 0; g < ngroups; ++g)
-            expand_block<T, kW, MT>(sh, lt * kRTile, g, rots, model, size, qvals, corr, mask, num_pix, r0, C,
+            expand_block<T, kW, MT, false>(sh, lt * kRTile, g, rots, model, size, qvals, corr, mask, num_pix, r0, C,
                                     pix_per_group, logw, upart, ubad, slot_rot, 1, 0);
         __threadfence();  // the tile's log W, written by every wave, is read below by every wave
         __syncthreads();
