@@ -211,7 +211,13 @@ std::vector<int> morton_order(int num_pix, const double *qvals) {
 }
 
 constexpr int kPixPerGroup = 1024;
-constexpr int kFramesPerPsumPart = 512;
+// Frames of one block of the psum_r partial sums (256 orientations): few enough for about eight
+// blocks a CU, at most 512 (each part is another row of num_rot partial sums). 3000 frames x 3240
+// orientations made 78 blocks at 512 and took 0.28 ms, now 0.06.
+int psum_part_frames(long frames, long num_rot) {
+    const long per = frames * ((num_rot + 255) / 256) / (8 * emc::kNumCus);
+    return (int)std::min(512L, std::max(16L, per));
+}
 constexpr int kFramesPerTomoPart = 12500;  // default of the full_part_frames option
 constexpr int kSigFullRowsPerTile = 1024;  // full-frame rows read by the pair tomogram, mean per tile
 constexpr int kMaxBucketRanges = 8192;     // pixel ranges of the pair tomogram's buckets (LDS counters)
@@ -1344,8 +1350,8 @@ int ensure_work(emc_engine *e) {
     if ((rc = e->rbad.alloc(Rp))) return rc;
     if ((rc = e->u.alloc(Rp))) return rc;
     if ((rc = e->psum_r.alloc(Rp))) return rc;
-    const size_t nparts = (N + kFramesPerPsumPart - 1) / kFramesPerPsumPart;
-    if ((rc = e->psum_part.alloc(nparts * (size_t)e->num_rot))) return rc;
+    const size_t per_psum = psum_part_frames(N, e->num_rot);
+    if ((rc = e->psum_part.alloc((N + per_psum - 1) / per_psum * (size_t)e->num_rot))) return rc;
     if ((rc = e->scalars.alloc(8))) return rc;
     if ((rc = e->model_part.alloc(kModelParts))) return rc;
     if ((rc = e->max_exp.alloc(N))) return rc;
@@ -1398,8 +1404,8 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
     if ((rc = e->Rsub.alloc((size_t)std::max<long>(e->num_pairs, 1) * emc::kRTile))) return rc;
     if (nF > 0) {
         if ((rc = e->RF.alloc((size_t)nF * T * emc::kRTile))) return rc;
-        const size_t pp = (nF + kFramesPerPsumPart - 1) / kFramesPerPsumPart;
-        if ((rc = e->psum_full_part.alloc(pp * (size_t)S))) return rc;
+        const size_t per_psum = psum_part_frames(nF, S);
+        if ((rc = e->psum_full_part.alloc((nF + per_psum - 1) / per_psum * (size_t)S))) return rc;
         if ((rc = e->psum_full.alloc(S))) return rc;
         if ((rc = e->scale_full.alloc(nF))) return rc;
         if ((rc = e->blacklist_full.alloc(nF))) return rc;
@@ -1637,7 +1643,7 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
                      if (nF > 0) {
                          emc::launch_frame_gather(s, e->scale.p, e->fidx.p, nF, e->scale_full.p);
                          emc::launch_frame_gather(s, e->blacklist.p, e->fidx.p, nF, e->blacklist_full.p);
-                         emc::launch_psum_r(s, e->RF.p, S, nF, kFramesPerPsumPart, e->scale_full.p, opts->need_scaling,
+                         emc::launch_psum_r(s, e->RF.p, S, nF, psum_part_frames(nF, S), e->scale_full.p, opts->need_scaling,
                                             e->blacklist_full.p, e->psum_full_part.p, e->psum_full.p);
                      }
                      emc::launch_pair_psum(s, e->Rsub.p, e->tile_off.p, e->tile_pair.p, e->pair_frame.p, T, e->scale.p,
@@ -2884,7 +2890,7 @@ int emc_maximize(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *stats
         if ((rc = e->quat_norm.alloc((size_t)N * M))) return rc;
         emc::launch_occupancy(s, e->R.p, Rn, N, M, e->quat_norm.p);
     }
-    emc::launch_psum_r(s, e->R.p, Rn, N, kFramesPerPsumPart, e->scale.p, opts->need_scaling,
+    emc::launch_psum_r(s, e->R.p, Rn, N, psum_part_frames(N, Rn), e->scale.p, opts->need_scaling,
                        e->blacklist.p, e->psum_part.p, e->psum_r.p);
     if (bgp) {
         // calc_psum_r's scalemax per orientation, for the background-aware tomogram

@@ -481,11 +481,14 @@ __global__ __launch_bounds__(kBlock) void psum_r_partial_kernel(
     const int part_id = blockIdx.y;
     if (r >= num_rot) return;
     const int d0 = part_id * frames_per_part, d1 = min(num_data, d0 + frames_per_part);
+    const double *__restrict__ col = P + (size_t)(r >> 6) * tsP + (r & 63);
     double acc = 0.;
+    // a blacklisted frame's row is zero and its factor (which may be anything) is left out; no
+    // branch, so that eight rows are in flight
+#pragma unroll 8
     for (int d = d0; d < d1; ++d) {
-        if (blacklist[d]) continue;
-        const double p = P[(size_t)(r >> 6) * tsP + (size_t)d * kRTile + (r & 63)];
-        acc += need_scaling ? p * scale[d] : p;
+        const double f = blacklist[d] ? 0. : (need_scaling ? scale[d] : 1.);
+        acc += col[(size_t)d * kRTile] * f;
     }
     part[(size_t)part_id * num_rot + r] = acc;
 }
