@@ -467,14 +467,14 @@ struct emc_engine {
     bool slot_bricks_valid = false;
     // frame photon lists of mask < 2 pixels sorted by engine pixel, with per-range offsets
     bool fsort_valid = false;
-    int nranges = 0;
+    int nranges = 0, bucket_nr = 0, bucket_bits = 6;
     DevBuf<long> fsort_off;
     DevBuf<int> fsort_pix, fsort_roff;
     DevBuf<double> fsort_cnt;
-    // each frame's distinct pixel ranges (fsort order): fr_off per frame, the range and its
-    // photons [fr_q0, fr_q1) per entry; and the pair tomogram's per-(tile, range) buckets
-    DevBuf<long> fr_off, fr_q0, fr_q1, bk_tot, bk_base;
-    DevBuf<int> fr_rg, bk_loc, bk_pair, bk_fr;
+    // the pair tomogram's per-(tile, range) buckets
+    DevBuf<long> bk_tot, bk_base;
+    DevBuf<int> bk_loc;
+    DevBuf<int2> bk_photon;
 
 };
 
@@ -1154,8 +1154,8 @@ int build_fsort(emc_engine *e) {
     const int N = e->num_data, P = e->num_pix;
     const int nr = (P + emc::kPairRange - 1) / emc::kPairRange;
     const uint8_t *mask = e->h_mask.data();
-    std::vector<long> off(N + 1, 0), r_off(N + 1, 0), r_q0, r_q1;
-    std::vector<int> pix, roff((size_t)N * (nr + 1)), r_rg;
+    std::vector<long> off(N + 1, 0);
+    std::vector<int> pix, roff((size_t)N * (nr + 1));
     std::vector<double> cnt;
     std::vector<std::pair<int, double>> fr;
     for (int d = 0; d < N; ++d) {
@@ -1175,28 +1175,11 @@ int build_fsort(emc_engine *e) {
             while (q < (int)fr.size() && fr[q].first < rg * emc::kPairRange) ++q;
             roff[(size_t)d * (nr + 1) + rg] = q;
         }
-        // the frame's distinct ranges and their photons
-        const long base = (long)pix.size();
-        for (size_t a = 0; a < fr.size();) {
-            const int rg = fr[a].first / emc::kPairRange;
-            size_t b = a + 1;
-            while (b < fr.size() && fr[b].first / emc::kPairRange == rg) ++b;
-            r_rg.push_back(rg);
-            r_q0.push_back(base + (long)a);
-            r_q1.push_back(base + (long)b);
-            a = b;
-        }
-        r_off[d + 1] = (long)r_rg.size();
         for (const auto &x : fr) {
             pix.push_back(x.first);
             cnt.push_back(x.second);
         }
         off[d + 1] = (long)pix.size();
-    }
-    if (r_rg.empty()) {
-        r_rg.push_back(0);
-        r_q0.push_back(0);
-        r_q1.push_back(0);
     }
     if (pix.empty()) {
         pix.push_back(0);
@@ -1208,11 +1191,11 @@ int build_fsort(emc_engine *e) {
     if ((rc = e->fsort_pix.upload(pix.data(), pix.size(), s))) return rc;
     if ((rc = e->fsort_cnt.upload(cnt.data(), cnt.size(), s))) return rc;
     if ((rc = e->fsort_roff.upload(roff.data(), roff.size(), s))) return rc;
-    if ((rc = e->fr_off.upload(r_off.data(), r_off.size(), s)) || (rc = e->fr_rg.upload(r_rg.data(), r_rg.size(), s)) ||
-        (rc = e->fr_q0.upload(r_q0.data(), r_q0.size(), s)) || (rc = e->fr_q1.upload(r_q1.data(), r_q1.size(), s)))
-        return rc;
     HIP_TRY(hipStreamSynchronize(s));
     e->nranges = nr;
+    // the buckets' ranges: 16 pixels, or whole patches where those would be too many to count in LDS
+    e->bucket_bits = nr * 4 <= kMaxBucketRanges ? 4 : 6;
+    e->bucket_nr = nr << (6 - e->bucket_bits);
     e->fsort_valid = true;
     return 0;
 }
@@ -1729,34 +1712,31 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
         const bool parts = nF > 0 && !sig_full;
         e->nz_counted = false;
         emc::launch_zero_u64(s, e->nz_count.p);
-        // per-(tile, range) buckets of the significant pairs' photons (eager only: their size is
-        // read back; without room for them the blocks walk their tiles' pairs instead)
+        // per-(tile, range) buckets of the significant rows' photons (eager only: their size is
+        // read back; without room for them the blocks walk their tiles' rows instead)
         emc::PairBuckets bkv;
-        if (e->tomo_buckets && !device_weights && !sig_full && e->nranges <= kMaxBucketRanges) {
-            const int nr = e->nranges;
+        if (e->tomo_buckets && !device_weights && e->bucket_nr <= kMaxBucketRanges) {
+            const int nr = e->bucket_nr;
             if ((rc = timed(7, [&]() -> int {
                      int r2;
                      if ((r2 = e->bk_loc.alloc((size_t)T * (nr + 1))) || (r2 = e->bk_tot.alloc((size_t)T)) ||
                          (r2 = e->bk_base.alloc((size_t)T + 1)))
                          return r2;
-                     emc::launch_pair_buckets(s, T, e->tile_off.p, e->sig_pair.p, e->sig_frame.p, e->sig_cnt.p,
-                                              e->fr_off.p, e->fr_rg.p, nr, e->bk_loc.p, e->bk_tot.p, e->bk_base.p,
-                                              nullptr, nullptr, 0);
+                     emc::launch_pair_buckets(s, T, e->tile_off.p, e->sig_pair.p, e->sig_frame.p, e->sig_cnt.p, frows,
+                                              e->fsort_off.p, e->fsort_pix.p, e->fsort_cnt.p, nr, e->bucket_bits, e->bk_loc.p, e->bk_tot.p, e->bk_base.p,
+                                              nullptr, 0);
                      HIP_TRY(hipGetLastError());
                      long total = 0;
                      HIP_TRY(hipMemcpyAsync(&total, e->bk_base.p + T, sizeof(long), hipMemcpyDeviceToHost, s));
                      HIP_TRY(hipStreamSynchronize(s));
-                     const size_t n = (size_t)std::max(total, 1L);
-                     if (e->bk_pair.alloc(n) || e->bk_fr.alloc(n)) {
-                         e->bk_pair.release();  // no room: the blocks walk their tiles' pairs
-                         e->bk_fr.release();
-                         return 0;
-                     }
-                     emc::launch_pair_buckets(s, T, e->tile_off.p, e->sig_pair.p, e->sig_frame.p, e->sig_cnt.p,
-                                              e->fr_off.p, e->fr_rg.p, nr, e->bk_loc.p, e->bk_tot.p, e->bk_base.p,
-                                              e->bk_pair.p, e->bk_fr.p, 1);
+                     // no room, or a tile too full: the blocks walk their tiles' pairs
+                     if (total < 0 || e->bk_photon.alloc((size_t)std::max(total, 1L))) return 0;
+                     emc::launch_pair_buckets(s, T, e->tile_off.p, e->sig_pair.p, e->sig_frame.p, e->sig_cnt.p, frows,
+                                              e->fsort_off.p, e->fsort_pix.p, e->fsort_cnt.p, nr, e->bucket_bits, e->bk_loc.p, e->bk_tot.p, e->bk_base.p,
+                                              e->bk_photon.p, 1);
                      HIP_TRY(hipGetLastError());
-                     bkv = emc::PairBuckets{e->bk_base.p, e->bk_loc.p, e->bk_pair.p, e->bk_fr.p, e->fr_q0.p, e->fr_q1.p};
+                     bkv = emc::PairBuckets{e->bk_base.p, e->bk_loc.p, e->bk_photon.p, nr, 1 << (6 - e->bucket_bits),
+                                            total / std::max(T, 1)};
                      return 0;
                  })))
                 return rc;

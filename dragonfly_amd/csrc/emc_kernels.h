@@ -254,22 +254,6 @@ void launch_pair_posterior(hipStream_t s, double *R, const long *pair_off, const
 void launch_pair_psum(hipStream_t s, const double *P, const long *tile_off, const int *tile_pair,
                       const int *pair_frame, int num_tiles, const double *scale, int need_scaling,
                       const double *psum_full, double *psum_slot);
-// Per-(tile, range) buckets of the significant pairs' frame ranges (launch_pair_buckets), read
-// by the pair tomogram instead of walking each tile's pairs; base null: none.
-struct PairBuckets {
-    const long *base = nullptr;  // [num_tiles + 1] first entry of each tile
-    const int *loc = nullptr;    // [num_tiles][nranges + 1] offsets of the ranges in their tile
-    const int *pair = nullptr, *fr = nullptr;  // entries: pair, frame range
-    const long *q0 = nullptr, *q1 = nullptr;   // frame range f: photons [q0[f], q1[f])
-};
-// pass 0: counts into loc (and each tile's total), then base; pass 1: the entries
-// (bk_pair / bk_fr sized base[num_tiles]). Dynamic LDS of (nr + 1) ints per block.
-void launch_pair_buckets(hipStream_t s, int num_tiles, const long *tile_off, const int *sig_pair,
-                         const int *sig_frame, const int *sig_cnt, const long *fr_off, const int *fr_rg, int nr,
-                         int *loc, long *tile_tot, long *base, int *bk_pair, int *bk_fr, int pass);
-// *x = 0; *total += set bits of m[0 .. n)
-void launch_zero_u64(hipStream_t s, unsigned long long *x);
-void launch_popcount(hipStream_t s, const unsigned long long *m, size_t n, unsigned long long *total);
 // Significant full-frame rows per tile (launch_sig_full_rows), read by the pair tomogram from
 // RF in place of partial sums; RF null: none.
 struct SigFullRows {
@@ -277,6 +261,25 @@ struct SigFullRows {
     int nF = 0;
     const int *row = nullptr, *frame = nullptr, *cnt = nullptr;
 };
+// Per-(tile, range) buckets of the significant rows' photons (launch_pair_buckets), read by the
+// pair tomogram instead of walking each tile's rows; base null: none.
+struct PairBuckets {
+    const long *base = nullptr;  // [num_tiles + 1] first entry of each tile
+    const int *loc = nullptr;    // [num_tiles][nr + 1] offsets of the ranges in their tile
+    const int2 *photon = nullptr;  // entries: row (pair, or ~full row), pixel in the patch | count << 6
+    int nr = 0, sub = 1;           // ranges: sub (4 or 1) of equal size to every 64-pixel patch
+    long per_tile = 0;             // entries of a tile, on average
+};
+// pass 0: counts into loc (and each tile's total), then base (base[num_tiles] = -1: some tile holds
+// more than INT_MAX entries, no buckets); pass 1: the entries (photon sized base[num_tiles]).
+// Dynamic LDS of (nr + 1) ints per block.
+void launch_pair_buckets(hipStream_t s, int num_tiles, const long *tile_off, const int *sig_pair,
+                         const int *sig_frame, const int *sig_cnt, const SigFullRows &fr, const long *foff,
+                         const int *fpix, const double *fcnt, int nr, int bits, int *loc, long *tile_tot, long *base,
+                         int2 *photon, int pass);
+// *x = 0; *total += set bits of m[0 .. n)
+void launch_zero_u64(hipStream_t s, unsigned long long *x);
+void launch_popcount(hipStream_t s, const unsigned long long *m, size_t n, unsigned long long *total);
 // flag: num_tiles * nF bytes; sigF_row / sigF_frame: num_tiles * nF; sigF_cnt: num_tiles;
 // total: the sum of sigF_cnt
 void launch_sig_full_rows(hipStream_t s, const double *RF, int nF, int num_tiles, const int *fidx, uint8_t *flag,

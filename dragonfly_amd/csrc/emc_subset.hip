@@ -20,6 +20,8 @@
 // across frames in psum_r and the tomogram differs from the reference.
 #include <algorithm>
 #include <cfloat>
+#include <climits>
+#include <type_traits>
 
 #include "emc_common.h"
 #include "emc_expand.h"
@@ -438,48 +440,59 @@ __global__ __launch_bounds__(kBlock) void sum_counts_kernel(const int *__restric
     if (threadIdx.x == 0) *total = s[0];
 }
 
-// Per-(tile, pixel range) buckets of the significant pairs' photons, so that a pair-tomogram
-// block reads only the entries of its own range instead of every pair of its tile: an entry
-// is (pair, frame range f), the frame's photons [fr_q0[f], fr_q1[f]) in range fr_rg[f] (the
-// frame's distinct ranges, fsort order). Count: one block per tile, LDS counters per range
-// (nr + 1 of them, dynamic LDS), then their exclusive scan: loc[T * (nr + 1) + rg] and the
-// tile's total.
-__global__ __launch_bounds__(kBlock) void bucket_count_kernel(const long *__restrict__ tile_off,
-                                                              const int *__restrict__ sig_frame,
-                                                              const int *__restrict__ sig_cnt,
-                                                              const long *__restrict__ fr_off,
-                                                              const int *__restrict__ fr_rg, int nr,
-                                                              int *__restrict__ loc, long *__restrict__ tile_tot) {
-    extern __shared__ int cnt[];
-    __shared__ int part[kBlock];
-    const int T = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    for (int i = tid; i <= nr; i += kBlock) cnt[i] = 0;
-    __syncthreads();
+// Per-(tile, pixel range) buckets of the significant rows' photons, so that a pair-tomogram block
+// reads only the photons of its own range of 2^bits pixels, each as one entry {row, pixel in its
+// 64-pixel patch | count << 6}; row: the pair, or ~f for row f of the tile's full frames. Two walks over
+// a tile's rows, one block a tile (a wave a row, lanes along its frame's photons): count, in LDS
+// counters (nr + 1, dynamic), and their exclusive scan loc[T * (nr + 1) + rg] with the tile's
+// total; then the entries.
+constexpr int kBucketThreads = 1024;
+
+// The tile's significant rows: pairs, then full-frame rows (sigF_*, nullable): fn(row, frame).
+template <typename F>
+__device__ __forceinline__ void for_each_sig_row(int T, const long *__restrict__ tile_off,
+                                                 const int *__restrict__ sig_pair, const int *__restrict__ sig_frame,
+                                                 const int *__restrict__ sig_cnt, const SigFullRows &fr, F &&fn) {
     const long j0 = tile_off[T];
-    const int n = sig_cnt[T];
-    for (int i = wave; i < n; i += kWavesPerBlock) {
-        const int d = sig_frame[j0 + i];
-        for (long f = fr_off[d] + lane; f < fr_off[d + 1]; f += 64) atomicAdd(&cnt[fr_rg[f]], 1);
+    const size_t f0 = (size_t)T * fr.nF;
+    const int nP = sig_cnt[T], n = nP + (fr.cnt ? fr.cnt[T] : 0);
+    for (int i = threadIdx.x >> 6; i < n; i += kBucketThreads / 64) {
+        if (i < nP) fn(sig_pair[j0 + i], sig_frame[j0 + i]);
+        else fn(~fr.row[f0 + i - nP], fr.frame[f0 + i - nP]);
     }
+}
+
+__global__ __launch_bounds__(kBucketThreads) void bucket_count_kernel(
+    const long *__restrict__ tile_off, const int *__restrict__ sig_pair, const int *__restrict__ sig_frame,
+    const int *__restrict__ sig_cnt, const SigFullRows fr, const long *__restrict__ foff, const int *__restrict__ fpix,
+    int nr, int bits, int *__restrict__ loc, long *__restrict__ tile_tot) {
+    extern __shared__ int cnt[];
+    __shared__ long part[kBucketThreads];
+    const int T = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    for (int i = tid; i <= nr; i += kBucketThreads) cnt[i] = 0;
+    __syncthreads();
+    for_each_sig_row(T, tile_off, sig_pair, sig_frame, sig_cnt, fr, [&](int, int d) {
+        const long q1 = foff[d + 1];
+        for (long q = foff[d] + lane; q < q1; q += 64) atomicAdd(&cnt[fpix[q] >> bits], 1);
+    });
     __syncthreads();
     // exclusive scan of cnt[0 .. nr): each thread a chunk, then the chunks' totals
-    const int per = (nr + kBlock - 1) / kBlock, a = tid * per, b = min(nr, a + per);
-    int sum = 0;
+    const int per = (nr + kBucketThreads - 1) / kBucketThreads, a = min(nr, tid * per), b = min(nr, a + per);
+    long sum = 0;
     for (int i = a; i < b; ++i) sum += cnt[i];
     part[tid] = sum;
     __syncthreads();
-    if (tid == 0) {
-        int run = 0;
-        for (int w = 0; w < kBlock; ++w) {
-            const int v = part[w];
-            part[w] = run;
-            run += v;
-        }
-        tile_tot[T] = run;
-        loc[(size_t)T * (nr + 1) + nr] = run;
+    for (int w = 1; w < kBucketThreads; w <<= 1) {
+        const long v = tid >= w ? part[tid - w] : 0;
+        __syncthreads();
+        part[tid] += v;
+        __syncthreads();
     }
-    __syncthreads();
-    int run = part[tid];
+    if (tid == kBucketThreads - 1) {
+        tile_tot[T] = part[tid];
+        loc[(size_t)T * (nr + 1) + nr] = (int)part[tid];
+    }
+    int run = (int)(part[tid] - sum);
     for (int i = a; i < b; ++i) {
         const int v = cnt[i];
         loc[(size_t)T * (nr + 1) + i] = run;
@@ -487,12 +500,19 @@ __global__ __launch_bounds__(kBlock) void bucket_count_kernel(const long *__rest
     }
 }
 
-// base[0] = 0, base[t + 1] = base[t] + tot[t] (one block)
+// base[0] = 0, base[t + 1] = base[t] + tot[t]; base[n] = -1 when a tile holds more entries than its
+// 32-bit offsets count (one block)
 __global__ __launch_bounds__(kBlock) void tile_scan_kernel(const long *__restrict__ tot, int n, long *__restrict__ base) {
     __shared__ long part[kBlock];
+    __shared__ int s_big;
     const int tid = threadIdx.x, per = (n + kBlock - 1) / kBlock, a = tid * per, b = min(n, a + per);
+    if (tid == 0) s_big = 0;
+    __syncthreads();
     long sum = 0;
-    for (int i = a; i < b; ++i) sum += tot[i];
+    for (int i = a; i < b; ++i) {
+        sum += tot[i];
+        if (tot[i] > INT_MAX) s_big = 1;
+    }
     part[tid] = sum;
     __syncthreads();
     if (tid == 0) {
@@ -502,7 +522,7 @@ __global__ __launch_bounds__(kBlock) void tile_scan_kernel(const long *__restric
             part[w] = run;
             run += v;
         }
-        base[n] = run;
+        base[n] = s_big ? -1 : run;
     }
     __syncthreads();
     long run = part[tid];
@@ -513,55 +533,58 @@ __global__ __launch_bounds__(kBlock) void tile_scan_kernel(const long *__restric
 }
 
 // Fill: the same walk, each entry at base[T] + loc[T][rg] + (its rank, from LDS counters)
-__global__ __launch_bounds__(kBlock) void bucket_fill_kernel(const long *__restrict__ tile_off,
-                                                             const int *__restrict__ sig_pair,
-                                                             const int *__restrict__ sig_frame,
-                                                             const int *__restrict__ sig_cnt,
-                                                             const long *__restrict__ fr_off,
-                                                             const int *__restrict__ fr_rg, int nr,
-                                                             const int *__restrict__ loc, const long *__restrict__ base,
-                                                             int *__restrict__ bk_pair, int *__restrict__ bk_fr) {
+__global__ __launch_bounds__(kBucketThreads) void bucket_fill_kernel(
+    const long *__restrict__ tile_off, const int *__restrict__ sig_pair, const int *__restrict__ sig_frame,
+    const int *__restrict__ sig_cnt, const SigFullRows fr, const long *__restrict__ foff, const int *__restrict__ fpix,
+    const double *__restrict__ fcnt, int nr, int bits, const int *__restrict__ loc, const long *__restrict__ base,
+    int2 *__restrict__ photon) {
     extern __shared__ int fill[];
-    const int T = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    for (int i = tid; i < nr; i += kBlock) fill[i] = loc[(size_t)T * (nr + 1) + i];
+    const int T = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    for (int i = tid; i < nr; i += kBucketThreads) fill[i] = loc[(size_t)T * (nr + 1) + i];
     __syncthreads();
-    const long j0 = tile_off[T], b0 = base[T];
-    const int n = sig_cnt[T];
-    for (int i = wave; i < n; i += kWavesPerBlock) {
-        const int k = sig_pair[j0 + i], d = sig_frame[j0 + i];
-        for (long f = fr_off[d] + lane; f < fr_off[d + 1]; f += 64) {
-            const long at = b0 + atomicAdd(&fill[fr_rg[f]], 1);
-            bk_pair[at] = k;
-            bk_fr[at] = (int)f;
+    int2 *__restrict__ out = photon + base[T];
+    for_each_sig_row(T, tile_off, sig_pair, sig_frame, sig_cnt, fr, [&](int row, int d) {
+        const long q1 = foff[d + 1];
+        for (long q = foff[d] + lane; q < q1; q += 64) {
+            const int p = fpix[q];
+            out[atomicAdd(&fill[p >> bits], 1)] = make_int2(row, p % kPairRange | (int)fcnt[q] * kPairRange);
         }
-    }
+    });
 }
 
 void launch_pair_buckets(hipStream_t s, int num_tiles, const long *tile_off, const int *sig_pair,
-                         const int *sig_frame, const int *sig_cnt, const long *fr_off, const int *fr_rg, int nr,
-                         int *loc, long *tile_tot, long *base, int *bk_pair, int *bk_fr, int pass) {
+                         const int *sig_frame, const int *sig_cnt, const SigFullRows &fr, const long *foff,
+                         const int *fpix, const double *fcnt, int nr, int bits, int *loc, long *tile_tot, long *base,
+                         int2 *photon, int pass) {
     if (num_tiles <= 0) return;
     const size_t lds = (size_t)(nr + 1) * sizeof(int);
     if (pass == 0) {
-        bucket_count_kernel<<<num_tiles, kBlock, lds, s>>>(tile_off, sig_frame, sig_cnt, fr_off, fr_rg, nr, loc,
-                                                          tile_tot);
+        bucket_count_kernel<<<num_tiles, kBucketThreads, lds, s>>>(tile_off, sig_pair, sig_frame, sig_cnt, fr, foff,
+                                                                  fpix, nr, bits, loc, tile_tot);
         tile_scan_kernel<<<1, kBlock, 0, s>>>(tile_tot, num_tiles, base);
     } else {
-        bucket_fill_kernel<<<num_tiles, kBlock, lds, s>>>(tile_off, sig_pair, sig_frame, sig_cnt, fr_off, fr_rg, nr,
-                                                         loc, base, bk_pair, bk_fr);
+        bucket_fill_kernel<<<num_tiles, kBucketThreads, lds, s>>>(tile_off, sig_pair, sig_frame, sig_cnt, fr, foff,
+                                                                 fpix, fcnt, nr, bits, loc, base, photon);
     }
 }
 
-// Tomogram of the chunk's tiles [t0, t0 + ntiles) over pixel ranges of kPairRange pixels:
+// Tomogram of the chunk's tiles [t0, t0 + ntiles) over pixel ranges of 2^kBits pixels:
 // block (tile, range) starts from the full frames' sums partial[tile][t][64] or from zero,
 // adds K * P (P > 1e-6) of the tile's significant partial-frame pairs (sig_pair, sig_cnt)
 // and, with RF, of its significant full-frame rows (sigF_*: rows RF[T][f][64], in place of the
 // partial sums) into LDS rows of the range's pixels (frame photon lists sorted by pixel, range
 // offsets roff[d][range]), divides by psum and writes the orientation-major
-// view[(T - t0) * 64 + j][t] (VT: double, or float for the FP32-sum merge). The tile's rows
-// are examined kBlock at a time, one per thread, and only those with photons in the range are
-// queued for the waves, so a row costs one read per range it has photons in.
-template <typename TP, typename VT, typename PT>
+// view[(T - t0) * 64 + j][t] (VT: double, or float where the merge reads an FP32 view).
+// With kBuckets a block's photons come as one list: a wave reads 64 entries at once, spreads them
+// by lane reads, and has the P rows of 16 photons in flight before it adds any; a photon costs one
+// 512-byte (FP32: 256) row from L2 and one ds_add_f64, which is what bounds it (15 cycles a wave).
+// The sums are FP64 for FP32 views too: ds_add_f32 takes 193 cycles. Entries per (pair, range) with
+// a chain of loads to their photons, and FP32 sums, took 20.5 ms for 40,000 frames of 247 photons
+// in 30 tiles each (and 2.3 for their buckets), now 12.2 (2.8); with FP32 gathers 36.2 in all, now 14.4.
+// Without (inside a graph, or no room for the lists) the tile's rows are examined kBlock at a time,
+// one per thread, and only those with photons in the range are queued for the waves, so a row
+// costs one read per range it has photons in.
+template <bool kBuckets, int kBits, bool kFull, typename TP, typename VT, typename PT>
 __global__ __launch_bounds__(kBlock) void pair_tomogram_kernel(
     const TP *__restrict__ P, const long *__restrict__ tile_off, const int *__restrict__ tile_pair,
     const int *__restrict__ tile_frame, const int *__restrict__ sig_cnt, const long *__restrict__ foff,
@@ -571,14 +594,16 @@ __global__ __launch_bounds__(kBlock) void pair_tomogram_kernel(
     unsigned long long *__restrict__ nzmask, const double *__restrict__ RF, int nF,
     const int *__restrict__ sigF_row, const int *__restrict__ sigF_frame, const int *__restrict__ sigF_cnt,
     const PairBuckets bk) {
-    static_assert(kPairRange == 64, "a pixel range is one 64-pixel merge patch");
-    // LDS sums in the view's type: FP64 for an FP64 view, FP32 for an FP32 one (half the LDS,
-    // more resident blocks; each sum has a few terms and is stored in FP32 anyway)
-    using A = VT;
-    __shared__ A acc[kPairRange][kRTile + 1];
-    __shared__ long s_row[kBlock];  // element offset of the row (P or RF)
-    __shared__ bool s_full[kBlock];
-    __shared__ long s_q0[kBlock], s_q1[kBlock];
+    // a range is a 64-pixel merge patch, or a quarter of one: 16 pixels keep the brightest block's
+    // photons near those of the others (a block that outlasts its tile brings the next tile's rows
+    // into the L2) and let five blocks share a CU
+    constexpr int kPix = 1 << kBits, kParts = 64 / kPix, kQueue = kBuckets ? 1 : kBlock;
+    using Mask = typename std::conditional<kBits == 6, unsigned long long, unsigned short>::type;
+    static_assert(kPix == 64 || (kBuckets && kPix == 16), "nonzero masks are written by the range");
+    __shared__ double acc[kPix][kRTile + 1];
+    __shared__ long s_row[kQueue];  // element offset of the row (P or RF)
+    __shared__ bool s_full[kQueue];
+    __shared__ long s_q0[kQueue], s_q1[kQueue];
     __shared__ int s_n;
     // XCD-aware order: workgroups go round-robin to the kNumXcd XCDs, so XCD x takes tiles
     // x, x + kNumXcd, ... one at a time, all ranges of a tile together, and its L2 keeps the
@@ -591,130 +616,150 @@ __global__ __launch_bounds__(kBlock) void pair_tomogram_kernel(
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int npatch = (num_pix + 63) / 64;
     const bool rows_full = RF != nullptr;
-    if (j0 == tile_off[T + 1] && !partial && !rows_full) {
-        // no frame takes this tile: psum 0, views 0 (unwritten), the merge skips the items
-        if (nzmask && tid < kRTile) nzmask[((size_t)lt * kRTile + tid) * npatch + rg] = 0ull;
+    // the range's bits of a slot's nonzero mask
+    Mask *__restrict__ nz = nzmask ? reinterpret_cast<Mask *>(nzmask) + (size_t)lt * kRTile * npatch * kParts + rg : nullptr;
+    const int2 *__restrict__ photon = nullptr;
+    int n_photon = 0;
+    bool empty = j0 == tile_off[T + 1] && !rows_full;  // no frame takes this tile: psum 0, views 0
+    if constexpr (kBuckets) {
+        const int *loc = bk.loc + (size_t)T * (bk.nr + 1) + rg * (bk.sub / kParts);
+        photon = bk.photon + bk.base[T] + loc[0];
+        n_photon = loc[bk.sub / kParts] - loc[0];
+        empty |= n_photon == 0;
+    }
+    if (empty && !partial && nz) {
+        // zero views are not written, the merge skips them
+        if (tid < kRTile) nz[(size_t)tid * npatch * kParts] = (Mask)0;
         return;
     }
-    // with buckets: this (tile, range)'s entries [e0, e0 + nRows); else every significant row
-    // of the tile, filtered below by its photons in the range
-    const bool buckets = bk.base != nullptr;
-    long e0 = 0, nP, nRows;
-    if (buckets) {
-        const int *loc = bk.loc + (size_t)T * (nranges + 1);
-        e0 = bk.base[T] + loc[rg];
-        nP = nRows = loc[rg + 1] - loc[rg];
-    } else {
-        nP = sig_cnt[T];
-        nRows = nP + (rows_full ? sigF_cnt[T] : 0);
+    // psum of the tile's slots (FP32 views: its reciprocal, one division per slot)
+    __shared__ double s_ps[kRTile], s_inv[kRTile];
+    if (tid < kRTile) {
+        const double ps = psum_slot[(size_t)T * kRTile + tid];
+        s_ps[tid] = ps;
+        s_inv[tid] = ps > 0. ? 1. / ps : 1.;
     }
     const size_t frow0 = (size_t)T * nF;
-    const int p0 = rg * kPairRange;
+    const int p0 = rg * kPix;
     if (partial) {
         const size_t tsW = (size_t)num_pix * kRTile;
-        for (int i = wave; i < kPairRange; i += kWavesPerBlock) {
+        for (int i = wave; i < kPix; i += kWavesPerBlock) {
             const int t = p0 + i;
             double a = 0.;
             if (t < num_pix) {
                 a = (double)partial[(size_t)lt * tsW + (size_t)t * kRTile + lane];
             }
-            acc[i][lane] = (A)a;
+            acc[i][lane] = a;
         }
     } else {
-        for (int i = tid; i < kPairRange * (kRTile + 1); i += kBlock) (&acc[0][0])[i] = (A)0;
+        for (int i = tid; i < kPix * (kRTile + 1); i += kBlock) (&acc[0][0])[i] = 0.;
     }
-    for (long jb = 0; jb < nRows; jb += kBlock) {
-        if (tid == 0) s_n = 0;
+    if constexpr (kBuckets) {
         __syncthreads();
-        const long j = jb + tid;
-        if (buckets) {
+        constexpr int kAhead = 16;
+        for (int jb = wave * 64; jb < n_photon; jb += kWavesPerBlock * 64) {
+            const int m = min(64, n_photon - jb);
+            int2 e = make_int2(0, 0);
+            if (lane < m) e = photon[jb + lane];
+            for (int i = 0; i < m; i += kAhead) {
+                double p[kAhead];
+                int code[kAhead];
+#pragma unroll
+                for (int u = 0; u < kAhead; ++u) {
+                    p[u] = 0.;
+                    code[u] = 0;
+                    if (i + u < m) {
+                        code[u] = __builtin_amdgcn_readlane(e.y, i + u);
+                        const int row = __builtin_amdgcn_readlane(e.x, i + u);
+                        if (kFull && row < 0) p[u] = RF[(frow0 + ~row) * kRTile + lane];
+                        else p[u] = (double)P[(size_t)row * kRTile + lane];
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < kAhead; ++u)
+                    if (p[u] > kProbMin)
+                        unsafeAtomicAdd(&acc[code[u] % kPix][lane], (double)((unsigned)code[u] / kPairRange) * p[u]);
+            }
+        }
+    } else {
+        // every significant row of the tile, filtered by its photons in the range
+        const long nP = sig_cnt[T], nRows = nP + (rows_full ? sigF_cnt[T] : 0);
+        for (long jb = 0; jb < nRows; jb += kBlock) {
+            if (tid == 0) s_n = 0;
+            __syncthreads();
+            const long j = jb + tid;
             if (j < nRows) {
-                // every entry has photons in the range: its queue position is its own
-                const int f = bk.fr[e0 + j];
-                s_row[tid] = (long)bk.pair[e0 + j] * kRTile;
-                s_full[tid] = false;
-                s_q0[tid] = bk.q0[f];
-                s_q1[tid] = bk.q1[f];
+                long row;
+                int d;
+                const bool full = j >= nP;
+                if (!full) {
+                    row = (long)tile_pair[j0 + j] * kRTile;
+                    d = tile_frame[j0 + j];
+                } else {
+                    const size_t i = frow0 + (size_t)(j - nP);
+                    row = ((long)frow0 + sigF_row[i]) * kRTile;
+                    d = sigF_frame[i];
+                }
+                const int *__restrict__ rr = roff + (size_t)d * (nranges + 1);
+                const int q0 = rr[rg], q1 = rr[rg + 1];
+                if (q0 < q1) {
+                    const int at = atomicAdd(&s_n, 1);
+                    s_row[at] = row;
+                    s_full[at] = full;
+                    s_q0[at] = foff[d] + q0;
+                    s_q1[at] = foff[d] + q1;
+                }
             }
-            if (tid == 0) s_n = (int)min((long)kBlock, nRows - jb);
-        } else if (j < nRows) {
-            long row;
-            int d;
-            const bool full = j >= nP;
-            if (!full) {
-                row = (long)tile_pair[j0 + j] * kRTile;
-                d = tile_frame[j0 + j];
-            } else {
-                const size_t i = frow0 + (size_t)(j - nP);
-                row = ((long)frow0 + sigF_row[i]) * kRTile;
-                d = sigF_frame[i];
-            }
-            const int *__restrict__ rr = roff + (size_t)d * (nranges + 1);
-            const int q0 = rr[rg], q1 = rr[rg + 1];
-            if (q0 < q1) {
-                const int at = atomicAdd(&s_n, 1);
-                s_row[at] = row;
-                s_full[at] = full;
-                s_q0[at] = foff[d] + q0;
-                s_q1[at] = foff[d] + q1;
-            }
-        }
-        __syncthreads();
-        const int n = s_n;
-        // the P rows and first photons (a frame has about one photon in a 128-pixel range) of
-        // kQueueRows queue entries are loaded before any is added, so a wave has that many
-        // reads in flight instead of one chain of dependent ones
-        constexpr int kQueueRows = 8;
-        for (int i0 = wave; i0 < n; i0 += kWavesPerBlock * kQueueRows) {
-            double p[kQueueRows], c0[kQueueRows];
-            int px0[kQueueRows];
-            long qa[kQueueRows], qb[kQueueRows];
+            __syncthreads();
+            const int n = s_n;
+            // the P rows and first photons (a frame has about one photon in a 128-pixel range) of
+            // kQueueRows queue entries are loaded before any is added, so a wave has that many
+            // reads in flight instead of one chain of dependent ones
+            constexpr int kQueueRows = 8;
+            for (int i0 = wave; i0 < n; i0 += kWavesPerBlock * kQueueRows) {
+                double p[kQueueRows], c0[kQueueRows];
+                int px0[kQueueRows];
+                long qa[kQueueRows], qb[kQueueRows];
 #pragma unroll
-            for (int u = 0; u < kQueueRows; ++u) {
-                const int i = i0 + u * kWavesPerBlock;
-                qa[u] = i < n ? s_q0[i] : 0;
-                qb[u] = i < n ? s_q1[i] : 0;
-                p[u] = i < n ? (s_full[i] ? RF[s_row[i] + lane] : (double)P[s_row[i] + lane]) : 0.;
-                px0[u] = i < n ? fpix[qa[u]] : 0;
-                c0[u] = i < n ? fcnt[qa[u]] : 0.;
-            }
+                for (int u = 0; u < kQueueRows; ++u) {
+                    const int i = i0 + u * kWavesPerBlock;
+                    qa[u] = i < n ? s_q0[i] : 0;
+                    qb[u] = i < n ? s_q1[i] : 0;
+                    p[u] = i < n ? (s_full[i] ? RF[s_row[i] + lane] : (double)P[s_row[i] + lane]) : 0.;
+                    px0[u] = i < n ? fpix[qa[u]] : 0;
+                    c0[u] = i < n ? fcnt[qa[u]] : 0.;
+                }
 #pragma unroll
-            for (int u = 0; u < kQueueRows; ++u) {
-                if (!(p[u] > kProbMin)) continue;  // also the entries past the queue (p = 0)
-                unsafeAtomicAdd(&acc[px0[u] - p0][lane], (A)(c0[u] * p[u]));
-                for (long q = qa[u] + 1; q < qb[u]; ++q)
-                    unsafeAtomicAdd(&acc[fpix[q] - p0][lane], (A)(fcnt[q] * p[u]));
+                for (int u = 0; u < kQueueRows; ++u) {
+                    if (!(p[u] > kProbMin)) continue;  // also the entries past the queue (p = 0)
+                    unsafeAtomicAdd(&acc[px0[u] - p0][lane], c0[u] * p[u]);
+                    for (long q = qa[u] + 1; q < qb[u]; ++q)
+                        unsafeAtomicAdd(&acc[fpix[q] - p0][lane], fcnt[q] * p[u]);
+                }
             }
+            __syncthreads();  // every wave has read the queue before it is refilled
         }
-        __syncthreads();  // every wave has read the queue before it is refilled
-    }
-    // psum of the tile's slots (FP32 views: its FP32 reciprocal, one division per slot)
-    __shared__ double s_ps[kRTile];
-    __shared__ float s_inv[kRTile];
-    if (tid < kRTile) {
-        const double ps = psum_slot[(size_t)T * kRTile + tid];
-        s_ps[tid] = ps;
-        s_inv[tid] = ps > 0. ? (float)(1. / ps) : 1.f;
     }
     __syncthreads();
     // divide by psum while transposing (lanes along pixels). With nzmask, item (slot, patch rg)
     // records which of its pixels have a nonzero view and only those are stored: the merge
     // reads no other.
-    for (int jj = wave; jj < kRTile; jj += kWavesPerBlock) {
-        const int t = p0 + lane;
+    const int px = lane % kPix, t = p0 + px;
+    for (int j0 = wave * kParts; j0 < kRTile; j0 += kWavesPerBlock * kParts) {
+        const int jj = j0 + lane / kPix;
         double v = 0.;
         if (t < num_pix) {
             if constexpr (sizeof(VT) == sizeof(float)) {
-                v = (double)(acc[lane][jj] * s_inv[jj]);
+                v = (double)(float)(acc[px][jj] * s_inv[jj]);
             } else {
                 const double ps = s_ps[jj];
-                v = ps > 0. ? (double)acc[lane][jj] / ps : (double)acc[lane][jj];
+                v = ps > 0. ? acc[px][jj] / ps : acc[px][jj];
             }
         }
         const size_t at = ((size_t)lt * kRTile + jj) * num_pix + t;
-        if (nzmask) {
+        if (nz) {
             const unsigned long long m = __ballot(v != 0.);
-            if (lane == 0) nzmask[((size_t)lt * kRTile + jj) * npatch + rg] = m;
+            if (px == 0) nz[(size_t)jj * npatch * kParts] = (Mask)(m >> (lane - px));
             if (v != 0.) view[at] = (VT)v;
         } else if (t < num_pix) {
             view[at] = (VT)v;
@@ -1020,11 +1065,21 @@ static void pair_tomogram_launch(hipStream_t s, const TP *P, const long *tile_of
                                  int ntiles, int num_pix, const PT *partial, VT *view,
                                  unsigned long long *nzmask, const SigFullRows &fr, const PairBuckets &bk) {
     if (ntiles <= 0) return;
-    const unsigned grid = (unsigned)((ntiles + kNumXcd - 1) / kNumXcd * kNumXcd) * (unsigned)nranges;
-    pair_tomogram_kernel<TP, VT, PT><<<grid, kBlock, 0, s>>>(P, tile_off, sig_pair, sig_frame, sig_cnt, foff, roff,
-                                                             nranges, fpix, fcnt, psum_slot, t0, ntiles, num_pix,
-                                                             partial, view, nzmask, fr.RF, fr.nF, fr.row,
-                                                             fr.frame, fr.cnt, bk);
+    // quarter patches where the lists are long enough to fill them (64 photons a block): with 190
+    // photons a quarter the stage takes 15.1 ms, 19.6 by whole patches; with 5, 2.0 against 1.8
+    const bool quarter = bk.base && bk.sub == 4 && bk.per_tile >= 64L * bk.nr;
+    const int nr = quarter ? bk.nr : nranges;
+    const unsigned grid = (unsigned)((ntiles + kNumXcd - 1) / kNumXcd * kNumXcd) * (unsigned)nr;
+#define EMC_PT(B, BITS, FULL)                                                                                        \
+    pair_tomogram_kernel<B, BITS, FULL, TP, VT, PT><<<grid, kBlock, 0, s>>>(                                         \
+        P, tile_off, sig_pair, sig_frame, sig_cnt, foff, roff, nr, fpix, fcnt, psum_slot, t0, ntiles, num_pix, partial, \
+        view, nzmask, fr.RF, fr.nF, fr.row, fr.frame, fr.cnt, bk)
+    if (quarter && fr.RF) EMC_PT(true, 4, true);
+    else if (quarter) EMC_PT(true, 4, false);
+    else if (bk.base && fr.RF) EMC_PT(true, 6, true);
+    else if (bk.base) EMC_PT(true, 6, false);
+    else EMC_PT(false, 6, true);
+#undef EMC_PT
 }
 
 void launch_pair_tomogram(hipStream_t s, const double *P, const long *tile_off, const int *sig_pair,
