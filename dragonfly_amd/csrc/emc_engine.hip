@@ -313,6 +313,7 @@ struct emc_engine {
     // upper bound on the orientation chunk width (0: memory decides)
     int max_chunk_cols = 0;
     DevBuf<double> tom_rows;      // the chunk's posterior as the tomogram reads it (128-byte rows)
+    DevBuf<unsigned long long> tom_marks;  // its rows that are not all zero
     DevBuf<double> tom_partial;   // subset path: the full frames' sums of a chunk
     DevBuf<float> tom_partial32;  // the same in FP32 (FP32 gathers)
     // log W of every slot (one orientation chunk), left by an expectation step of the subset
@@ -1219,6 +1220,11 @@ size_t brick_list_extra(const std::vector<emc_engine::BrickChunk> &chunks, size_
     return want > held ? want - held : 0;
 }
 
+// bytes of the tomogram's row marks per orientation column, rounded up
+size_t mark_bytes_per_column(size_t frames) {
+    return emc::tomo_mark_words(frames, emc::kRTile) * sizeof(unsigned long long) / emc::kRTile + 1;
+}
+
 int ensure_work(emc_engine *e) {
     int rc;
     const size_t N = e->num_data, Rp = e->Rp, P = e->num_pix;
@@ -1232,7 +1238,7 @@ int ensure_work(emc_engine *e) {
     size_t budget = freeb > reserve ? freeb - reserve : 0;
     const size_t cap = (size_t)120 << 30;
     budget += e->logw.cap * sizeof(double);
-    budget += e->tom_rows.cap * sizeof(double);
+    budget += e->tom_rows.cap * sizeof(double) + e->tom_marks.cap * sizeof(unsigned long long);
     budget += (e->lw_hi.cap + e->lw_lo.cap + e->p16.cap) * sizeof(_Float16);
     const bool mp = mp_mode(e);
     const bool g32 = e->precision == 3;
@@ -1257,6 +1263,7 @@ int ensure_work(emc_engine *e) {
                               : P * sizeof(double) +
                                     (g32 ? P * sizeof(float) + N * sizeof(float)
                                          : (e->tomo_tile_mode == 2 ? N * sizeof(double) : 0)) +
+                                    mark_bytes_per_column(N) +
                                     (split ? (size_t)e->lik_split * N * sizeof(double) : 0);
     size_t cmax = budget / per_col;
     if (e->max_chunk_cols > 0 && cmax > (size_t)e->max_chunk_cols) cmax = e->max_chunk_cols;
@@ -1267,6 +1274,7 @@ int ensure_work(emc_engine *e) {
         // exact sizes: the budget above counted these buffers as free
         e->bricks_valid = false;
         e->tom_rows.release();
+        e->tom_marks.release();
         e->logw.release();
         e->lik_part.release();
         e->logw32.release();
@@ -1276,6 +1284,9 @@ int ensure_work(emc_engine *e) {
     }
     e->tom_partial.release();  // the subset path's
     if (mp || g32 || e->tomo_tile_mode != 2) e->tom_rows.release();
+    const size_t n_marks = !mp && (g32 || e->tomo_tile_mode == 2) ? emc::tomo_mark_words(N, e->C) : 0;
+    if (n_marks == 0) e->tom_marks.release();
+    else if ((rc = e->tom_marks.alloc(n_marks))) return rc;
     if (mp) {
         const size_t rows_c = round_up((size_t)e->C, emc::kGemmBN);
         if (rows_c != e->mp_rows_c || !e->lw_hi.p || mp_two(e) != (e->lw_lo.p != nullptr)) {
@@ -1380,6 +1391,7 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
             e->logw_resident = false;
         }
         e->tom_rows.release();
+        e->tom_marks.release();
         e->tom_partial.release();
         e->tom_partial32.release();
         e->p32.release();
@@ -1415,7 +1427,7 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
     // full frames: else they keep their room for the next lists that have some)
     size_t budget = (freeb > reserve ? freeb - reserve : 0) + e->logw.cap * sizeof(double) +
                     e->logw32.cap * sizeof(float) +
-                    (nF > 0 ? (e->tom_rows.cap + e->tom_partial.cap) * sizeof(double) +
+                    (nF > 0 ? (e->tom_rows.cap + e->tom_partial.cap + e->tom_marks.cap) * sizeof(double) +
                                   (e->p32.cap + e->tom_partial32.cap) * sizeof(float)
                             : 0);
     budget = std::min(budget, (size_t)120 << 30);
@@ -1423,6 +1435,7 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
     // FP32 gathers all FP32), and the view's nonzero masks
     const size_t parts_col = nF > 0 ? 1 : 0;
     const size_t per_col = ((size_t)P * (1 + parts_col) + (size_t)nF) * (g32 ? sizeof(float) : sizeof(double)) +
+                           (nF > 0 ? mark_bytes_per_column(nF) : 0) +
                            (size_t)((P + 63) / 64) * sizeof(unsigned long long);
     size_t cmax = budget / per_col;
     if (e->max_chunk_cols > 0) cmax = std::min(cmax, (size_t)e->max_chunk_cols);
@@ -1443,6 +1456,9 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
     };
     auto fit = [](auto &buf, size_t n) -> int { return n > 0 ? buf.alloc(n) : 0; };
     const size_t C128 = round_up((size_t)C, 128);  // FP32 log W: 128-wide tiles
+    const size_t n_marks = nF > 0 ? emc::tomo_mark_words(nF, C) : 0;
+    shrink(e->tom_marks, n_marks);
+    if ((rc = fit(e->tom_marks, n_marks))) return rc;
     if (g32 ? e->logw.cap > 0 : e->logw.cap != (size_t)P * C) {
         // the FP64 log W / view buffer: none with FP32 gathers (log W and the view are FP32)
         e->logw.release();
@@ -1746,11 +1762,11 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
             const int t0 = bc.r0 / emc::kRTile, t1 = (bc.r0 + bc.Cc) / emc::kRTile;
             if (parts && (rc = timed(6, [&] {
                                if (g32) {
-                                   emc::launch_posterior_rows(s, e->RF.p, nF, bc.r0, bc.Cc, S, e->p32.p);
-                                   emc::launch_tomogram_rows(s, e->p32.p, nF, bc.Cc, flists, P, e->tom_partial32.p);
+                                   emc::launch_posterior_rows(s, e->RF.p, nF, bc.r0, bc.Cc, S, e->p32.p, e->tom_marks.p);
+                                   emc::launch_tomogram_rows(s, e->p32.p, e->tom_marks.p, nF, bc.Cc, flists, P, e->tom_partial32.p);
                                } else {
-                                   emc::launch_posterior_rows(s, e->RF.p, nF, bc.r0, bc.Cc, S, e->tom_rows.p);
-                                   emc::launch_tomogram_rows(s, e->tom_rows.p, nF, bc.Cc, flists, P, nullptr, 0,
+                                   emc::launch_posterior_rows(s, e->RF.p, nF, bc.r0, bc.Cc, S, e->tom_rows.p, e->tom_marks.p);
+                                   emc::launch_tomogram_rows(s, e->tom_rows.p, e->tom_marks.p, nF, bc.Cc, flists, P, nullptr, 0,
                                                              e->tom_partial.p, false);
                                }
                                return 0;
@@ -2033,6 +2049,7 @@ void emc_destroy(emc_engine *e) {
     e->tp_frame.release();
     e->tp_cnt.release();
     e->tom_rows.release();
+    e->tom_marks.release();
     e->tom_partial.release();
     e->ft_off.release();
     e->fe_off.release();
@@ -2990,11 +3007,11 @@ int emc_maximize(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *stats
                                     1. / pscale))
                 return fail(EMC_E_STATE, "tomogram product: shape does not fit the tiles");
         } else if (g32) {
-            emc::launch_posterior_rows(s, e->R.p, N, r0, Cc, Rn, e->p32.p);
-            emc::launch_tomogram_rows(s, e->p32.p, N, Cc, lists, P, e->psum_r.p + r0, Rn - r0, e->logw.p, bricks);
+            emc::launch_posterior_rows(s, e->R.p, N, r0, Cc, Rn, e->p32.p, e->tom_marks.p);
+            emc::launch_tomogram_rows(s, e->p32.p, e->tom_marks.p, N, Cc, lists, P, e->psum_r.p + r0, Rn - r0, e->logw.p, bricks);
         } else if (parts) {
-            emc::launch_posterior_rows(s, e->R.p, N, r0, Cc, Rn, e->tom_rows.p);
-            emc::launch_tomogram_rows(s, e->tom_rows.p, N, Cc, lists, P, e->psum_r.p + r0, Rn - r0, e->logw.p, bricks);
+            emc::launch_posterior_rows(s, e->R.p, N, r0, Cc, Rn, e->tom_rows.p, e->tom_marks.p);
+            emc::launch_tomogram_rows(s, e->tom_rows.p, e->tom_marks.p, N, Cc, lists, P, e->psum_r.p + r0, Rn - r0, e->logw.p, bricks);
         }
         else if (e->tomo_tile_mode == 1)
             emc::launch_tomogram_tiles(s, e->R.p, N, r0, Cc, e->ft_off.p, e->ft_frame.p,

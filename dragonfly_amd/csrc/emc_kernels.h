@@ -130,9 +130,16 @@ void launch_tomogram_tiles(hipStream_t s, const double *P, int num_data, int r0,
                            double *view);
 // ---- tomogram (emc_tomogram.hip) ----
 // rows of the chunk's posterior in tiles of kTomoRowBytes rows (C a multiple of 64 columns from
-// orientation r0; P <= 1e-6 and columns past num_rot are 0): num_data * C elements
-void launch_posterior_rows(hipStream_t s, const double *P, int num_data, int r0, int C, int num_rot, double *rows);
-void launch_posterior_rows(hipStream_t s, const double *P, int num_data, int r0, int C, int num_rot, float *rows);
+// orientation r0; P <= 1e-6 and columns past num_rot are 0): num_data * C elements; marks: the rows
+// that are not all 0, a bit a frame, and their number, tile after tile: tomo_mark_words(num_data, C)
+// words at most
+inline size_t tomo_mark_words(size_t num_data, size_t C) {
+    return ((num_data + 63) / 64 + 1) * (C / (kTomoRowBytes / 8));
+}
+void launch_posterior_rows(hipStream_t s, const double *P, int num_data, int r0, int C, int num_rot, double *rows,
+                           unsigned long long *marks);
+void launch_posterior_rows(hipStream_t s, const double *P, int num_data, int r0, int C, int num_rot, float *rows,
+                           unsigned long long *marks);
 // photon lists of nparts frame ranges (range x, pixel t: entries off[x * num_pix + t] up to the
 // next offset; frame, count), and the pixel units (first, number) the blocks take
 struct TomoLists {
@@ -146,12 +153,15 @@ struct TomoLists {
 std::vector<int2> tomo_units(const long *off, int nparts, int num_pix);
 // the chunk's view from those rows and lists, divided by psum (of the chunk's columns; num_psum of
 // them are orientations; null: sums only); orientation-major or tile-major
-void launch_tomogram_rows(hipStream_t s, const double *rows, int num_data, int C, const TomoLists &l, int num_pix,
+void launch_tomogram_rows(hipStream_t s, const double *rows, const unsigned long long *marks, int num_data, int C,
+                          const TomoLists &l, int num_pix,
                           const double *psum, int num_psum, double *view, bool rmajor);
-void launch_tomogram_rows(hipStream_t s, const float *rows, int num_data, int C, const TomoLists &l, int num_pix,
+void launch_tomogram_rows(hipStream_t s, const float *rows, const unsigned long long *marks, int num_data, int C,
+                          const TomoLists &l, int num_pix,
                           const double *psum, int num_psum, double *view, bool rmajor);
 // tile-major FP32 sums (each the FP64 sum rounded once per frame range)
-void launch_tomogram_rows(hipStream_t s, const float *rows, int num_data, int C, const TomoLists &l, int num_pix,
+void launch_tomogram_rows(hipStream_t s, const float *rows, const unsigned long long *marks, int num_data, int C,
+                          const TomoLists &l, int num_pix,
                           float *sums);
 // ---- brick merge (emc_merge.hip) ----
 // per-brick item lists: pass 0 counts, pass 1 writes the item ids and, beside each, the mask of

@@ -106,6 +106,22 @@ def test_tomogram_rows(frames, num_rot):
     eng.close()
 
 
+@pytest.mark.parametrize('frames, num_rot, mean_count', ((1, 20, 3000.), (3, 420, 3000.), (64, 129, 400.),
+                                                         (65, 420, 400.), (700, 420, 150.), (17000, 33, 400.)))
+def test_tomogram_marked_rows(frames, num_rot, mean_count):
+    """The same with bright frames, whose posterior lies in a few orientations: tiles without any
+    marked row, with few (taken by their marks) and with most of them, two frame ranges."""
+    p = P.build(P.tiny_config(num_data=frames, mean_count=mean_count), quats=_lib.quat_gen(2)[:num_rot], num_ave=200)
+    o = P.run_oracle(p, dict(iteration=1), dense_prob=False)
+    eng = P.engine_for(p)
+    for precision, merge_mode, bar in ((0, 1, 1e-9), (0, 0, 1e-9), (3, 1, 1e-4)):
+        eng.set_precision(precision)
+        eng.set_option('merge_mode', merge_mode)
+        eng.maximize(1, 0, 1, 0)
+        assert P.rel_err(eng.get('model2'), o['model2']) <= bar, (precision, merge_mode)
+    eng.close()
+
+
 @pytest.mark.parametrize('precision', (0, 3))
 @pytest.mark.parametrize('part_frames', (12500, 7))
 def test_full_frames_tomogram_ranges(precision, part_frames):
@@ -129,3 +145,82 @@ def test_full_frames_tomogram_ranges(precision, part_frames):
         out.append(P.run_engine(eng, dict(iteration=1)))
         eng.close()
     assert P.rel_err(out[0]['model2'], out[1]['model2']) <= (1e-9 if precision == 0 else 1e-4)
+
+
+@pytest.mark.parametrize('precision', (0, 3))
+@pytest.mark.parametrize('repeat, buckets', ((1, 1), (8, 1), (8, 0)))
+@pytest.mark.parametrize('full', (False, True))
+def test_pair_tomogram_photon_lists(precision, repeat, buckets, full):
+    """The pair tomogram from its tiles' photon lists, by whole patches (24 frames) and by quarter
+    patches (192 frames of the same counts; 440 pixels end inside a patch), with and without rows
+    of full frames in the lists, and from the walk over the tiles' rows, against the masked full
+    search."""
+    counts = COUNTS * repeat
+    p = counted_problem(counts, 420)
+    qc = _lib.quat_gen(1)
+    cells = _lib.voronoi_subset(qc, p['quats'])
+    rng = np.random.default_rng(6)
+    sets = [np.array([-1], 'i4') if full and d % 2 else np.sort(rng.permutation(len(qc))[:9]).astype('i4')
+            for d in range(len(counts))]
+    off = np.concatenate([[0], np.cumsum([len(s) for s in sets])]).astype('i8')
+    out = []
+    for subset in (1, 0):
+        eng = P.engine_for(p)
+        eng.set_precision(precision)
+        eng.set_option('subset', subset)
+        eng.set_option('tomo_buckets', buckets)
+        eng.set_refine(len(qc), cells, off, np.concatenate(sets))
+        out.append(P.run_engine(eng, dict(iteration=1)))
+        eng.close()
+    assert P.rel_err(out[0]['model2'], out[1]['model2']) <= (1e-9 if precision == 0 else 1e-4)
+    assert P.rel_err(out[0]['inter_weight'], out[1]['inter_weight']) <= 1e-9
+
+
+@pytest.mark.parametrize('size', (81, 128, 163))
+def test_volume_readback(size):
+    """Volumes of one piece and a remainder, whole pieces, and more pieces than copying threads
+    come back byte for byte."""
+    p = counted_problem((5,), 3)
+    eng = P.engine_for(p)
+    vol = np.random.default_rng(size).random((size,) * 3)
+    eng.set_model(vol)
+    for _ in range(2):
+        assert np.array_equal(eng.get('model1').view('u8'), vol.view('u8'))
+    assert not eng.get('model2').any()
+    eng.close()
+
+
+@pytest.mark.parametrize('frames', (1, 15, 17, 33, 700))
+def test_psum_parts(frames):
+    """psum_r (the divisor of the views) over one and several frame parts, the last one short, with
+    blacklisted and scaled frames and 257 orientations (one past a block's)."""
+    p = P.build(P.tiny_config(num_data=frames, mean_count=25.), quats=_lib.quat_gen(2)[:257], num_ave=200)
+    fp = p['fparams']
+    fp['beta'] = np.full(frames, 0.1)
+    fp['scale'] = np.linspace(0.7, 1.4, frames)
+    fp['blacklist'] = (np.arange(frames) % 3 == 1).astype('u1')
+    fp['num_blacklist'] = int(fp['blacklist'].sum())
+    flags = dict(iteration=2, need_scaling=1)
+    o = P.run_oracle(p, flags)
+    eng = P.engine_for(p)
+    g = P.run_engine(eng, flags)
+    eng.close()
+    for k in ('likelihood', 'prob', 'model2', 'inter_weight'):
+        assert P.rel_err(g[k], o[k]) <= 1e-9, k
+
+
+@pytest.mark.parametrize('frames, beta', ((3, 1.), (40, 0.05)))
+def test_merge_some_and_all_orientations(frames, beta):
+    """Bright frames leave all but one orientation without any posterior, and so out of the merge;
+    faint ones leave none out."""
+    p = P.build(P.tiny_config(num_data=frames, mean_count=6000. if beta == 1. else 20.), num_ave=200)
+    p['fparams']['beta'] = np.full(frames, beta)
+    o = P.run_oracle(p, dict(iteration=1))
+    assert (o['prob'].max(0) == 0.).any() == (beta == 1.)
+    eng = P.engine_for(p)
+    for merge_mode in (1, 0):
+        eng.set_option('merge_mode', merge_mode)
+        eng.maximize(1, 0, 1, 0)
+        assert P.rel_err(eng.get('model2'), o['model2']) <= 1e-9, merge_mode
+        assert P.rel_err(eng.get('inter_weight'), o['inter_weight']) <= 1e-9, merge_mode
+    eng.close()

@@ -154,3 +154,30 @@ def test_trained_proposal_captures_posterior_mass():
           % (hist[0], hist[-1], k, mass_net, mass_fixed), flush=True)
     assert hist[-1] < hist[0]
     assert mass_net > 3 * mass_fixed
+
+
+@pytest.mark.parametrize('M, N, K', ((256, 256, 128), (256, 512, 384), (256, 256, 192), (512, 256, 160),
+                                     (4096, 4096, 64), (4096, 4096, 256)))
+def test_products_of_every_tile(M, N, K):
+    """The small tile (K a multiple of 128, fewer large tiles than CUs), the large one in steps of
+    64 and of 32: one step, odd numbers of steps, ragged valid rows and columns. BF16 products are
+    exact in FP32, so a sum of K terms is within K 2^-23 of the sum of their magnitudes."""
+    import torch
+    from dragonfly_amd import _lib
+    g = torch.Generator(device='cpu').manual_seed(M + N + K)
+    A = (torch.rand((M, K), generator=g) - 0.5).to(torch.bfloat16).cuda()
+    B = (torch.rand((N, K), generator=g) - 0.5).to(torch.bfloat16).cuda()
+    bias = torch.rand(N, generator=g).cuda()
+    m, n = M - 3, N - 65
+    out = torch.full((M, N), 7., device='cuda')
+    dW = torch.full((M, N), 7., device='cuda')
+    L, s = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    assert L.emc_nn_forward(s, A.data_ptr(), K, B.data_ptr(), K, M, N, K, m, n, bias.data_ptr(), 0, 1,
+                            out.data_ptr(), N) == 0
+    assert L.emc_nn_backward_weight(s, A.data_ptr(), K, B.data_ptr(), K, M, N, K, m, n, dW.data_ptr(), N) == 0
+    ref = A.double() @ B.double().T
+    mag = A.double().abs() @ B.double().abs().T
+    for got, want in ((out, ref + bias.double()), (dW, ref)):
+        err = (got.double() - want).abs()[:m, :n]
+        assert bool((err <= K * 2. ** -23 * (mag[:m, :n] + 1.)).all())
+        assert bool((got[m:] == 7.).all()) and bool((got[:, n:] == 7.).all())
