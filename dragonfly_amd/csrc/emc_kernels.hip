@@ -87,17 +87,22 @@ __global__ void u_reduce_kernel(const double *__restrict__ upart, const int *__r
     rbad[r0 + c] = bad;
 }
 
-// rescale = mean_count / sum_r w_r u_r (max_prob.c:40, :59); one block, fixed order.
-__global__ __launch_bounds__(kBlock) void rescale_kernel(const double *__restrict__ quats,
-                                                         const double *__restrict__ u, int num_rot,
-                                                         double mean_count, double modes,
-                                                         double *__restrict__ scalars) {
-    __shared__ double s[kBlock];
+// One-block sums in a fixed order: 16 waves and eight loads in flight a thread, since nothing else
+// runs beside them (4 waves with one load each: 30 us for the 10,880 orientations of rescale, now 14).
+constexpr int kSumThreads = 1024;
+
+// rescale = mean_count / sum_r w_r u_r (max_prob.c:40, :59)
+__global__ __launch_bounds__(kSumThreads) void rescale_kernel(const double *__restrict__ quats,
+                                                              const double *__restrict__ u, int num_rot,
+                                                              double mean_count, double modes,
+                                                              double *__restrict__ scalars) {
+    __shared__ double s[kSumThreads];
     double acc = 0.;
-    for (int r = threadIdx.x; r < num_rot; r += kBlock) acc += quats[5 * (size_t)r + 4] * u[r];
+#pragma unroll 8
+    for (int r = threadIdx.x; r < num_rot; r += kSumThreads) acc += quats[5 * (size_t)r + 4] * u[r];
     s[threadIdx.x] = acc;
     __syncthreads();
-    for (int w = kBlock / 2; w > 0; w >>= 1) {
+    for (int w = kSumThreads / 2; w > 0; w >>= 1) {
         if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
         __syncthreads();
     }
@@ -498,6 +503,7 @@ __global__ void psum_r_reduce_kernel(const double *__restrict__ part, int nparts
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= num_rot) return;
     double acc = 0.;
+#pragma unroll 16
     for (int i = 0; i < nparts; ++i) acc += part[(size_t)i * num_rot + r];
     psum_r[r] = acc;
 }
@@ -743,14 +749,15 @@ __global__ __launch_bounds__(kBlock) void merge_box_kernel(
 }
 
 // count of orientations with psum_r <= 0 (they are not merged, max_update.c:34-36); one block
-__global__ __launch_bounds__(kBlock) void count_unmerged_kernel(const double *__restrict__ psum_r,
-                                                                int num_rot, int *__restrict__ count) {
-    __shared__ int s[kBlock];
+__global__ __launch_bounds__(kSumThreads) void count_unmerged_kernel(const double *__restrict__ psum_r,
+                                                                     int num_rot, int *__restrict__ count) {
+    __shared__ int s[kSumThreads];
     int local = 0;
-    for (int r = threadIdx.x; r < num_rot; r += kBlock) local += !(psum_r[r] > 0.);
+#pragma unroll 8
+    for (int r = threadIdx.x; r < num_rot; r += kSumThreads) local += !(psum_r[r] > 0.);
     s[threadIdx.x] = local;
     __syncthreads();
-    for (int w = kBlock / 2; w > 0; w >>= 1) {
+    for (int w = kSumThreads / 2; w > 0; w >>= 1) {
         if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
         __syncthreads();
     }
@@ -786,21 +793,31 @@ __global__ void slice_merge_kernel(const double *__restrict__ rot, const double 
 
 // ---- per-frame statistics and scale ------------------------------------------------------
 // sums of likelihood and info over non-blacklisted frames (max_prob.c:367-374).
-__global__ __launch_bounds__(kBlock) void frame_stats_kernel(
+__global__ __launch_bounds__(kSumThreads) void frame_stats_kernel(
     const double *__restrict__ likelihood, const double *__restrict__ info,
     const uint8_t *__restrict__ blacklist, int num_data, int denom, double *__restrict__ scalars) {
-    __shared__ double s[kBlock];
+    __shared__ double s[2][kSumThreads];
     double a = 0., b = 0.;
-    for (int d = threadIdx.x; d < num_data; d += kBlock)
-        if (!blacklist[d]) {
-            a += likelihood[d];
-            b += info[d];
+#pragma unroll 8
+    for (int d = threadIdx.x; d < num_data; d += kSumThreads) {
+        const bool in = !blacklist[d];
+        const double lk = likelihood[d], inf = info[d];
+        a += in ? lk : 0.;
+        b += in ? inf : 0.;
+    }
+    s[0][threadIdx.x] = a;
+    s[1][threadIdx.x] = b;
+    __syncthreads();
+    for (int w = kSumThreads / 2; w > 0; w >>= 1) {
+        if (threadIdx.x < w) {
+            s[0][threadIdx.x] += s[0][threadIdx.x + w];
+            s[1][threadIdx.x] += s[1][threadIdx.x + w];
         }
-    const double ta = block_sum(a, s);
-    const double tb = block_sum(b, s);
+        __syncthreads();
+    }
     if (threadIdx.x == 0) {
-        scalars[1] = ta / denom;
-        scalars[2] = tb / denom;
+        scalars[1] = s[0][0] / denom;
+        scalars[2] = s[1][0] / denom;
     }
 }
 
@@ -1019,7 +1036,7 @@ void launch_u_reduce(hipStream_t s, const double *upart, const int *ubad, int ng
 
 void launch_rescale(hipStream_t s, const double *quats, const double *u, int num_rot,
                     double mean_count, double *scalars, int modes) {
-    rescale_kernel<<<1, kBlock, 0, s>>>(quats, u, num_rot, mean_count, (double)modes, scalars);
+    rescale_kernel<<<1, kSumThreads, 0, s>>>(quats, u, num_rot, mean_count, (double)modes, scalars);
 }
 
 // 1-D XCD-aware grid of a likelihood launch over gy column tiles (xcd: XCDs sharing a tile, 1,
@@ -1437,7 +1454,7 @@ void launch_merge(hipStream_t s, const double *rots, int r0, int C, int num_rot,
 }
 
 void launch_count_unmerged(hipStream_t s, const double *psum_r, int num_rot, int *count) {
-    count_unmerged_kernel<<<1, kBlock, 0, s>>>(psum_r, num_rot, count);
+    count_unmerged_kernel<<<1, kSumThreads, 0, s>>>(psum_r, num_rot, count);
 }
 
 void launch_slice_gen(hipStream_t s, const double *rot, const double *model, long size,
@@ -1455,7 +1472,7 @@ void launch_slice_merge(hipStream_t s, const double *rot, const double *view, co
 
 void launch_frame_stats(hipStream_t s, const double *likelihood, const double *info,
                         const uint8_t *blacklist, int num_data, int denom, double *scalars) {
-    frame_stats_kernel<<<1, kBlock, 0, s>>>(likelihood, info, blacklist, num_data, denom, scalars);
+    frame_stats_kernel<<<1, kSumThreads, 0, s>>>(likelihood, info, blacklist, num_data, denom, scalars);
 }
 
 void launch_scale(hipStream_t s, const int *fcounts, const double *psum_d, const uint8_t *blacklist,
