@@ -210,7 +210,18 @@ std::vector<int> morton_order(int num_pix, const double *qvals) {
     return perm;
 }
 
-constexpr int kPixPerGroup = 1024;
+constexpr int kFusedPixPerGroup = 1024;  // of the persistent expand + likelihood
+// Pixels of one expand block: 64, a block's least (one compact patch): the blocks that an XCD holds at
+// once then read neighbouring patches of the same orientations, one region of the model, instead
+// of walking distant 1024-pixel groups side by side, and small detectors fill the chip. More, up to
+// 1024, only where the grid would pass 4 million blocks or 65,535 groups. 64, 128, 256 and 1024 pixels: 5.99, 6.45, 7.15
+// and 8.14 ms (10,880 orientations on 251^3), 2.68, 3.11, 3.32 and 3.69 with FP32 gathers, 0.43, 0.44, 0.47 and
+// 0.58 (3240 on 125^3), 12.7, 12.4, 13.5 and 14.5 (refinement subsets).
+int pix_per_group(long num_pix, long C) {
+    int n = 64;
+    while (n < 1024 && ((num_pix + n - 1) / n > 65535 || (num_pix + n - 1) / n * (C / emc::kRTile) > 1L << 22)) n *= 2;
+    return n;
+}
 // Frames of one block of the psum_r partial sums (256 orientations): few enough for about eight
 // blocks a CU, at most 512 (each part is another row of num_rot partial sums). 3000 frames x 3240
 // orientations made 78 blocks at 512 and took 0.28 ms, now 0.06.
@@ -1220,6 +1231,9 @@ size_t brick_list_extra(const std::vector<emc_engine::BrickChunk> &chunks, size_
     return want > held ? want - held : 0;
 }
 
+// bytes of the expand's partial u_r and flags per orientation column
+size_t u_bytes_per_column(size_t num_pix) { return (num_pix + 63) / 64 * (sizeof(double) + sizeof(int)); }
+
 // bytes of the tomogram's row marks per orientation column, rounded up
 size_t mark_bytes_per_column(size_t frames) {
     return emc::tomo_mark_words(frames, emc::kRTile) * sizeof(unsigned long long) / emc::kRTile + 1;
@@ -1239,6 +1253,7 @@ int ensure_work(emc_engine *e) {
     const size_t cap = (size_t)120 << 30;
     budget += e->logw.cap * sizeof(double);
     budget += e->tom_rows.cap * sizeof(double) + e->tom_marks.cap * sizeof(unsigned long long);
+    budget += e->upart.cap * sizeof(double) + e->ubad.cap * sizeof(int);
     budget += (e->lw_hi.cap + e->lw_lo.cap + e->p16.cap) * sizeof(_Float16);
     const bool mp = mp_mode(e);
     const bool g32 = e->precision == 3;
@@ -1265,7 +1280,7 @@ int ensure_work(emc_engine *e) {
                                          : (e->tomo_tile_mode == 2 ? N * sizeof(double) : 0)) +
                                     mark_bytes_per_column(N) +
                                     (split ? (size_t)e->lik_split * N * sizeof(double) : 0);
-    size_t cmax = budget / per_col;
+    size_t cmax = budget / (per_col + u_bytes_per_column(P));
     if (e->max_chunk_cols > 0 && cmax > (size_t)e->max_chunk_cols) cmax = e->max_chunk_cols;
     cmax = cmax / emc::kRTile * emc::kRTile;
     if (cmax < (size_t)emc::kRTile) return fail(EMC_E_NOMEM, "no device memory for an orientation chunk");
@@ -1338,7 +1353,7 @@ int ensure_work(emc_engine *e) {
         e->logw32.release();
         e->p32.release();
     }
-    const size_t ngroups = (P + kPixPerGroup - 1) / kPixPerGroup;
+    const size_t per_group = pix_per_group(P, e->C), ngroups = (P + per_group - 1) / per_group;
     if ((rc = e->upart.alloc(ngroups * (size_t)e->C))) return rc;
     if ((rc = e->ubad.alloc(ngroups * (size_t)e->C))) return rc;
     if ((rc = e->rbad.alloc(Rp))) return rc;
@@ -1429,14 +1444,15 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
                     e->logw32.cap * sizeof(float) +
                     (nF > 0 ? (e->tom_rows.cap + e->tom_partial.cap + e->tom_marks.cap) * sizeof(double) +
                                   (e->p32.cap + e->tom_partial32.cap) * sizeof(float)
-                            : 0);
+                            : 0) +
+                    e->upart.cap * sizeof(double) + e->ubad.cap * sizeof(int);
     budget = std::min(budget, (size_t)120 << 30);
     // per slot column: log W / view, the full frames' sums and their posterior column (FP64; with
     // FP32 gathers all FP32), and the view's nonzero masks
     const size_t parts_col = nF > 0 ? 1 : 0;
     const size_t per_col = ((size_t)P * (1 + parts_col) + (size_t)nF) * (g32 ? sizeof(float) : sizeof(double)) +
                            (nF > 0 ? mark_bytes_per_column(nF) : 0) +
-                           (size_t)((P + 63) / 64) * sizeof(unsigned long long);
+                           (size_t)((P + 63) / 64) * sizeof(unsigned long long) + u_bytes_per_column(P);
     size_t cmax = budget / per_col;
     if (e->max_chunk_cols > 0) cmax = std::min(cmax, (size_t)e->max_chunk_cols);
     cmax = cmax / emc::kRTile * emc::kRTile;
@@ -1485,7 +1501,7 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
         shrink(e->tom_rows, n_rows);
         if ((rc = fit(e->tom_partial, n_part)) || (rc = fit(e->tom_rows, n_rows))) return rc;
     }
-    const int ngroups = (P + kPixPerGroup - 1) / kPixPerGroup;
+    const int per_group = pix_per_group(P, C), ngroups = (P + per_group - 1) / per_group;
     if ((rc = e->upart.alloc((size_t)ngroups * C))) return rc;
     if ((rc = e->ubad.alloc((size_t)ngroups * C))) return rc;
     if ((rc = e->nzmask.alloc((size_t)C * ((P + 63) / 64)))) return rc;
@@ -1547,17 +1563,17 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
                              if (g32)
                                  emc::launch_fused_expand_likelihood(
                                      s, e->rots_slot.p, e->model32.p, e->size, e->qvals.p, e->corr.p, e->mask.p, P, s0,
-                                     Cc, kPixPerGroup, e->logw32.p, e->upart.p, e->ubad.p, e->slot_rot.p, e->lik_off.p,
+                                     Cc, kFusedPixPerGroup, e->logw32.p, e->upart.p, e->ubad.p, e->slot_rot.p, e->lik_off.p,
                                      e->lik_pix.p, e->lik_cnt.p, e->pair_frame.p, e->pair_tile.p, e->tile_off.p,
                                      e->tile_pair.p, t0, e->fused_counter.p, e->Rsub.p);
                              else
                                  emc::launch_fused_expand_likelihood(
                                      s, e->rots_slot.p, e->model1.p, e->size, e->qvals.p, e->corr.p, e->mask.p, P, s0,
-                                     Cc, kPixPerGroup, e->logw.p, e->upart.p, e->ubad.p, e->slot_rot.p, e->lik_off.p,
+                                     Cc, kFusedPixPerGroup, e->logw.p, e->upart.p, e->ubad.p, e->slot_rot.p, e->lik_off.p,
                                      e->lik_pix.p, e->lik_cnt.p, e->pair_frame.p, e->pair_tile.p, e->tile_off.p,
                                      e->tile_pair.p, t0, e->fused_counter.p, e->Rsub.p);
-                             emc::launch_u_reduce(s, e->upart.p, e->ubad.p, ngroups, Cc, s0, S, e->u_slot.p,
-                                                  e->rbad_slot.p);
+                             emc::launch_u_reduce(s, e->upart.p, e->ubad.p, (P + kFusedPixPerGroup - 1) / kFusedPixPerGroup,
+                                                  Cc, s0, S, e->u_slot.p, e->rbad_slot.p);
                              if (nF > 0) {
                                  if (g32)
                                      emc::launch_likelihood_mapped(s, e->logw32.p, Cc, P, e->lik_off.p, e->lik_pix.p,
@@ -1576,11 +1592,11 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
                 if (!resident && (rc = timed(0, [&] {
                                       if (g32)
                                           emc::launch_expand(s, e->rots_slot.p, e->model32.p, e->size, e->qvals.p,
-                                                             e->corr.p, e->mask.p, P, s0, Cc, kPixPerGroup,
+                                                             e->corr.p, e->mask.p, P, s0, Cc, per_group,
                                                              e->logw32.p, e->upart.p, e->ubad.p, e->slot_rot.p);
                                       else
                                           emc::launch_expand(s, e->rots_slot.p, e->model1.p, e->size, e->qvals.p,
-                                                             e->corr.p, e->mask.p, P, s0, Cc, kPixPerGroup,
+                                                             e->corr.p, e->mask.p, P, s0, Cc, per_group,
                                                              e->logw.p, e->upart.p, e->ubad.p, e->slot_rot.p);
                                       emc::launch_u_reduce(s, e->upart.p, e->ubad.p, ngroups, Cc, s0, S, e->u_slot.p,
                                                            e->rbad_slot.p);
@@ -2654,7 +2670,7 @@ static int update_scale_bg(emc_engine *e, const emc_iter_opts *opts) {
             // the views of the current model (the tomogram wrote its own into this buffer)
             if (!(one_chunk && views_ready))
                 emc::launch_expand(s, e->rots.p, e->model1.p, e->size, e->qvals.p, e->corr.p, e->mask.p, P, r0, Cc,
-                                   kPixPerGroup, e->logw.p, e->upart.p, e->ubad.p, nullptr, 1, 1);
+                                   pix_per_group(P, C), e->logw.p, e->upart.p, e->ubad.p, nullptr, 1, 1);
             emc::launch_gradient_d(s, e->logw.p, P, e->R.p, N, r0, Cc, Rn, e->lik_off.p, e->lik_pix.p, e->lik_cnt.p,
                                    e->bg_dmask.p, e->bg_s.p, e->bgscale.p, e->bg.p, rescale, e->bg_gpart.p,
                                    e->bg_gacc.p);
@@ -2798,7 +2814,7 @@ int emc_maximize(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *stats
     hipStream_t s = e->stream;
     const int N = e->num_data, Rn = e->num_rot, P = e->num_pix, C = e->C, M = e->num_modes;
     const size_t vol = (size_t)e->size * e->size * e->size * M;  // every mode's volume
-    const int ngroups = (P + kPixPerGroup - 1) / kPixPerGroup;
+    const int per_group = pix_per_group(P, C), ngroups = (P + per_group - 1) / per_group;
     const int use_scale = opts->need_scaling && (opts->iteration > 1 || opts->known_scale);
     const int want_psum_d = opts->need_scaling && opts->update_scale;
     float ms_expand = 0.f, ms_lik = 0.f, ms_tomo = 0.f, ms_reduce = 0.f, ms_merge = 0.f;
@@ -2829,14 +2845,14 @@ int emc_maximize(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *stats
         HIP_TRY(hipEventRecord(e->ev[0], s));
         if (mp)
             emc::launch_expand_mp(s, e->rots.p, e->model1.p, e->size, e->qvals.p, e->corr.p, e->mask.p,
-                                  e->center_t.p, P, r0, Cc, kPixPerGroup, e->mp_ldp, mp_two(e),
+                                  e->center_t.p, P, r0, Cc, per_group, e->mp_ldp, mp_two(e),
                                   e->lw_hi.p, e->lw_lo.p, e->upart.p, e->ubad.p, mp_bf16(e));
         else if (g32)
             emc::launch_expand(s, e->rots.p, e->model32.p, e->size, e->qvals.p, e->corr.p, e->mask.p,
-                               P, r0, Cc, kPixPerGroup, e->logw32.p, e->upart.p, e->ubad.p, nullptr, M);
+                               P, r0, Cc, per_group, e->logw32.p, e->upart.p, e->ubad.p, nullptr, M);
         else
             emc::launch_expand(s, e->rots.p, e->model1.p, e->size, e->qvals.p, e->corr.p, e->mask.p,
-                               P, r0, Cc, kPixPerGroup, e->logw.p, e->upart.p, e->ubad.p, nullptr, M, bgp);
+                               P, r0, Cc, per_group, e->logw.p, e->upart.p, e->ubad.p, nullptr, M, bgp);
         emc::launch_u_reduce(s, e->upart.p, e->ubad.p, ngroups, Cc, r0, Rn, e->u.p, e->rbad.p);
         HIP_TRY(hipEventRecord(e->ev[1], s));
         if (mp) {

@@ -71,25 +71,36 @@ static unsigned expand_grid(int C, int num_pix, int pix_per_group) {
     return (unsigned)(kNumXcd * per * ((num_pix + pix_per_group - 1) / pix_per_group));
 }
 
-// u[r0 + c] = sum over pixel groups, fixed order.
-__global__ void u_reduce_kernel(const double *__restrict__ upart, const int *__restrict__ ubad,
-                                int ngroups, int C, int r0, int num_rot, double *__restrict__ u,
-                                int *__restrict__ rbad) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= C || r0 + c >= num_rot) return;
+// u[r0 + c] = sum over pixel groups, fixed order; block = 64 columns, its waves every kSumWaves-th
+// group each.
+// 16 waves, because nothing else runs beside this or the one-block sums below (4 waves with one load
+// in flight each: 30 us for the 10,880 orientations of rescale, now 14).
+constexpr int kSumThreads = 1024, kSumWaves = kSumThreads / 64;
+__global__ __launch_bounds__(kSumThreads) void u_reduce_kernel(const double *__restrict__ upart,
+                                                               const int *__restrict__ ubad, int ngroups, int C,
+                                                               int r0, int num_rot, double *__restrict__ u,
+                                                               int *__restrict__ rbad) {
+    __shared__ double s_u[kSumWaves][64];
+    __shared__ int s_bad[kSumWaves][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = blockIdx.x * 64 + lane;
     double acc = 0.;
     int bad = 0;
-    for (int g = 0; g < ngroups; ++g) {
+#pragma unroll 8
+    for (int g = wave; g < ngroups; g += kSumWaves) {
         acc += upart[(size_t)g * C + c];
         bad |= ubad[(size_t)g * C + c];
+    }
+    s_u[wave][lane] = acc;
+    s_bad[wave][lane] = bad;
+    __syncthreads();
+    if (wave > 0 || r0 + c >= num_rot) return;
+    for (int w = 1; w < kSumWaves; ++w) {
+        acc += s_u[w][lane];
+        bad |= s_bad[w][lane];
     }
     u[r0 + c] = acc;
     rbad[r0 + c] = bad;
 }
-
-// One-block sums in a fixed order: 16 waves and eight loads in flight a thread, since nothing else
-// runs beside them (4 waves with one load each: 30 us for the 10,880 orientations of rescale, now 14).
-constexpr int kSumThreads = 1024;
 
 // rescale = mean_count / sum_r w_r u_r (max_prob.c:40, :59)
 __global__ __launch_bounds__(kSumThreads) void rescale_kernel(const double *__restrict__ quats,
@@ -1031,7 +1042,7 @@ void launch_copy_f32_brick(hipStream_t s, const double *in, long size, int modes
 
 void launch_u_reduce(hipStream_t s, const double *upart, const int *ubad, int ngroups, int C,
                      int r0, int num_rot, double *u, int *rbad) {
-    u_reduce_kernel<<<cdiv(C, 256), 256, 0, s>>>(upart, ubad, ngroups, C, r0, num_rot, u, rbad);
+    u_reduce_kernel<<<C / 64, kSumThreads, 0, s>>>(upart, ubad, ngroups, C, r0, num_rot, u, rbad);
 }
 
 void launch_rescale(hipStream_t s, const double *quats, const double *u, int num_rot,
