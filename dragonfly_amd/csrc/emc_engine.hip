@@ -789,6 +789,13 @@ int build_lik_split(emc_engine *e, int X) {
 // Per-chunk brick item lists and work units of the brick merge (geometry only). `rots` holds
 // `total` rotations (a multiple of 64) walked in chunks of C; rotations at or past num_valid,
 // and slots with slot_rot < 0 when slot_rot is given, make no items.
+// A work unit (block) takes at most unit_items entries of a brick's list, fewer where the chunk has
+// few: about kUnitsPerCu units a CU (four are resident), each clearing and adding one brick, in
+// steps of the 256 entries that a block's waves read at once. Against 2048 entries everywhere: 420
+// orientations on 21^3 0.26 -> 0.05 ms (8 units before), 3240 on 125^3 0.71 -> 0.47, 6480 in two modes on 77^3
+// 0.61 -> 0.37, 6300 on 125^3 1.73 -> 1.46; 10,880 on 251^3 take 1536 entries and 6.55 ms either way
+// (256: 7.2).
+constexpr long kUnitsPerCu = 40, kLeastUnitItems = 256;
 int build_bricks(emc_engine *e, std::vector<emc_engine::BrickChunk> &out, const double *rots, int total,
                  int C, int num_valid, const int *slot_rot, int modes) {
     hipStream_t s = e->stream;
@@ -816,12 +823,15 @@ int build_bricks(emc_engine *e, std::vector<emc_engine::BrickChunk> &out, const 
         HIP_TRY(hipMemcpyAsync(counts.data(), e->brick_counts.p, nb * sizeof(int), hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
         long tot = 0;
+        for (size_t b = 0; b < nb; ++b) tot += counts[b];
+        const long share = tot / (kUnitsPerCu * emc::kNumCus);
+        const long per_unit = std::min<long>(e->unit_items, (share / kLeastUnitItems + 1) * kLeastUnitItems);
+        tot = 0;
         std::vector<int4> units;
         for (size_t b = 0; b < nb; ++b) {
             off[b] = tot;
-            for (int k = 0; k < counts[b]; k += e->unit_items)
-                units.push_back(make_int4((int)b, (int)(tot + k),
-                                          (int)(tot + std::min(counts[b], k + e->unit_items)), 0));
+            for (long k = 0; k < counts[b]; k += per_unit)
+                units.push_back(make_int4((int)b, (int)(tot + k), (int)(tot + std::min<long>(counts[b], k + per_unit)), 0));
             tot += counts[b];
         }
         if (tot >= INT32_MAX) return fail(EMC_E_ARG, "brick merge: too many work items");
