@@ -169,8 +169,11 @@ __global__ __launch_bounds__(kBlock) void expand_mp_kernel(
     __shared__ double s_u[kWavesPerBlock][kRTile];
     __shared__ int s_bad[kWavesPerBlock][kRTile];
     const int tid = threadIdx.x;
-    const int c0 = blockIdx.x * kRTile;
-    const int g = blockIdx.y;
+    // the order of expand_kernel: an XCD takes a range of tiles, patch after patch
+    const int ntiles = C / kRTile, per = (ntiles + kNumXcd - 1) / kNumXcd;
+    const int b = blockIdx.x / kNumXcd, tile = blockIdx.x % kNumXcd * per + b % per, g = b / per;
+    if (tile >= ntiles) return;
+    const int c0 = tile * kRTile;
     if (tid < kLogTable) log_table_entry(tid, s_logs);
     __syncthreads();
     const double center = (double)(size / 2);
@@ -310,7 +313,8 @@ void launch_expand_mp(hipStream_t s, const double *rots, const double *model, lo
                       const double *center_t, int num_pix, int r0, int C, int pix_per_group,
                       size_t ldp, int two_terms, _Float16 *lw_hi, _Float16 *lw_lo, double *upart,
                       int *ubad, int bf16) {
-    dim3 grid(C / kRTile, (num_pix + pix_per_group - 1) / pix_per_group);
+    const int per = (C / kRTile + kNumXcd - 1) / kNumXcd;
+    const unsigned grid = (unsigned)((long)kNumXcd * per * ((num_pix + pix_per_group - 1) / pix_per_group));
     if (bf16)
         expand_mp_kernel<__bf16><<<grid, kBlock, 0, s>>>(rots, model, size, qvals, corr, mask, center_t,
                                                          num_pix, r0, C, pix_per_group, ldp, two_terms,
