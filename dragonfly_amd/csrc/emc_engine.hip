@@ -1363,9 +1363,9 @@ int ensure_work(emc_engine *e) {
         e->logw32.release();
         e->p32.release();
     }
-    const size_t per_group = pix_per_group(P, e->C), ngroups = (P + per_group - 1) / per_group;
-    if ((rc = e->upart.alloc(ngroups * (size_t)e->C))) return rc;
-    if ((rc = e->ubad.alloc(ngroups * (size_t)e->C))) return rc;
+    const size_t npatch = (P + 63) / 64;
+    if ((rc = e->upart.alloc(npatch * (size_t)e->C))) return rc;
+    if ((rc = e->ubad.alloc(npatch * (size_t)e->C))) return rc;
     if ((rc = e->rbad.alloc(Rp))) return rc;
     if ((rc = e->u.alloc(Rp))) return rc;
     if ((rc = e->psum_r.alloc(Rp))) return rc;
@@ -1511,9 +1511,9 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
         shrink(e->tom_rows, n_rows);
         if ((rc = fit(e->tom_partial, n_part)) || (rc = fit(e->tom_rows, n_rows))) return rc;
     }
-    const int per_group = pix_per_group(P, C), ngroups = (P + per_group - 1) / per_group;
-    if ((rc = e->upart.alloc((size_t)ngroups * C))) return rc;
-    if ((rc = e->ubad.alloc((size_t)ngroups * C))) return rc;
+    const int per_group = pix_per_group(P, C), npatch = (P + 63) / 64;
+    if ((rc = e->upart.alloc((size_t)npatch * C))) return rc;
+    if ((rc = e->ubad.alloc((size_t)npatch * C))) return rc;
     if ((rc = e->nzmask.alloc((size_t)C * ((P + 63) / 64)))) return rc;
     if ((rc = e->nz_count.alloc(1))) return rc;
     if ((rc = e->u_slot.alloc(S))) return rc;
@@ -1582,8 +1582,8 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
                                      Cc, kFusedPixPerGroup, e->logw.p, e->upart.p, e->ubad.p, e->slot_rot.p, e->lik_off.p,
                                      e->lik_pix.p, e->lik_cnt.p, e->pair_frame.p, e->pair_tile.p, e->tile_off.p,
                                      e->tile_pair.p, t0, e->fused_counter.p, e->Rsub.p);
-                             emc::launch_u_reduce(s, e->upart.p, e->ubad.p, (P + kFusedPixPerGroup - 1) / kFusedPixPerGroup,
-                                                  Cc, s0, S, e->u_slot.p, e->rbad_slot.p);
+                             emc::launch_u_reduce(s, e->upart.p, e->ubad.p, npatch, Cc, s0, S, e->u_slot.p,
+                                                  e->rbad_slot.p);
                              if (nF > 0) {
                                  if (g32)
                                      emc::launch_likelihood_mapped(s, e->logw32.p, Cc, P, e->lik_off.p, e->lik_pix.p,
@@ -1608,7 +1608,7 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
                                           emc::launch_expand(s, e->rots_slot.p, e->model1.p, e->size, e->qvals.p,
                                                              e->corr.p, e->mask.p, P, s0, Cc, per_group,
                                                              e->logw.p, e->upart.p, e->ubad.p, e->slot_rot.p);
-                                      emc::launch_u_reduce(s, e->upart.p, e->ubad.p, ngroups, Cc, s0, S, e->u_slot.p,
+                                      emc::launch_u_reduce(s, e->upart.p, e->ubad.p, npatch, Cc, s0, S, e->u_slot.p,
                                                            e->rbad_slot.p);
                                       return 0;
                                   })))
@@ -2824,7 +2824,15 @@ int emc_maximize(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *stats
     hipStream_t s = e->stream;
     const int N = e->num_data, Rn = e->num_rot, P = e->num_pix, C = e->C, M = e->num_modes;
     const size_t vol = (size_t)e->size * e->size * e->size * M;  // every mode's volume
-    const int per_group = pix_per_group(P, C), ngroups = (P + per_group - 1) / per_group;
+    const int per_group = pix_per_group(P, C), npatch = (P + 63) / 64;
+    // bright pixels' rows in LDS where the default gather's blocks fill the chip
+    emc::HotLists hot{nullptr, 0, 1, nullptr, nullptr};
+    if (!mp && !bgp && !e->lik_part.p && e->lik_tiles < 2 && e->lik_xcd == 1) {
+        if (!e->hot_valid && (rc = build_hot_lists(e))) return rc;
+        const long tiles = std::min(C, e->Rp) / (g32 ? 32 : 16);
+        if (e->hot_num > 0 && tiles * e->hot_parts >= emc::kNumCus)
+            hot = emc::HotLists{e->hot_pix.p, e->hot_num, e->hot_parts, e->hot_mid.p, e->hot_entry.p};
+    }
     const int use_scale = opts->need_scaling && (opts->iteration > 1 || opts->known_scale);
     const int want_psum_d = opts->need_scaling && opts->update_scale;
     float ms_expand = 0.f, ms_lik = 0.f, ms_tomo = 0.f, ms_reduce = 0.f, ms_merge = 0.f;
@@ -2863,7 +2871,7 @@ int emc_maximize(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *stats
         else
             emc::launch_expand(s, e->rots.p, e->model1.p, e->size, e->qvals.p, e->corr.p, e->mask.p,
                                P, r0, Cc, per_group, e->logw.p, e->upart.p, e->ubad.p, nullptr, M, bgp);
-        emc::launch_u_reduce(s, e->upart.p, e->ubad.p, ngroups, Cc, r0, Rn, e->u.p, e->rbad.p);
+        emc::launch_u_reduce(s, e->upart.p, e->ubad.p, npatch, Cc, r0, Rn, e->u.p, e->rbad.p);
         HIP_TRY(hipEventRecord(e->ev[1], s));
         if (mp) {
             const size_t ts = (size_t)N * emc::kRTile;

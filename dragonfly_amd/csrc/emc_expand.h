@@ -63,8 +63,6 @@ __device__ __forceinline__ void expand_block(
     const int nb = model_bricks(size);
     const int t_begin = g * pix_per_group;
     const int t_end = min(num_pix, t_begin + pix_per_group);
-    double uacc = 0.;
-    int bad = 0;  // some mask < 1 pixel has W <= 0 (log W = -inf or NaN)
     for (int tb = t_begin; tb < t_end; tb += 64) {
         const int t = tb + lane;
         if (t < t_end) {
@@ -85,6 +83,8 @@ __device__ __forceinline__ void expand_block(
             }
         }
         __syncthreads();
+        double uacc = 0.;
+        int bad = 0;  // some mask < 1 pixel has W <= 0 (log W = -inf or NaN)
         for (int k = 0; k < 64 / kWavesPerBlock; ++k) {
             const int p = wave + kWavesPerBlock * k;
             const int tt = tb + p;
@@ -112,14 +112,15 @@ __device__ __forceinline__ void expand_block(
                 }
             }
         }
+        sh.u[wave][lane] = uacc;
+        sh.bad[wave][lane] = bad;
         __syncthreads();
-    }
-    sh.u[wave][lane] = uacc;
-    sh.bad[wave][lane] = bad;
-    __syncthreads();
-    if (tid < kRTile) {
-        upart[(size_t)g * C + c0 + tid] = sh.u[0][tid] + sh.u[1][tid] + sh.u[2][tid] + sh.u[3][tid];
-        ubad[(size_t)g * C + c0 + tid] = sh.bad[0][tid] | sh.bad[1][tid] | sh.bad[2][tid] | sh.bad[3][tid];
+        // one partial per 64 pixels, whatever a block's share: the sum's order stays the same
+        if (tid < kRTile) {
+            const size_t at = (size_t)(tb / 64) * C + c0 + tid;
+            upart[at] = sh.u[0][tid] + sh.u[1][tid] + sh.u[2][tid] + sh.u[3][tid];
+            ubad[at] = sh.bad[0][tid] | sh.bad[1][tid] | sh.bad[2][tid] | sh.bad[3][tid];
+        }
     }
     __syncthreads();  // the LDS is free again for the block's next piece of work
 }

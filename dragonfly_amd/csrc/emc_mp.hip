@@ -180,8 +180,6 @@ __global__ __launch_bounds__(kBlock) void expand_mp_kernel(
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int t_begin = g * pix_per_group;
     const int t_end = min(num_pix, t_begin + pix_per_group);
-    double uacc = 0.;
-    int bad = 0;
     for (int tb = t_begin; tb < t_end; tb += 64) {
         const int t = tb + lane;
         if (t < t_end) {
@@ -208,6 +206,8 @@ __global__ __launch_bounds__(kBlock) void expand_mp_kernel(
             }
         }
         __syncthreads();
+        double uacc = 0.;
+        int bad = 0;
         for (int k = 0; k < 64 / kWavesPerBlock; ++k) {
             const int p = wave + kWavesPerBlock * k;
             const int tt = tb + p;
@@ -217,14 +217,14 @@ __global__ __launch_bounds__(kBlock) void expand_mp_kernel(
                 bad |= !(W > 0.);
             }
         }
+        s_u[wave][lane] = uacc;
+        s_bad[wave][lane] = bad;
         __syncthreads();
-    }
-    s_u[wave][lane] = uacc;
-    s_bad[wave][lane] = bad;
-    __syncthreads();
-    if (tid < kRTile) {
-        upart[(size_t)g * C + c0 + tid] = s_u[0][tid] + s_u[1][tid] + s_u[2][tid] + s_u[3][tid];
-        ubad[(size_t)g * C + c0 + tid] = s_bad[0][tid] | s_bad[1][tid] | s_bad[2][tid] | s_bad[3][tid];
+        if (tid < kRTile) {  // one partial per 64 pixels
+            const size_t at = (size_t)(tb / 64) * C + c0 + tid;
+            upart[at] = s_u[0][tid] + s_u[1][tid] + s_u[2][tid] + s_u[3][tid];
+            ubad[at] = s_bad[0][tid] | s_bad[1][tid] | s_bad[2][tid] | s_bad[3][tid];
+        }
     }
 }
 
