@@ -2825,14 +2825,6 @@ int emc_maximize(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *stats
     const int N = e->num_data, Rn = e->num_rot, P = e->num_pix, C = e->C, M = e->num_modes;
     const size_t vol = (size_t)e->size * e->size * e->size * M;  // every mode's volume
     const int per_group = pix_per_group(P, C), npatch = (P + 63) / 64;
-    // bright pixels' rows in LDS where the default gather's blocks fill the chip
-    emc::HotLists hot{nullptr, 0, 1, nullptr, nullptr};
-    if (!mp && !bgp && !e->lik_part.p && e->lik_tiles < 2 && e->lik_xcd == 1) {
-        if (!e->hot_valid && (rc = build_hot_lists(e))) return rc;
-        const long tiles = std::min(C, e->Rp) / (g32 ? 32 : 16);
-        if (e->hot_num > 0 && tiles * e->hot_parts >= emc::kNumCus)
-            hot = emc::HotLists{e->hot_pix.p, e->hot_num, e->hot_parts, e->hot_mid.p, e->hot_entry.p};
-    }
     const int use_scale = opts->need_scaling && (opts->iteration > 1 || opts->known_scale);
     const int want_psum_d = opts->need_scaling && opts->update_scale;
     float ms_expand = 0.f, ms_lik = 0.f, ms_tomo = 0.f, ms_reduce = 0.f, ms_merge = 0.f;
