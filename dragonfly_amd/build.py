@@ -11,7 +11,7 @@ CSRC = os.path.join(HERE, 'csrc')
 LIB = os.path.join(HERE, 'libemc_hip.so')
 INCLUDE = os.path.join(os.path.dirname(HERE), 'include')
 
-SOURCES = ['emc_engine.hip', 'emc_kernels.hip', 'emc_mp.hip', 'emc_merge.hip', 'emc_tomogram.hip', 'emc_nn.hip', 'emc_subset.hip', 'emc_background.hip',
+SOURCES = ['emc_engine.hip', 'emc_kernels.hip', 'emc_mp.hip', 'emc_merge.hip', 'emc_tomogram.hip', 'emc_hot.hip', 'emc_nn.hip', 'emc_subset.hip', 'emc_background.hip',
            'quat_gen.cpp']
 
 # -ffp-contract=off: no fused multiply-add anywhere, so every FP64 value keeps the

@@ -13,13 +13,9 @@
 #pragma once
 
 #include "emc_common.h"
+#include "emc_kernels.h"
 
 namespace emc {
-
-struct RowEntry {
-    int row;
-    float count;  // exact: photon counts are below 2^23 (checked when the lists are built)
-};
 
 // 16 bytes of a row
 template <typename T>

@@ -9,6 +9,12 @@
 
 namespace emc {
 
+// a photon of a gather's list: a row and its (exact, below 2^23) count
+struct RowEntry {
+    int row;
+    float count;
+};
+
 void launch_expand(hipStream_t s, const double *rots, const double *model, long size,
                    const double *qvals, const double *corr, const uint8_t *mask, int num_pix,
                    int r0, int C, int pix_per_group, double *logw, double *upart, int *ubad,
@@ -26,6 +32,22 @@ void launch_copy_f32_brick(hipStream_t s, const double *in, long size, int modes
 void launch_likelihood(hipStream_t s, const float *logw, int C, int num_pix, const long *off,
                        const int *pix, const double *cnt, const uint8_t *blacklist, int num_data,
                        double *G, int r0, int unroll, int xcd_order);
+// ---- likelihood with the brightest pixels' rows in LDS (emc_hot.hip) ----
+constexpr int kHotRows = 288;  // 144 KB of LDS
+// the frames' lists split at mid[d]: {pixel, count} of other pixels, then {place in pix, count} of the
+// num bright ones; parts: frame parts, a block each per orientation tile
+struct HotLists {
+    const int *pix;
+    int num, parts;
+    const long *mid;
+    const RowEntry *entry;
+};
+void launch_hot_lists(hipStream_t s, const long *off, const int *pix, const double *cnt, const int *slot, int num_data,
+                      RowEntry *entry, long *mid);
+void launch_likelihood_hot(hipStream_t s, const double *logw, int C, int num_pix, const HotLists &h, const long *off,
+                           const uint8_t *blacklist, int num_data, double *G, int r0);
+void launch_likelihood_hot(hipStream_t s, const float *logw, int C, int num_pix, const HotLists &h, const long *off,
+                           const uint8_t *blacklist, int num_data, double *G, int r0);
 // Likelihood over X pixel ranges (lists split per range, off8[d * (X + 1) + x]) into partials
 // part[X][C / 64][num_data][64], then added in range order into the chunk's tiles of G.
 void launch_likelihood_split(hipStream_t s, const double *logw, int C, int num_pix, const long *off8, int X,

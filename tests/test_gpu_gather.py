@@ -66,6 +66,28 @@ def test_likelihood_photon_counts(num_rot, unroll):
 
 
 @pytest.mark.parametrize('precision', (0, 3))
+def test_likelihood_bright_pixels(precision):
+    """The likelihood with the brightest pixels' rows in LDS (1344 frames x 3201 orientations: more than
+    256 blocks, the last tile short) against the gather through L2 alone (lik_xcd 2), with frames of
+    every count around the stages, without photons and blacklisted: the same rows, summed in another
+    order."""
+    counts = COUNTS * 56
+    p = counted_problem(counts, 3240)
+    p['quats'] = _lib.quat_gen(4)[:3201]
+    p['fparams']['blacklist'] = (np.arange(len(counts)) % 50 == 3).astype('u1')
+    p['fparams']['num_blacklist'] = int(p['fparams']['blacklist'].sum())
+    out = []
+    for xcd in (1, 2):
+        eng = P.engine_for(p)
+        eng.set_precision(precision)
+        eng.set_option('lik_xcd', xcd)
+        out.append(P.run_engine(eng, dict(iteration=1)))
+        eng.close()
+    for k in ('max_exp', 'p_norm', 'likelihood', 'prob'):
+        assert P.rel_err(out[0][k], out[1][k]) <= 1e-9, k
+
+
+@pytest.mark.parametrize('precision', (0, 3))
 def test_pair_likelihood_photon_counts(precision):
     """The same lists on refinement subsets (pairs of frames and 64-slot tiles) against the
     masked full search of the engine."""
