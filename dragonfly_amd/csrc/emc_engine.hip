@@ -435,6 +435,8 @@ struct emc_engine {
     unsigned long gen = 0, estep_gen = ~0ul;
     DevBuf<float> model32;        // FP32 brick copy of model1 for the FP32-gather expand
     bool model32_valid = false;   // cleared whenever model1 changes
+    DevBuf<emc::BrickVoxel> model_b;  // FP64 brick copy of model1 for the expand (empty: model1 is read)
+    bool model_b_valid = false;       // cleared whenever model1 changes
     DevBuf<long> mass_off;
     DevBuf<int> mass_idx;
     DevBuf<double> mass_out;
@@ -549,6 +551,37 @@ int ensure_model32(emc_engine *e) {
     HIP_TRY(hipGetLastError());
     e->model32_valid = true;
     return 0;
+}
+
+// The FP64 brick copy of model1, refreshed after model1 changed; none (the expand reads model1) for
+// sizes that stay linear or when the device has not 16 times its size to spare.
+int ensure_model_bricks(emc_engine *e) {
+    const size_t n = emc::brick_copy_elems(e->size, e->num_modes);
+    if (n != e->model_b.n) e->model_b_valid = false;
+    if (n == 0 || n > e->model_b.cap) {
+        e->model_b.release();
+        size_t freeb = 0, totalb = 0;
+        HIP_TRY(hipMemGetInfo(&freeb, &totalb));
+        if (n == 0 || freeb / 16 < n * sizeof(emc::BrickVoxel)) return 0;
+    }
+    int rc;
+    if ((rc = e->model_b.alloc(n))) return rc;
+    if (e->model_b_valid) return 0;
+    emc::launch_copy_brick(e->stream, e->model1.p, e->size, e->num_modes, e->model_b.p);
+    HIP_TRY(hipGetLastError());
+    e->model_b_valid = true;
+    return 0;
+}
+
+// log W (raw: W) of Cc orientations from r0 of rots into e->logw, from the brick copy if there is one
+void expand_f64(emc_engine *e, const double *rots, int r0, int Cc, int per_group, const int *slot_rot, int modes,
+                int raw) {
+    if (e->model_b.p)
+        emc::launch_expand(e->stream, rots, e->model_b.p, e->size, e->qvals.p, e->corr.p, e->mask.p, e->num_pix, r0, Cc,
+                           per_group, e->logw.p, e->upart.p, e->ubad.p, slot_rot, modes, raw);
+    else
+        emc::launch_expand(e->stream, rots, e->model1.p, e->size, e->qvals.p, e->corr.p, e->mask.p, e->num_pix, r0, Cc,
+                           per_group, e->logw.p, e->upart.p, e->ubad.p, slot_rot, modes, raw);
 }
 
 // precision modes of the dense-frame products: 1, 2 FP16 log W (one term, hi + lo); 4, 5 the
@@ -1302,7 +1335,10 @@ int ensure_work(emc_engine *e) {
     // the sparse-subset rows are not needed by the plain path
     e->Rsub.release();
     e->RF.release();
+    if (e->R.cap < N * Rp) e->model_b.release();
     if ((rc = e->R.alloc(N * Rp))) return rc;
+    if (e->precision == 3) e->model_b.release();
+    else if ((rc = ensure_model_bricks(e))) return rc;
     size_t freeb = 0, totalb = 0;
     HIP_TRY(hipMemGetInfo(&freeb, &totalb));
     const size_t reserve = ((size_t)4 << 30) + brick_list_extra(e->bricks, Rp, P);
@@ -1491,6 +1527,8 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
         if ((rc = e->sigF_cnt.alloc((size_t)T))) return rc;
         if ((rc = e->sigF_total.alloc(1))) return rc;
     }
+    if (g32 || e->fused) e->model_b.release();
+    else if ((rc = ensure_model_bricks(e))) return rc;
     if (g32 && (rc = ensure_model32(e))) return rc;
     size_t freeb = 0, totalb = 0;
     HIP_TRY(hipMemGetInfo(&freeb, &totalb));
@@ -1652,9 +1690,7 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
                                                              e->corr.p, e->mask.p, P, s0, Cc, per_group,
                                                              e->logw32.p, e->upart.p, e->ubad.p, e->slot_rot.p);
                                       else
-                                          emc::launch_expand(s, e->rots_slot.p, e->model1.p, e->size, e->qvals.p,
-                                                             e->corr.p, e->mask.p, P, s0, Cc, per_group,
-                                                             e->logw.p, e->upart.p, e->ubad.p, e->slot_rot.p);
+                                          expand_f64(e, e->rots_slot.p, s0, Cc, per_group, e->slot_rot.p, 1, 0);
                                       emc::launch_u_reduce(s, e->upart.p, e->ubad.p, npatch, Cc, s0, S, e->u_slot.p,
                                                            e->rbad_slot.p);
                                       return 0;
@@ -2215,7 +2251,7 @@ static int upload_quats(emc_engine *e) {
 
 int emc_set_modes(emc_engine *e, int num_modes) {
     if (e) ++e->gen, ++e->layout_gen;
-    if (e) e->model32_valid = false, e->logw_resident = false;  // model1 changes below
+    if (e) e->model32_valid = e->model_b_valid = false, e->logw_resident = false;  // model1 changes below
     if (!e || num_modes < 1 || num_modes > EMC_MAX_MODES)
         return fail(EMC_E_ARG, "emc_set_modes: num_modes must be 1..%d", EMC_MAX_MODES);
     if (num_modes == e->num_modes) return 0;
@@ -2252,7 +2288,7 @@ int emc_set_quats(emc_engine *e, int num_rot, const double *quats) {
 
 int emc_set_model(emc_engine *e, long size, const double *model1) {
     if (e) ++e->gen;  // the same buffer unless the size changes (then it is allocated anew)
-    if (e) e->model32_valid = false, e->logw_resident = false;  // model1 changes below
+    if (e) e->model32_valid = e->model_b_valid = false, e->logw_resident = false;  // model1 changes below
     if (!e || size < 3 || !model1) return fail(EMC_E_ARG, "emc_set_model: bad argument");
     HIP_TRY(hipSetDevice(e->device));
     const size_t vol = (size_t)size * size * size * e->num_modes;  // every mode's volume
@@ -2272,7 +2308,7 @@ int emc_set_model(emc_engine *e, long size, const double *model1) {
 
 int emc_copy_model(emc_engine *dst, const emc_engine *src) {
     if (dst) ++dst->gen;
-    if (dst) dst->model32_valid = false, dst->logw_resident = false;  // model1 changes below
+    if (dst) dst->model32_valid = dst->model_b_valid = false, dst->logw_resident = false;  // model1 changes below
     if (!dst || !src) return fail(EMC_E_ARG, "emc_copy_model: null engine");
     if (!src->size || !src->model1.p) return fail(EMC_E_STATE, "emc_copy_model: the source holds no model");
     if (src->device != dst->device || src->num_modes != dst->num_modes)
@@ -2726,8 +2762,7 @@ static int update_scale_bg(emc_engine *e, const emc_iter_opts *opts) {
             const int Cc = (Rp - r0 < C) ? (Rp - r0) : C;
             // the views of the current model (the tomogram wrote its own into this buffer)
             if (!(one_chunk && views_ready))
-                emc::launch_expand(s, e->rots.p, e->model1.p, e->size, e->qvals.p, e->corr.p, e->mask.p, P, r0, Cc,
-                                   pix_per_group(P, C), e->logw.p, e->upart.p, e->ubad.p, nullptr, 1, 1);
+                expand_f64(e, e->rots.p, r0, Cc, pix_per_group(P, C), nullptr, 1, 1);
             emc::launch_gradient_d(s, e->logw.p, P, e->R.p, N, r0, Cc, Rn, e->lik_off.p, e->lik_pix.p, e->lik_cnt.p,
                                    e->bg_dmask.p, e->bg_s.p, e->bgscale.p, e->bg.p, rescale, e->bg_gpart.p,
                                    e->bg_gacc.p);
@@ -2908,16 +2943,20 @@ int emc_maximize(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *stats
         const int Cc = (e->Rp - r0 < C) ? (e->Rp - r0) : C;
         float a = 0.f, b = 0.f;
         HIP_TRY(hipEventRecord(e->ev[0], s));
-        if (mp)
-            emc::launch_expand_mp(s, e->rots.p, e->model1.p, e->size, e->qvals.p, e->corr.p, e->mask.p,
-                                  e->center_t.p, P, r0, Cc, per_group, e->mp_ldp, mp_two(e),
-                                  e->lw_hi.p, e->lw_lo.p, e->upart.p, e->ubad.p, mp_bf16(e));
-        else if (g32)
+        if (mp) {
+            if (e->model_b.p)
+                emc::launch_expand_mp(s, e->rots.p, e->model_b.p, e->size, e->qvals.p, e->corr.p, e->mask.p,
+                                      e->center_t.p, P, r0, Cc, per_group, e->mp_ldp, mp_two(e),
+                                      e->lw_hi.p, e->lw_lo.p, e->upart.p, e->ubad.p, mp_bf16(e));
+            else
+                emc::launch_expand_mp(s, e->rots.p, e->model1.p, e->size, e->qvals.p, e->corr.p, e->mask.p,
+                                      e->center_t.p, P, r0, Cc, per_group, e->mp_ldp, mp_two(e),
+                                      e->lw_hi.p, e->lw_lo.p, e->upart.p, e->ubad.p, mp_bf16(e));
+        } else if (g32)
             emc::launch_expand(s, e->rots.p, e->model32.p, e->size, e->qvals.p, e->corr.p, e->mask.p,
                                P, r0, Cc, per_group, e->logw32.p, e->upart.p, e->ubad.p, nullptr, M);
         else
-            emc::launch_expand(s, e->rots.p, e->model1.p, e->size, e->qvals.p, e->corr.p, e->mask.p,
-                               P, r0, Cc, per_group, e->logw.p, e->upart.p, e->ubad.p, nullptr, M, bgp);
+            expand_f64(e, e->rots.p, r0, Cc, per_group, nullptr, M, bgp);
         emc::launch_u_reduce(s, e->upart.p, e->ubad.p, npatch, Cc, r0, Rn, e->u.p, e->rbad.p);
         HIP_TRY(hipEventRecord(e->ev[1], s));
         if (mp) {
@@ -3152,7 +3191,7 @@ int emc_maximize(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *stats
 
 int emc_update_model(emc_engine *e, double alpha, double *rms_change) {
     if (e) ++e->gen;
-    if (e) e->model32_valid = false, e->logw_resident = false;  // model1 changes below
+    if (e) e->model32_valid = e->model_b_valid = false, e->logw_resident = false;  // model1 changes below
     if (!e || !e->size) return fail(EMC_E_STATE, "emc_update_model: model not set");
     HIP_TRY(hipSetDevice(e->device));
     int rc;
@@ -3171,7 +3210,7 @@ int emc_update_model(emc_engine *e, double alpha, double *rms_change) {
 
 int emc_normalize_scale(emc_engine *e, double *mean_scale) {
     if (e) ++e->gen;
-    if (e) e->model32_valid = false, e->logw_resident = false;  // model1 changes below
+    if (e) e->model32_valid = e->model_b_valid = false, e->logw_resident = false;  // model1 changes below
     if (!e || !e->have_params || !e->size) return fail(EMC_E_STATE, "emc_normalize_scale: state not set");
     HIP_TRY(hipSetDevice(e->device));
     int rc;

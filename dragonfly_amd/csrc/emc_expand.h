@@ -18,6 +18,7 @@ namespace emc {
 // (slice_value_f32h).
 // elements of one mode's volume: size^3 for the FP64 model, the brick grid for the FP32 copy
 __device__ __forceinline__ size_t mode_stride(const double *, long size) { return (size_t)(size * size * size); }
+__device__ __forceinline__ size_t mode_stride(const BrickVoxel *, long size) { return BrickLayout(size).elems(); }
 __device__ __forceinline__ size_t mode_stride(const float *, long size) {
     const size_t nb = (size_t)model_bricks(size);
     return nb * nb * nb * kHaloBrickFloats;

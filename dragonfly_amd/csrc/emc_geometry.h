@@ -5,6 +5,7 @@
 #include <cfloat>
 
 #include "emc_common.h"
+#include "emc_kernels.h"
 
 namespace emc {
 
@@ -57,6 +58,38 @@ __device__ __forceinline__ double slice_value(const double *__restrict__ model, 
     const long s2 = (long)sz * sz;
     const VoxelPair m00 = *(const VoxelPair *)m, m01 = *(const VoxelPair *)(m + sz);
     const VoxelPair m10 = *(const VoxelPair *)(m + s2), m11 = *(const VoxelPair *)(m + s2 + sz);
+    const double cx = 1. - c.fx, cy = 1. - c.fy, cz = 1. - c.fz;
+    const double fx = c.fx, fy = c.fy, fz = c.fz;
+    const double v = cx * cy * cz * m00.x + cx * cy * fz * m00.y + cx * fy * cz * m01.x + cx * fy * fz * m01.y +
+                     fx * cy * cz * m10.x + fx * cy * fz * m10.y + fx * fy * cz * m11.x + fx * fy * fz * m11.y;
+    return ok ? v * corr : DBL_MIN;
+}
+
+// FP64 model copy in bricks of 4 x 4 x 4 trilinear cells: 16 rows (x % 4, y % 4) of the five voxels
+// that four cells along z touch, 640 bytes a brick. A compact detector patch rotated into the
+// volume touches a few whole lines of it at any orientation, where lines of 16 voxels along z give
+// a patch across z one or two voxels each.
+struct BrickLayout {
+    int nb, nbz;  // bricks along x and y, and along z
+    __host__ __device__ explicit BrickLayout(long size) : nb((int)((size + 3) / 4)), nbz((int)((size + 2) / 4)) {}
+    static constexpr int kVoxels = 80;
+    __host__ __device__ size_t elems() const { return (size_t)nb * nb * nbz * kVoxels; }
+};
+
+// slice_value from the brick copy: the same values and operations (a copy is below 2^31 elements).
+__device__ __forceinline__ double slice_value(const BrickVoxel *__restrict__ model, long size, const double *rot,
+                                              double q0, double q1, double q2, double corr, double center) {
+    Cell c;
+    const bool ok = locate(rot, q0, q1, q2, center, size, c);
+    const BrickLayout b(size);
+    const int x = ok ? (int)c.x : 0, y = ok ? (int)c.y : 0, z = ok ? (int)c.z : 0;
+    const int row = b.nbz * BrickLayout::kVoxels, slab = b.nb * row;  // a brick further along y, along x
+    const int at = (x >> 2) * slab + (y >> 2) * row + (z >> 2) * BrickLayout::kVoxels + (x & 3) * 20 + (y & 3) * 5 + (z & 3);
+    const int dx = (x & 3) == 3 ? slab - 60 : 20, dy = (y & 3) == 3 ? row - 15 : 5;
+    const double *__restrict__ m = &model->v;
+    const VoxelPair m00 = *(const VoxelPair *)(m + (unsigned)at), m01 = *(const VoxelPair *)(m + (unsigned)(at + dy));
+    const VoxelPair m10 = *(const VoxelPair *)(m + (unsigned)(at + dx)),
+                    m11 = *(const VoxelPair *)(m + (unsigned)(at + dx + dy));
     const double cx = 1. - c.fx, cy = 1. - c.fy, cz = 1. - c.fz;
     const double fx = c.fx, fy = c.fy, fz = c.fz;
     const double v = cx * cy * cz * m00.x + cx * cy * fz * m00.y + cx * fy * cz * m01.x + cx * fy * fz * m01.y +

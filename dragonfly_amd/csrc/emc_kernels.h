@@ -15,10 +15,23 @@ struct RowEntry {
     float count;
 };
 
+// an element of the FP64 brick copy of a model (launch_copy_brick)
+struct BrickVoxel {
+    double v;
+};
+
 void launch_expand(hipStream_t s, const double *rots, const double *model, long size,
                    const double *qvals, const double *corr, const uint8_t *mask, int num_pix,
                    int r0, int C, int pix_per_group, double *logw, double *upart, int *ubad,
                    const int *slot_rot = nullptr, int modes = 1, int raw = 0);
+// the same from the FP64 brick copy of the model
+void launch_expand(hipStream_t s, const double *rots, const BrickVoxel *model, long size,
+                   const double *qvals, const double *corr, const uint8_t *mask, int num_pix,
+                   int r0, int C, int pix_per_group, double *logw, double *upart, int *ubad,
+                   const int *slot_rot = nullptr, int modes = 1, int raw = 0);
+// FP64 copy of `modes` volumes in bricks (BrickLayout); 0 elements: this size stays linear
+size_t brick_copy_elems(long size, int modes);
+void launch_copy_brick(hipStream_t s, const double *in, long size, int modes, BrickVoxel *out);
 // FP32 log W from an FP32 copy of the model (FP32-gather path)
 void launch_expand(hipStream_t s, const double *rots, const float *model, long size,
                    const double *qvals, const double *corr, const uint8_t *mask, int num_pix,
@@ -244,6 +257,11 @@ void launch_center(hipStream_t s, const double *rots, int num_rot, const double 
 void launch_center_base(hipStream_t s, const long *off, const int *pix, const double *cnt,
                         const double *center_t, int num_data, double *base);
 void launch_expand_mp(hipStream_t s, const double *rots, const double *model, long size,
+                      const double *qvals, const double *corr, const uint8_t *mask,
+                      const double *center_t, int num_pix, int r0, int C, int pix_per_group,
+                      size_t ldp, int two_terms, _Float16 *lw_hi, _Float16 *lw_lo, double *upart,
+                      int *ubad, int bf16 = 0);
+void launch_expand_mp(hipStream_t s, const double *rots, const BrickVoxel *model, long size,
                       const double *qvals, const double *corr, const uint8_t *mask,
                       const double *center_t, int num_pix, int r0, int C, int pix_per_group,
                       size_t ldp, int two_terms, _Float16 *lw_hi, _Float16 *lw_lo, double *upart,

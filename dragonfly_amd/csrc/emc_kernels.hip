@@ -962,16 +962,32 @@ static inline unsigned cdiv(size_t a, size_t b) { return (unsigned)((a + b - 1) 
 static inline unsigned grid_cap(size_t blocks) { return (unsigned)(blocks < 65536 ? blocks : 65536); }
 static inline int round_up_int(int a, int b) { return (a + b - 1) / b * b; }
 
-void launch_expand(hipStream_t s, const double *rots, const double *model, long size,
-                   const double *qvals, const double *corr, const uint8_t *mask, int num_pix,
-                   int r0, int C, int pix_per_group, double *logw, double *upart, int *ubad,
-                   const int *slot_rot, int modes, int raw) {
+template <typename MT>
+static void expand_launch(hipStream_t s, const double *rots, const MT *model, long size, const double *qvals,
+                          const double *corr, const uint8_t *mask, int num_pix, int r0, int C, int pix_per_group,
+                          double *logw, double *upart, int *ubad, const int *slot_rot, int modes, int raw) {
 #define EMC_EXPAND(M)                                                                                              \
-    expand_kernel<double, kRTile, double, M><<<expand_grid(C, num_pix, pix_per_group), kBlock, 0, s>>>(             \
+    expand_kernel<double, kRTile, MT, M><<<expand_grid(C, num_pix, pix_per_group), kBlock, 0, s>>>(                 \
         rots, model, size, qvals, corr, mask, num_pix, r0, C, pix_per_group, logw, upart, ubad, slot_rot, modes, raw)
     if (modes > 1) EMC_EXPAND(true);
     else EMC_EXPAND(false);
 #undef EMC_EXPAND
+}
+
+void launch_expand(hipStream_t s, const double *rots, const double *model, long size,
+                   const double *qvals, const double *corr, const uint8_t *mask, int num_pix,
+                   int r0, int C, int pix_per_group, double *logw, double *upart, int *ubad,
+                   const int *slot_rot, int modes, int raw) {
+    expand_launch(s, rots, model, size, qvals, corr, mask, num_pix, r0, C, pix_per_group, logw, upart, ubad, slot_rot,
+                  modes, raw);
+}
+
+void launch_expand(hipStream_t s, const double *rots, const BrickVoxel *model, long size,
+                   const double *qvals, const double *corr, const uint8_t *mask, int num_pix,
+                   int r0, int C, int pix_per_group, double *logw, double *upart, int *ubad,
+                   const int *slot_rot, int modes, int raw) {
+    expand_launch(s, rots, model, size, qvals, corr, mask, num_pix, r0, C, pix_per_group, logw, upart, ubad, slot_rot,
+                  modes, raw);
 }
 
 void launch_expand(hipStream_t s, const double *rots, const float *model, long size,
@@ -1027,6 +1043,34 @@ __global__ void copy_f32_brick_kernel(const double *__restrict__ in, long size, 
         }
         out[i] = v;
     }
+}
+
+// The FP64 brick copy (BrickLayout); voxels past the volume's end (the last row's padding) are 0.
+__global__ void copy_brick_kernel(const double *__restrict__ in, long size, int modes, BrickVoxel *__restrict__ out) {
+    const BrickLayout b(size);
+    const size_t per_mode = b.elems(), n = per_mode * modes, vol = (size_t)size * size * size;
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
+        const size_t m = i / per_mode;
+        const unsigned j = (unsigned)(i % per_mode), brick = j / BrickLayout::kVoxels, l = j % BrickLayout::kVoxels;
+        const unsigned x = brick / (b.nb * b.nbz) * 4 + l / 20, y = brick / b.nbz % b.nb * 4 + l / 5 % 4,
+                       z = brick % b.nbz * 4 + l % 5;
+        out[i].v = x < size && y < size && z < size ? in[m * vol + ((size_t)x * size + y) * size + z] : 0.;
+    }
+}
+
+// From 160^3: there a model passes the L2 of an XCD several times and the copy pays. Expand stage from
+// model1 and from the copy, ms: 10,880 orientations on 251^3 5.93, 4.94 (in FP16 rows 6.1, 5.5), 25,680 slots of
+// refinement subsets 12.6, 11.0, 10,880 on 185^3 2.69, 2.40; on 125^3 0.78, 0.78 (6300) and 0.43, 0.43 (3240), on 77^3
+// 0.27, 0.28. The copy of 251^3 (158 MB) takes 0.1 ms.
+size_t brick_copy_elems(long size, int modes) {
+    const size_t n = size >= 160 ? BrickLayout(size).elems() : 0;
+    return n < ((size_t)1 << 31) ? n * modes : 0;
+}
+
+void launch_copy_brick(hipStream_t s, const double *in, long size, int modes, BrickVoxel *out) {
+    const size_t n = brick_copy_elems(size, modes);
+    if (n == 0) return;
+    copy_brick_kernel<<<grid_cap(cdiv(n, 256)), 256, 0, s>>>(in, size, modes, out);
 }
 
 size_t model_brick_elems(long size, int modes) {

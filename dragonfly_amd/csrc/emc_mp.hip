@@ -157,9 +157,9 @@ __global__ __launch_bounds__(kBlock) void center_base_kernel(const long *__restr
 // and the centred log W split into 16-bit (T: FP16 or BF16) hi / lo rows lw[c][t] (lanes
 // along pixels, so the stores are contiguous without a transpose). mask >= 1 and non-finite
 // entries store 0.
-template <typename T>
+template <typename T, typename MT>
 __global__ __launch_bounds__(kBlock) void expand_mp_kernel(
-    const double *__restrict__ rots, const double *__restrict__ model, long size,
+    const double *__restrict__ rots, const MT *__restrict__ model, long size,
     const double *__restrict__ qvals, const double *__restrict__ corr,
     const uint8_t *__restrict__ mask, const double *__restrict__ center_t, int num_pix, int r0,
     int C, int pix_per_group, size_t ldp, int two_terms, T *__restrict__ lw_hi,
@@ -308,7 +308,8 @@ void launch_center_base(hipStream_t s, const long *off, const int *pix, const do
         off, pix, cnt, center_t, num_data, base);
 }
 
-void launch_expand_mp(hipStream_t s, const double *rots, const double *model, long size,
+template <typename MT>
+static void expand_mp_launch(hipStream_t s, const double *rots, const MT *model, long size,
                       const double *qvals, const double *corr, const uint8_t *mask,
                       const double *center_t, int num_pix, int r0, int C, int pix_per_group,
                       size_t ldp, int two_terms, _Float16 *lw_hi, _Float16 *lw_lo, double *upart,
@@ -316,13 +317,31 @@ void launch_expand_mp(hipStream_t s, const double *rots, const double *model, lo
     const int per = (C / kRTile + kNumXcd - 1) / kNumXcd;
     const unsigned grid = (unsigned)((long)kNumXcd * per * ((num_pix + pix_per_group - 1) / pix_per_group));
     if (bf16)
-        expand_mp_kernel<__bf16><<<grid, kBlock, 0, s>>>(rots, model, size, qvals, corr, mask, center_t,
+        expand_mp_kernel<__bf16, MT><<<grid, kBlock, 0, s>>>(rots, model, size, qvals, corr, mask, center_t,
                                                          num_pix, r0, C, pix_per_group, ldp, two_terms,
                                                          (__bf16 *)lw_hi, (__bf16 *)lw_lo, upart, ubad);
     else
-        expand_mp_kernel<_Float16><<<grid, kBlock, 0, s>>>(rots, model, size, qvals, corr, mask, center_t,
+        expand_mp_kernel<_Float16, MT><<<grid, kBlock, 0, s>>>(rots, model, size, qvals, corr, mask, center_t,
                                                            num_pix, r0, C, pix_per_group, ldp, two_terms, lw_hi,
                                                            lw_lo, upart, ubad);
+}
+
+void launch_expand_mp(hipStream_t s, const double *rots, const double *model, long size,
+                      const double *qvals, const double *corr, const uint8_t *mask,
+                      const double *center_t, int num_pix, int r0, int C, int pix_per_group,
+                      size_t ldp, int two_terms, _Float16 *lw_hi, _Float16 *lw_lo, double *upart,
+                      int *ubad, int bf16) {
+    expand_mp_launch(s, rots, model, size, qvals, corr, mask, center_t, num_pix, r0, C, pix_per_group, ldp, two_terms,
+                     lw_hi, lw_lo, upart, ubad, bf16);
+}
+
+void launch_expand_mp(hipStream_t s, const double *rots, const BrickVoxel *model, long size,
+                      const double *qvals, const double *corr, const uint8_t *mask,
+                      const double *center_t, int num_pix, int r0, int C, int pix_per_group,
+                      size_t ldp, int two_terms, _Float16 *lw_hi, _Float16 *lw_lo, double *upart,
+                      int *ubad, int bf16) {
+    expand_mp_launch(s, rots, model, size, qvals, corr, mask, center_t, num_pix, r0, C, pix_per_group, ldp, two_terms,
+                     lw_hi, lw_lo, upart, ubad, bf16);
 }
 
 void launch_posterior_fp16(hipStream_t s, const double *P, int num_data, int r0, int C, size_t ldd,

@@ -246,3 +246,19 @@ def test_merge_some_and_all_orientations(frames, beta):
         assert P.rel_err(eng.get('model2'), o['model2']) <= 1e-9, merge_mode
         assert P.rel_err(eng.get('inter_weight'), o['inter_weight']) <= 1e-9, merge_mode
     eng.close()
+
+
+@pytest.mark.parametrize('size', (159, 160, 161, 162, 163))
+def test_expand_from_brick_copy(size):
+    """log W from model1 (159) and from its brick copy, with volumes that end at every place of a
+    brick, with two models after one another."""
+    p = P.build(P.tiny_config(size=size, num_data=12, mean_count=60.), quats=_lib.quat_gen(2)[:70], num_ave=100)
+    p['fparams']['beta'] = np.full(12, 0.05)
+    eng = P.engine_for(p)
+    for model in (p['model1'], p['model1'][::-1].copy()):
+        eng.set_model(model)
+        o = P.run_oracle(p, dict(iteration=1), model1=model)
+        g = P.run_engine(eng, dict(iteration=1))
+        for k in ('u', 'max_exp', 'p_norm', 'likelihood', 'prob', 'model2'):
+            assert P.rel_err(g[k], o[k]) <= 1e-9, k
+    eng.close()
