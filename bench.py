@@ -204,8 +204,8 @@ def roofline(prob, itr, stage_tot, steps, nchunks, pairs, workload, value_bytes=
     D = itr.tot_num_data - int((itr.blacklist != 0).sum())
     npix = len(prob['det']['mask'])
     C = itr.quat.num_rot / nchunks
-    kern = {'likelihood': ('likelihood_kernel', ps['lik']),
-            'tomogram': ('tomogram_part_kernel', ps['tomo'])}
+    kern = {'likelihood': ('likelihood_hot_kernel', ps['lik']),
+            'tomogram': ('tomogram_rows_kernel', ps['tomo'])}
     stage = max(kern, key=lambda k: stage_tot.get(k, 0.))
     name, (n, m) = kern[stage]
     launch_ms = stage_tot[stage] / steps / nchunks
@@ -259,7 +259,7 @@ def roofline_learned(res, slots, num_pix, size, num_photons, num_frames, workloa
             'merge': masks + 4. * nnz + 16. * float(size) ** 3}
     ms = {'expand': st1.get('expand', 0.), 'tomogram': st.get('tomogram', 0.), 'reduce': st.get('reduce', 0.),
           'merge': st.get('merge', 0.)}
-    kernels = {'expand': 'expand_kernel', 'tomogram': 'tomogram_part_w128_kernel', 'reduce': 'pair_tomogram_kernel',
+    kernels = {'expand': 'expand_kernel', 'tomogram': 'tomogram_rows_kernel', 'reduce': 'pair_tomogram_kernel',
                'merge': 'merge_brick_model_kernel'}
     stage = max(ms, key=ms.get)
     per = {k: dict(kernel=kernels[k], launch_ms=round(ms[k], 3), compulsory_bytes=round(comp[k]),
