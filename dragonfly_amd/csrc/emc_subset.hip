@@ -26,6 +26,7 @@
 #include "emc_common.h"
 #include "emc_expand.h"
 #include "emc_gather.h"
+#include "emc_grid.h"
 #include "emc_kernels.h"
 
 namespace emc {
@@ -1069,17 +1070,24 @@ static void pair_tomogram_launch(hipStream_t s, const TP *P, const long *tile_of
     // photons a quarter the stage takes 15.1 ms, 19.6 by whole patches; with 5, 2.0 against 1.8
     const bool quarter = bk.base && bk.sub == 4 && bk.per_tile >= 64L * bk.nr;
     const int nr = quarter ? bk.nr : nranges;
-    const unsigned grid = (unsigned)((ntiles + kNumXcd - 1) / kNumXcd * kNumXcd) * (unsigned)nr;
+    // a block a (tile, range): 257,000 slots x 66,820 pixels in quarter patches are past a grid's 32 bits
+    for_each_tile_span(ntiles, kNumXcd, nr, kBlock, [&](long first, long count, unsigned grid) {
+        const int from = t0 + (int)first, n = (int)count;
+        const size_t slot = (size_t)first * kRTile;
+        const PT *sums = partial ? partial + slot * num_pix : nullptr;
+        VT *v = view + slot * num_pix;
+        unsigned long long *nz = nzmask ? nzmask + slot * ((num_pix + 63) / 64) : nullptr;
 #define EMC_PT(B, BITS, FULL)                                                                                        \
     pair_tomogram_kernel<B, BITS, FULL, TP, VT, PT><<<grid, kBlock, 0, s>>>(                                         \
-        P, tile_off, sig_pair, sig_frame, sig_cnt, foff, roff, nr, fpix, fcnt, psum_slot, t0, ntiles, num_pix, partial, \
-        view, nzmask, fr.RF, fr.nF, fr.row, fr.frame, fr.cnt, bk)
-    if (quarter && fr.RF) EMC_PT(true, 4, true);
-    else if (quarter) EMC_PT(true, 4, false);
-    else if (bk.base && fr.RF) EMC_PT(true, 6, true);
-    else if (bk.base) EMC_PT(true, 6, false);
-    else EMC_PT(false, 6, true);
+        P, tile_off, sig_pair, sig_frame, sig_cnt, foff, roff, nr, fpix, fcnt, psum_slot, from, n, num_pix, sums, v, \
+        nz, fr.RF, fr.nF, fr.row, fr.frame, fr.cnt, bk)
+        if (quarter && fr.RF) EMC_PT(true, 4, true);
+        else if (quarter) EMC_PT(true, 4, false);
+        else if (bk.base && fr.RF) EMC_PT(true, 6, true);
+        else if (bk.base) EMC_PT(true, 6, false);
+        else EMC_PT(false, 6, true);
 #undef EMC_PT
+    });
 }
 
 void launch_pair_tomogram(hipStream_t s, const double *P, const long *tile_off, const int *sig_pair,
