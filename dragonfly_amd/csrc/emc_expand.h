@@ -8,6 +8,7 @@
 
 #include "emc_common.h"
 #include "emc_geometry.h"
+#include "emc_log.h"
 
 namespace emc {
 
@@ -34,7 +35,7 @@ struct ExpandShared {
     static constexpr bool f32 = sizeof(MT) == sizeof(float);
     using V = typename std::conditional<f32, float, double>::type;
     V rot[f32 ? kRTile * 9 : 1];
-    double2 logs[f32 ? 1 : kLogTable];
+    LogEntry logs[f32 ? 1 : kLogTable];
     V tile[64][kRTile + 1];
     double u[kWavesPerBlock][kRTile];
     int bad[kWavesPerBlock][kRTile];
@@ -56,7 +57,7 @@ __device__ __forceinline__ void expand_block(
     if constexpr (f32)
         for (int i = tid; i < kRTile * 9; i += kBlock) sh.rot[i] = (float)rots[(size_t)(r0 + c0) * 9 + i];
     else if (tid < kLogTable)
-        log_table_entry(tid, sh.logs);
+        sh.logs[tid] = kLogEntries.entry[tid];
     __syncthreads();
     // padding slots of the subset order (slot_rot < 0) get W = 1; lane = orientation when storing
     const bool pad = slot_rot != nullptr && slot_rot[r0 + c0 + lane] < 0;

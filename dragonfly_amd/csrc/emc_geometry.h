@@ -97,36 +97,6 @@ __device__ __forceinline__ double slice_value(const BrickVoxel *__restrict__ mod
     return ok ? v * corr : DBL_MIN;
 }
 
-// log of a positive normal number by table (P. T. P. Tang's scheme: the mantissa's interval gives 1 / c
-// and log c, and log1p of r = z / c - 1, |r| <= 2^-8, is a polynomial): 20 FP64 operations and one
-// 16-byte LDS read where the device library's log takes 70 operations. The two intervals beside 1
-// take c = 1, so that a logarithm near 0 keeps its relative precision. Against 80-bit logarithms of 4
-// million values each: at most 1.5 ulp in [0.5, 2] (7e-17 absolute), 0.6 where |log x| > 2. Anything
-// else goes to log().
-constexpr int kLogTable = 128;
-__device__ __forceinline__ void log_table_entry(int i, double2 *tab) {
-    const double inv = 1. / __hiloint2double(0x3fe60000 + (i << 13) + (1 << 12), 0);
-    const bool one = i == 79 || i == 80;  // [1 - 2^-8, 1) and [1, 1 + 2^-7)
-    tab[i] = one ? make_double2(1., 0.) : make_double2(inv, -log(inv));
-}
-__device__ __forceinline__ double table_log(double x, const double2 *tab) {
-    const int hi = __double2hiint(x);
-    if ((unsigned)hi - 0x00100000u >= 0x7fe00000u) return log(x);  // 0, subnormal, negative, inf, NaN
-    const int tmp = hi - 0x3fe60000;  // intervals of the mantissa from 0.6875 to 1.375
-    const double2 t = tab[(tmp >> 13) & (kLogTable - 1)];
-    const double z = __hiloint2double(hi - (tmp & (int)0xfff00000), __double2loint(x));
-    const double r = __builtin_fma(z, t.x, -1.), k = (double)(tmp >> 20);
-    const double kh = k * 0x1.62e42fefa3800p-1, w = kh + t.y;  // k ln 2: the high part times k is exact
-    const double s = w + r, lo = __builtin_fma(k, 0x1.ef35793c76730p-45, ((kh - w) + t.y) + ((w - s) + r));
-    double p = __builtin_fma(r, -1. / 8., 1. / 7.);
-    p = __builtin_fma(r, p, -1. / 6.);
-    p = __builtin_fma(r, p, 1. / 5.);
-    p = __builtin_fma(r, p, -1. / 4.);
-    p = __builtin_fma(r, p, 1. / 3.);
-    p = __builtin_fma(r, p, -1. / 2.);
-    return s + __builtin_fma(r * r, p, lo);
-}
-
 // FP32 model copy in bricks of 4 x 4 x 4 trilinear cells: brick (X/4, Y/4, Z/4) of an nb^3
 // grid (nb = (size - 2) / 4 + 1, the cells x <= size - 2 of the grid) holds the 5 x 5 x 5
 // corners of its cells (shared faces are stored twice), padded to 128 floats, z fastest. The

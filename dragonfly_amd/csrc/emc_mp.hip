@@ -33,6 +33,7 @@
 #include "emc_gemm.h"
 #include "emc_geometry.h"
 #include "emc_kernels.h"
+#include "emc_log.h"
 
 namespace emc {
 
@@ -164,7 +165,7 @@ __global__ __launch_bounds__(kBlock) void expand_mp_kernel(
     const uint8_t *__restrict__ mask, const double *__restrict__ center_t, int num_pix, int r0,
     int C, int pix_per_group, size_t ldp, int two_terms, T *__restrict__ lw_hi,
     T *__restrict__ lw_lo, double *__restrict__ upart, int *__restrict__ ubad) {
-    __shared__ double2 s_logs[kLogTable];
+    __shared__ LogEntry s_logs[kLogTable];
     __shared__ double s_tile[64][kRTile + 1];
     __shared__ double s_u[kWavesPerBlock][kRTile];
     __shared__ int s_bad[kWavesPerBlock][kRTile];
@@ -174,7 +175,7 @@ __global__ __launch_bounds__(kBlock) void expand_mp_kernel(
     const int b = blockIdx.x / kNumXcd, tile = blockIdx.x % kNumXcd * per + b % per, g = b / per;
     if (tile >= ntiles) return;
     const int c0 = tile * kRTile;
-    if (tid < kLogTable) log_table_entry(tid, s_logs);
+    if (tid < kLogTable) s_logs[tid] = kLogEntries.entry[tid];
     __syncthreads();
     const double center = (double)(size / 2);
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
