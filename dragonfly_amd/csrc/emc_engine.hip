@@ -5,7 +5,6 @@
 
 #include <algorithm>
 #include <cmath>
-#include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
 #include <cctype>
@@ -20,119 +19,16 @@
 
 #include "../../include/emc_hip.h"
 #include "emc_common.h"
+#include "emc_host.h"
 #include "emc_kernels.h"
 
 namespace {
 
-thread_local std::string g_last_error;
-
-int fail(int code, const char *fmt, ...) {
-    char buf[512];
-    va_list ap;
-    va_start(ap, fmt);
-    vsnprintf(buf, sizeof buf, fmt, ap);
-    va_end(ap);
-    g_last_error = buf;
-    return code;
-}
-
-// Counts device allocations and frees of the engine buffers (every engine): a captured graph
-// holds buffer addresses, so it is captured again once any buffer may have moved.
-std::atomic<unsigned long> g_alloc_gen{0};
-
-#define HIP_TRY(expr)                                                                        \
-    do {                                                                                     \
-        hipError_t err_ = (expr);                                                            \
-        if (err_ != hipSuccess)                                                              \
-            return fail(EMC_E_HIP, "%s failed: %s", #expr, hipGetErrorString(err_));        \
-    } while (0)
-
-// Device buffer with an element count.
-template <typename T>
-struct DevBuf {
-    T *p = nullptr;
-    size_t n = 0;    // elements in use
-    size_t cap = 0;  // elements allocated: a smaller request reuses the allocation
-    DevBuf() = default;
-    DevBuf(const DevBuf &) = delete;
-    DevBuf &operator=(const DevBuf &) = delete;
-    DevBuf(DevBuf &&o) noexcept : p(o.p), n(o.n), cap(o.cap) {
-        o.p = nullptr;
-        o.n = o.cap = 0;
-    }
-    DevBuf &operator=(DevBuf &&o) noexcept {
-        if (this != &o) {
-            release();
-            p = o.p;
-            n = o.n;
-            cap = o.cap;
-            o.p = nullptr;
-            o.n = o.cap = 0;
-        }
-        return *this;
-    }
-    ~DevBuf() { release(); }
-    int alloc(size_t count) {
-        if (p && count <= cap && count > 0) {
-            n = count;
-            return 0;
-        }
-        release();
-        if (count == 0) return 0;
-        ++g_alloc_gen;
-        hipError_t err = hipMalloc((void **)&p, count * sizeof(T));
-        if (err != hipSuccess) {
-            p = nullptr;
-            return fail(EMC_E_NOMEM, "hipMalloc of %zu bytes failed: %s", count * sizeof(T),
-                        hipGetErrorString(err));
-        }
-        n = cap = count;
-        return 0;
-    }
-    int upload(const T *src, size_t count, hipStream_t s) {
-        int rc = alloc(count);
-        if (rc) return rc;
-        if (count) HIP_TRY(hipMemcpyAsync(p, src, count * sizeof(T), hipMemcpyHostToDevice, s));
-        return 0;
-    }
-    void release() {
-        if (p) {
-            ++g_alloc_gen;
-            (void)hipFree(p);
-        }
-        p = nullptr;
-        n = cap = 0;
-    }
-};
-
-// Page-locked host memory (grow only) that the per-iteration lists are built in, so that
-// their uploads run at the host link's speed without a staging copy.
-template <typename T>
-struct PinnedBuf {
-    T *p = nullptr;
-    size_t cap = 0;
-    PinnedBuf() = default;
-    PinnedBuf(const PinnedBuf &) = delete;
-    PinnedBuf &operator=(const PinnedBuf &) = delete;
-    ~PinnedBuf() { release(); }
-    int reserve(size_t count) {
-        count = std::max<size_t>(count, 1);
-        if (p && count <= cap) return 0;
-        release();
-        const size_t want = count + count / 4;  // room for lists that grow a little
-        if (hipHostMalloc((void **)&p, want * sizeof(T), hipHostMallocDefault) != hipSuccess) {
-            p = nullptr;
-            return fail(EMC_E_NOMEM, "hipHostMalloc of %zu bytes failed", want * sizeof(T));
-        }
-        cap = want;
-        return 0;
-    }
-    void release() {
-        if (p) (void)hipHostFree(p);
-        p = nullptr;
-        cap = 0;
-    }
-};
+using emc::DevBuf;
+using emc::fail;
+using emc::g_alloc_gen;
+using emc::g_last_error;
+using emc::PinnedBuf;
 
 // Host threads for a loop over n items, at least per items each, at most 16.
 int host_threads(long n, long per) {

@@ -88,3 +88,53 @@ int main() {
 }''')
     worst, mean = map(float, out.split())
     assert worst <= 0.52 and mean <= 0.251, out
+
+
+# What of HIP the engine's buffers call, with a runtime whose last error stays until it is read (as HIP's
+# does) and whose allocations fail above a size
+FAKE_HIP = r'''#pragma once
+#include <cstdlib>
+#include <cstring>
+typedef int hipError_t;
+typedef void *hipStream_t;
+enum { hipSuccess = 0, hipErrorOutOfMemory = 2, hipMemcpyHostToDevice = 1, hipHostMallocDefault = 0 };
+inline hipError_t last = hipSuccess;
+inline size_t most = 1000;
+inline hipError_t hipMalloc(void **p, size_t n) { return n > most ? last = hipErrorOutOfMemory : (*p = malloc(n), hipSuccess); }
+inline hipError_t hipHostMalloc(void **p, size_t n, int) { return hipMalloc(p, n); }
+inline hipError_t hipFree(void *p) { return free(p), hipSuccess; }
+inline hipError_t hipHostFree(void *p) { return hipFree(p); }
+inline hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, int, hipStream_t) { return memcpy(d, s, n), hipSuccess; }
+inline hipError_t hipGetLastError() { const hipError_t e = last; return last = hipSuccess, e; }
+inline const char *hipGetErrorString(hipError_t) { return "out of memory"; }
+'''
+
+
+def test_failed_allocation_leaves_no_error(run_cpp, tmp_path):
+    """A buffer that gets no memory reports it once and leaves no error for the check after the next launch
+    to find: the engine goes on without lists and staging memory that are only there for speed."""
+    (tmp_path / 'hip').mkdir()
+    (tmp_path / 'hip' / 'hip_runtime_api.h').write_text(FAKE_HIP)
+    run_cpp(r'''#include <vector>
+#include "emc_host.h"
+static int failing_call() {
+    HIP_TRY(last = hipErrorOutOfMemory);
+    return 0;
+}
+int main() {
+    emc::DevBuf<double> d;
+    emc::PinnedBuf<char> h;
+    const std::vector<double> v(2000);
+    if (d.alloc(10) || hipGetLastError()) return 1;
+    if (d.alloc(2000) != EMC_E_NOMEM || d.p || d.n || d.cap) return 2;
+    if (emc::g_last_error.find("16000 bytes") == std::string::npos) return 3;
+    if (hipGetLastError()) return 4;
+    if (d.upload(v.data(), 2000, nullptr) != EMC_E_NOMEM || hipGetLastError()) return 5;
+    if (h.reserve(2000) != EMC_E_NOMEM || h.p || hipGetLastError()) return 6;
+    if (failing_call() != EMC_E_HIP || hipGetLastError()) return 7;
+    if (d.alloc(10) || d.upload(v.data(), 100, nullptr) || h.reserve(10)) return 8;
+    // a bad argument asks the runtime nothing
+    last = hipErrorOutOfMemory;
+    if (emc::fail(EMC_E_ARG, "x") != EMC_E_ARG || hipGetLastError() != hipErrorOutOfMemory) return 9;
+    return 0;
+}''', '-I%s' % tmp_path)
