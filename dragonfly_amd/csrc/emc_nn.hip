@@ -308,9 +308,14 @@ bool tiles_ok(int M, int N, int K, size_t lda, size_t ldb) {
 }
 }  // namespace
 
-// Tile of a product: 256 x 256 where its blocks give every CU one, else 64 x 64 (K a multiple of
+// Tile of a product: 256 x 256 where its blocks give half of the CUs one, else 64 x 64 (K a multiple of
 // its step): a minibatch of 1024 rows by 1024 outputs makes 16 large blocks or 256 small ones.
-// Loss and gradients of 1024 rows through 4096-1024-1024-1024-3240: 910 -> 344 us.
+// Loss and gradients of 1024 rows through 4096-1024-1024-1024-3240: 910 -> 344 us. The large tile takes one
+// block's time up to 256 of them, the small one grows with the output from 256 blocks on, at about
+// half the rate (a wave's one 32 x 32 tile needs two LDS fragments an MFMA). Forward / weight gradient at K =
+// 1024 and 4096, us, small against large: 16 large tiles 9/8 and 27/26 against 46/32 and 121/107; 104: 40/34 and
+// 116/115 against 48/34 and 124/111; 128: 44/38 and 128/126 against 49/35 and 128/114; 208: 69/58 and 207/199 against
+// 49/37 and 129/115.
 struct NnLaunch {
     NnTile tile;
     int mt, nt;
@@ -320,7 +325,7 @@ struct NnLaunch {
 
 static NnLaunch nn_launch(int M, int N, int K) {
     const long large = (long)(M / kGemmBM) * (N / kGemmBN);
-    if (large < kNumCus && K % kSmallBK == 0) {
+    if (large < kNumCus / 2 && K % kSmallBK == 0) {
         const int mt = M / kSmallTile, nt = N / kSmallTile;
         return {NnTile::kSmall, mt, nt, (unsigned)(mt * nt), kSmallLdsElems * sizeof(bf16)};
     }

@@ -157,9 +157,9 @@ def test_trained_proposal_captures_posterior_mass():
 
 
 @pytest.mark.parametrize('M, N, K', ((256, 256, 128), (256, 512, 384), (256, 256, 192), (512, 256, 160),
-                                     (4096, 4096, 64), (4096, 4096, 256)))
+                                     (4096, 4096, 64), (4096, 4096, 256), (3840, 2048, 128), (4096, 2048, 128)))
 def test_products_of_every_tile(M, N, K):
-    """The small tile (K a multiple of 128, fewer large tiles than CUs), the large one in steps of
+    """The small tile (K a multiple of 128, up to 120 large tiles), the large one (from 128) in steps of
     64 and of 32: one step, odd numbers of steps, ragged valid rows and columns. BF16 products are
     exact in FP32, so a sum of K terms is within K 2^-23 of the sum of their magnitudes."""
     import torch
