@@ -393,6 +393,8 @@ class Engine:
         _check(lib().emc_set_option(self._h, name.encode(), int(value)))
 
     def get_option(self, name):
+        """An option's value, or lik_hot: the bright pixels whose rows the last iteration's likelihood kept
+        in LDS (0: another likelihood kernel ran)."""
         v = C.c_int(0)
         _check(lib().emc_get_option(self._h, name.encode(), C.byref(v)))
         return v.value

@@ -217,6 +217,7 @@ struct emc_engine {
     // the lists split into photons of bright pixels (hot_pix, hot_num of them) and others
     bool hot_valid = false;
     int hot_num = 0, hot_parts = 1;
+    int lik_hot = 0;  // bright pixels' rows in LDS in the last iteration's likelihood (0: another kernel ran)
     DevBuf<int> hot_pix, hot_slot;
     DevBuf<long> hot_mid;
     DevBuf<emc::RowEntry> hot_entry;
@@ -1365,6 +1366,7 @@ int ensure_work(emc_engine *e) {
 // every slot tile of the full frames). Same outputs as emc_maximize's plain path;
 // per-orientation outputs are mapped back to the caller's orientation order.
 int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *stats) {
+    e->lik_hot = 0;
     int rc;
     hipStream_t s = e->stream;
     const int N = e->num_data, Rn = e->num_rot, P = e->num_pix, S = e->num_slots, T = e->num_tiles;
@@ -2018,6 +2020,10 @@ int emc_set_option(emc_engine *e, const char *name, int value) {
 
 int emc_get_option(emc_engine *e, const char *name, int *value) {
     if (!e || !name || !value) return fail(EMC_E_ARG, "emc_get_option: null argument");
+    if (!strcmp(name, "lik_hot")) {
+        *value = e->lik_hot;
+        return 0;
+    }
     for (const EngineOption &o : kOptions)
         if (!strcmp(o.name, name)) {
             *value = e->*(o.field);
@@ -2811,6 +2817,7 @@ int emc_maximize(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *stats
         if (e->hot_num > 0 && tiles * e->hot_parts >= emc::kNumCus)
             hot = emc::HotLists{e->hot_pix.p, e->hot_num, e->hot_parts, e->hot_mid.p, e->hot_entry.p};
     }
+    e->lik_hot = hot.num;
     const int use_scale = opts->need_scaling && (opts->iteration > 1 || opts->known_scale);
     const int want_psum_d = opts->need_scaling && opts->update_scale;
     float ms_expand = 0.f, ms_lik = 0.f, ms_tomo = 0.f, ms_reduce = 0.f, ms_merge = 0.f;

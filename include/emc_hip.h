@@ -184,7 +184,9 @@ int emc_set_precision(emc_engine *e, int mode);
  * work unit, >= 64), tomo_buckets (1, default: the subset path's pair tomogram reads per-(tile,
  * pixel range) photon lists of its significant rows; 0: each block walks its tile's rows). Start
  * values come from EMC_<NAME>. The likelihood with the brightest pixels' rows in LDS is used
- * with lik_tiles 1, lik_xcd 1 and lik_split 1 (the defaults).                                */
+ * with lik_tiles 1, lik_xcd 1 and lik_split 1 (the defaults), where there is a block of it for every CU; it
+ * does not read lik_unroll. emc_get_option also answers lik_hot (read only): how many pixels' rows it kept in
+ * the last iteration, 0 when another kernel ran.                                            */
 int emc_set_option(emc_engine *e, const char *name, int value);
 int emc_get_option(emc_engine *e, const char *name, int *value);
 /* per-frame state of struct iterate: scale, beta, blacklist, fcounts, sum_fact,

@@ -67,11 +67,11 @@ def test_likelihood_photon_counts(num_rot, unroll):
 
 @pytest.mark.parametrize('precision', (0, 3))
 def test_likelihood_bright_pixels(precision):
-    """The likelihood with the brightest pixels' rows in LDS (1344 frames x 3201 orientations: more than
-    256 blocks, the last tile short) against the gather through L2 alone (lik_xcd 2), with frames of
+    """The likelihood with the brightest pixels' rows in LDS (1536 frames x 3201 orientations: 12 parts of
+    51 FP64 or 25.5 FP32 tiles, more than 256 blocks, the last tile short) against the gather through L2 alone (lik_xcd 2), with frames of
     every count around the stages, without photons and blacklisted: the same rows, summed in another
     order."""
-    counts = COUNTS * 56
+    counts = COUNTS * 64
     p = counted_problem(counts, 3240)
     p['quats'] = _lib.quat_gen(4)[:3201]
     p['fparams']['blacklist'] = (np.arange(len(counts)) % 50 == 3).astype('u1')
@@ -82,6 +82,7 @@ def test_likelihood_bright_pixels(precision):
         eng.set_precision(precision)
         eng.set_option('lik_xcd', xcd)
         out.append(P.run_engine(eng, dict(iteration=1)))
+        assert (eng.get_option('lik_hot') > 0) == (xcd == 1)  # else the gather is compared with itself
         eng.close()
     for k in ('max_exp', 'p_norm', 'likelihood', 'prob'):
         assert P.rel_err(out[0][k], out[1][k]) <= 1e-9, k
