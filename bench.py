@@ -187,13 +187,22 @@ def load_traffic(workload, kernel):
     return float(ent['bytes_per_launch']), tab[workload].get('_profile', 'profiles/pmc_traffic.json')
 
 
-def roofline(prob, itr, stage_tot, steps, nchunks, pairs, workload, value_bytes=8):
+def likelihood_kernel(engine):
+    """The likelihood kernel that the engine's last full-search iteration ran."""
+    if engine.get_option('lik_hot') > 0:
+        return 'likelihood_hot_kernel'
+    if engine.get_option('lik_split') > 1:
+        return 'likelihood_split_kernel'
+    return 'likelihood_kernel' if engine.get_option('lik_tiles') > 1 else 'likelihood_rows_kernel'
+
+
+def roofline(prob, itr, stage_tot, steps, nchunks, pairs, workload, lik_kernel, value_bytes=8):
     """HBM roofline of the dominant photon kernel (likelihood or tomogram gather, whichever
     takes longer), timed with HIP events on the engine's stream.
 
     `achieved` counts compulsory bytes: every operand of one launch moved once -- for the
-    likelihood the log W chunk (8 B per orientation x pixel), the frames' photon lists
-    (int32 pixel + f64 count) and R written (8 B per pair); for the tomogram the posterior
+    likelihood (`lik_kernel`) the log W chunk (8 B per orientation x pixel), the frames' photon
+    lists (int32 pixel + f64 count) and R written (8 B per pair); for the tomogram the posterior
     chunk (8 B per pair), the pixels' photon lists (int32 frame + f64 count) and the view
     written (8 B per orientation x pixel). `gather_bytes` is what the kernel requests through
     the caches instead (one 8-byte log W or P value per photon and orientation, 12 n + 4 m
@@ -204,7 +213,7 @@ def roofline(prob, itr, stage_tot, steps, nchunks, pairs, workload, value_bytes=
     D = itr.tot_num_data - int((itr.blacklist != 0).sum())
     npix = len(prob['det']['mask'])
     C = itr.quat.num_rot / nchunks
-    kern = {'likelihood': ('likelihood_hot_kernel', ps['lik']),
+    kern = {'likelihood': (lik_kernel, ps['lik']),
             'tomogram': ('tomogram_rows_kernel', ps['tomo'])}
     stage = max(kern, key=lambda k: stage_tot.get(k, 0.))
     name, (n, m) = kern[stage]
@@ -341,6 +350,8 @@ def bench_dense(args):
     D, R = itr.tot_num_data, itr.quat.num_rot
     pairs = (D - int((itr.blacklist != 0).sum())) * R
     el_mp, st_mp, nch_mp, tr_mp = run_steps(recon, itr, args.warmup, args.steps, keep_models=True)
+    # FP32 gathers have the bright-row kernel and the plain gather only
+    lik_kernel = 'likelihood_hot_kernel' if recon.engine.get_option('lik_hot') else 'likelihood_rows_kernel'
     recon.free()
     del recon
     torch.cuda.empty_cache()
@@ -377,7 +388,7 @@ def bench_dense(args):
         path = 'mixed precision, %d-term FP16 log W' % terms
         dtype = 'f16 products / f32 accumulate / f64 rest'
     else:
-        roof = roofline(prob, itr, st_mp, args.steps, nch_mp, pairs, None, value_bytes=4)
+        roof = roofline(prob, itr, st_mp, args.steps, nch_mp, pairs, None, lik_kernel, value_bytes=4)
         path = 'FP32 log W and posterior gathers, FP64 sums'
         dtype = 'f32 gathers / f64 rest'
     
@@ -892,7 +903,8 @@ def main():
 
     default_size = args.num_data is None and args.num_div is None
     roof = None if bgd is not None else roofline(prob, itr, stage_tot, args.steps, nchunks, pairs,
-                                                 args.config if default_size else None)
+                                                 args.config if default_size else None,
+                                                 likelihood_kernel(recon.engine))
     cpu = None
     if not args.no_cpu:
         threads = min(16, os.cpu_count() or 1)

@@ -82,6 +82,22 @@ def test_roofline_of_the_judged_iteration_units():
     assert st['tomogram']['frac'] is None
 
 
+@pytest.mark.parametrize('options, kernel', (
+    (dict(lik_hot=288, lik_split=1, lik_tiles=1), 'likelihood_hot_kernel'),
+    (dict(lik_hot=0, lik_split=1, lik_tiles=1), 'likelihood_rows_kernel'),
+    (dict(lik_hot=0, lik_split=4, lik_tiles=2), 'likelihood_split_kernel'),
+    (dict(lik_hot=0, lik_split=1, lik_tiles=2), 'likelihood_kernel')))
+def test_roofline_names_the_likelihood_that_ran(options, kernel):
+    from types import SimpleNamespace
+    import numpy as np
+    assert bench.likelihood_kernel(SimpleNamespace(get_option=options.get)) == kernel
+    # 2 frames x 64 orientations of 2 pixels: the likelihood stage is the longer one
+    prob = dict(frames=dict(place_ones=np.array([0, 1, 1]), place_multi=np.array([0])), det=dict(mask=np.zeros(2, 'u1')))
+    itr = SimpleNamespace(tot_num_data=2, blacklist=np.zeros(2, 'u1'), quat=SimpleNamespace(num_rot=64))
+    out = bench.roofline(prob, itr, {'likelihood': 2., 'tomogram': 1.}, 1, 1, 128, None, kernel)
+    assert out['kernel'] == kernel and out['launch_ms'] == 2.
+
+
 def test_cpu_baseline_fit_on_a_tiny_problem():
     """bench.cpu_baseline end to end on the tiny geometry (3240 orientations, 60 frames, the
     oracle on 2 threads at three orientation subsets of 32 frames): each run's split adds up
