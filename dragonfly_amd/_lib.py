@@ -399,6 +399,10 @@ class Engine:
         _check(lib().emc_get_option(self._h, name.encode(), C.byref(v)))
         return v.value
 
+    def option_in_use(self, name):
+        """False where the last iteration's kernels do not read the option."""
+        return name != 'lik_unroll' or self.get_option('lik_hot') == 0
+
     def cell_posterior(self, num_coarse, quat_mapping):
         """(num_data, num_coarse) float32: each frame's posterior mass in each coarse cell
         (quat_mapping[r] = cell of orientation r) after the last iteration."""

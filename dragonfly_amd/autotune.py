@@ -24,9 +24,13 @@ PLAIN_SPACE = (
 def tune(engine, iteration=1, need_scaling=0, known_scale=0, space=PLAIN_SPACE, log=None):
     """Tune `engine` in place. Returns {option: chosen value} and the timings
     {option: {value: ms}}. Every candidate runs one full maximize (model2, inter_weight and
-    the per-frame outputs are overwritten; scale factors are left alone)."""
+    the per-frame outputs are overwritten; scale factors are left alone). An option that the
+    kernels of the last iteration do not read is left as it is."""
     chosen, timings = {}, {}
+    in_use = getattr(engine, 'option_in_use', lambda name: True)
     for name, values, stages in space:
+        if not in_use(name):
+            continue
         times = {}
         for v in values:
             engine.set_option(name, v)

@@ -234,6 +234,31 @@ def test_autotune_greedy_choice():
     assert not any(eng.calls)
 
 
+def test_autotune_leaves_options_that_nothing_reads():
+    """An option that the kernels in use do not read is not decided by the noise of equal runs."""
+    from dragonfly_amd import autotune
+
+    class FakeEngine:
+        def __init__(self):
+            self.opt = {'lik_xcd': 1, 'lik_unroll': 8}
+
+        def set_option(self, name, value):
+            self.opt[name] = value
+
+        def option_in_use(self, name):
+            return name != 'lik_unroll' or self.opt['lik_xcd'] != 1  # as the bright-row likelihood
+
+        def maximize(self, iteration, need_scaling, update_scale, known_scale):
+            # whatever is tried later looks a little faster
+            self.t = getattr(self, 't', 10.) - 0.01
+            return {'stage_ms': {'likelihood': self.t + 5. * (self.opt['lik_xcd'] != 1)}}
+
+    eng = FakeEngine()
+    space = (('lik_xcd', (1, 2, 0), ('likelihood',)), ('lik_unroll', (8, 16, 4), ('likelihood',)))
+    chosen, times = autotune.tune(eng, space=space)
+    assert chosen == {'lik_xcd': 1} and eng.opt['lik_unroll'] == 8 and 'lik_unroll' not in times
+
+
 def test_refine_lists_match_refine_sets():
     """The flattened proposal lists equal the per-frame sets (top-k sorted, or every cell for
     a fall-back frame), and a reused buffer gives the same lists."""
