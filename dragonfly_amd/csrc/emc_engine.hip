@@ -1412,6 +1412,9 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
         if ((rc = e->blacklist_full.alloc(nF))) return rc;
     }  // with no full frames RF keeps its room: the next set of lists may have them again
     const bool g32 = e->precision == 3;
+    // the full frames' sums: FP64, or FP32 with FP32 gathers and one frame range (several ranges add to
+    // the sums of the ones before, which are not rounded in between)
+    const bool sums32 = g32 && e->full_parts == 1;
     if (g32 && (rc = e->Rsub32.alloc((size_t)std::max<long>(e->num_pairs, 1) * emc::kRTile))) return rc;
     if ((rc = e->sig_pair.alloc((size_t)std::max<long>(e->num_pairs, 1)))) return rc;
     if ((rc = e->sig_frame.alloc((size_t)std::max<long>(e->num_pairs, 1)))) return rc;
@@ -1440,10 +1443,10 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
                             : 0) +
                     e->upart.cap * sizeof(double) + e->ubad.cap * sizeof(int);
     budget = std::min(budget, (size_t)120 << 30);
-    // per slot column: log W / view, the full frames' sums and their posterior column (FP64; with
-    // FP32 gathers all FP32), and the view's nonzero masks
-    const size_t parts_col = nF > 0 ? 1 : 0;
-    const size_t per_col = ((size_t)P * (1 + parts_col) + (size_t)nF) * (g32 ? sizeof(float) : sizeof(double)) +
+    // per slot column: log W / view and the full frames' posterior column (FP64; with FP32 gathers
+    // FP32), the full frames' sums, and the view's nonzero masks
+    const size_t per_col = ((size_t)P + (size_t)nF) * (g32 ? sizeof(float) : sizeof(double)) +
+                           (nF > 0 ? (size_t)P * (sums32 ? sizeof(float) : sizeof(double)) : 0) +
                            (nF > 0 ? mark_bytes_per_column(nF) : 0) +
                            (size_t)((P + 63) / 64) * sizeof(unsigned long long) + u_bytes_per_column(P);
     size_t cmax = budget / per_col;
@@ -1476,23 +1479,27 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
         if (!g32 && (rc = e->logw.alloc((size_t)P * C))) return rc;
     }
     if (g32 && e->logw32.cap > (size_t)P * C128) e->logw_resident = false;  // released below
+    const size_t n_part = nF > 0 ? (size_t)P * C : 0, n_part32 = sums32 ? n_part : 0, n_part64 = sums32 ? 0 : n_part;
     if (g32) {
-        const size_t n_part = nF > 0 ? (size_t)P * C : 0, n_logw = (size_t)P * C128, n_p32 = (size_t)nF * C;
-        e->tom_partial.release();
+        const size_t n_logw = (size_t)P * C128, n_p32 = (size_t)nF * C;
+        if (sums32) e->tom_partial.release();
+        else e->tom_partial32.release();
         e->tom_rows.release();
         shrink(e->logw32, n_logw);
-        shrink(e->tom_partial32, n_part);
+        shrink(e->tom_partial32, n_part32);
+        shrink(e->tom_partial, n_part64);
         shrink(e->p32, n_p32);
-        if ((rc = fit(e->logw32, n_logw)) || (rc = fit(e->tom_partial32, n_part)) || (rc = fit(e->p32, n_p32)))
+        if ((rc = fit(e->logw32, n_logw)) || (rc = fit(e->tom_partial32, n_part32)) ||
+            (rc = fit(e->tom_partial, n_part64)) || (rc = fit(e->p32, n_p32)))
             return rc;
     } else {
         e->tom_partial32.release();
         e->logw32.release();
         e->p32.release();
-        const size_t n_part = nF > 0 ? (size_t)P * C : 0, n_rows = (size_t)nF * C;
-        shrink(e->tom_partial, n_part);
+        const size_t n_rows = (size_t)nF * C;
+        shrink(e->tom_partial, n_part64);
         shrink(e->tom_rows, n_rows);
-        if ((rc = fit(e->tom_partial, n_part)) || (rc = fit(e->tom_rows, n_rows))) return rc;
+        if ((rc = fit(e->tom_partial, n_part64)) || (rc = fit(e->tom_rows, n_rows))) return rc;
     }
     const int per_group = pix_per_group(P, C), npatch = (P + 63) / 64;
     if ((rc = e->upart.alloc((size_t)npatch * C))) return rc;
@@ -1768,14 +1775,18 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
             const auto &bc = e->slot_bricks[k];
             const int t0 = bc.r0 / emc::kRTile, t1 = (bc.r0 + bc.Cc) / emc::kRTile;
             if (parts && (rc = timed(6, [&] {
-                               if (g32) {
+                               if (g32)
                                    emc::launch_posterior_rows(s, e->RF.p, nF, bc.r0, bc.Cc, S, e->p32.p, e->tom_marks.p);
-                                   emc::launch_tomogram_rows(s, e->p32.p, e->tom_marks.p, nF, bc.Cc, flists, P, e->tom_partial32.p);
-                               } else {
+                               else
                                    emc::launch_posterior_rows(s, e->RF.p, nF, bc.r0, bc.Cc, S, e->tom_rows.p, e->tom_marks.p);
+                               if (sums32)
+                                   emc::launch_tomogram_rows(s, e->p32.p, e->tom_marks.p, nF, bc.Cc, flists, P, e->tom_partial32.p);
+                               else if (g32)
+                                   emc::launch_tomogram_rows(s, e->p32.p, e->tom_marks.p, nF, bc.Cc, flists, P, nullptr, 0,
+                                                             e->tom_partial.p, false);
+                               else
                                    emc::launch_tomogram_rows(s, e->tom_rows.p, e->tom_marks.p, nF, bc.Cc, flists, P, nullptr, 0,
                                                              e->tom_partial.p, false);
-                               }
                                return 0;
                            })))
                 return rc;
@@ -1784,7 +1795,13 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
             unsigned long long *nz = g32 || device_weights || cached_weight ? e->nzmask.p : nullptr;
             if ((rc = timed(7, [&] {
                      // FP32 gathers: an FP32 view (in the FP32 log W buffer, free in the M-step)
-                     if (g32)
+                     if (g32 && !sums32)
+                         emc::launch_pair_tomogram(s, e->Rsub32.p, e->tile_off.p, e->sig_pair.p, e->sig_frame.p,
+                                                   e->sig_cnt.p, e->fsort_off.p, e->fsort_roff.p, e->nranges,
+                                                   e->fsort_pix.p, e->fsort_cnt.p, e->psum_slot.p, t0, t1 - t0, P,
+                                                   parts ? e->tom_partial.p : nullptr, e->logw32.p, nz,
+                                                   frows, bkv);
+                     else if (g32)
                          emc::launch_pair_tomogram(s, e->Rsub32.p, e->tile_off.p, e->sig_pair.p, e->sig_frame.p,
                                                    e->sig_cnt.p, e->fsort_off.p, e->fsort_roff.p, e->nranges,
                                                    e->fsort_pix.p, e->fsort_cnt.p, e->psum_slot.p, t0, t1 - t0, P,

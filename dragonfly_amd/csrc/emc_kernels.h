@@ -194,7 +194,7 @@ void launch_tomogram_rows(hipStream_t s, const double *rows, const unsigned long
 void launch_tomogram_rows(hipStream_t s, const float *rows, const unsigned long long *marks, int num_data, int C,
                           const TomoLists &l, int num_pix,
                           const double *psum, int num_psum, double *view, bool rmajor);
-// tile-major FP32 sums (each the FP64 sum rounded once per frame range)
+// tile-major FP32 sums of one frame range (l.nparts is 1)
 void launch_tomogram_rows(hipStream_t s, const float *rows, const unsigned long long *marks, int num_data, int C,
                           const TomoLists &l, int num_pix,
                           float *sums);
@@ -347,6 +347,12 @@ void launch_pair_tomogram(hipStream_t s, const float *P, const long *tile_off, c
                           const int *sig_frame, const int *sig_cnt, const long *foff, const int *roff, int nranges,
                           const int *fpix, const double *fcnt, const double *psum_slot, int t0, int ntiles,
                           int num_pix, const float *partial, float *view, unsigned long long *nzmask,
+                          const SigFullRows &fr = SigFullRows(), const PairBuckets &bk = PairBuckets());
+// an FP32 view that starts from FP64 sums
+void launch_pair_tomogram(hipStream_t s, const float *P, const long *tile_off, const int *sig_pair,
+                          const int *sig_frame, const int *sig_cnt, const long *foff, const int *roff, int nranges,
+                          const int *fpix, const double *fcnt, const double *psum_slot, int t0, int ntiles,
+                          int num_pix, const double *partial, float *view, unsigned long long *nzmask,
                           const SigFullRows &fr = SigFullRows(), const PairBuckets &bk = PairBuckets());
 // pairs with some P > 1e-6 in their row, per tile in the tile's order (flag: num_pairs bytes;
 // sig_pair / sig_frame: tile_off layout; sig_cnt: per tile)

@@ -1108,6 +1108,15 @@ void launch_pair_tomogram(hipStream_t s, const float *P, const long *tile_off, c
                          t0, ntiles, num_pix, partial, view, nzmask, fr, bk);
 }
 
+void launch_pair_tomogram(hipStream_t s, const float *P, const long *tile_off, const int *sig_pair,
+                          const int *sig_frame, const int *sig_cnt, const long *foff, const int *roff, int nranges,
+                          const int *fpix, const double *fcnt, const double *psum_slot, int t0, int ntiles,
+                          int num_pix, const double *partial, float *view,
+                          unsigned long long *nzmask, const SigFullRows &fr, const PairBuckets &bk) {
+    pair_tomogram_launch(s, P, tile_off, sig_pair, sig_frame, sig_cnt, foff, roff, nranges, fpix, fcnt, psum_slot,
+                         t0, ntiles, num_pix, partial, view, nzmask, fr, bk);
+}
+
 template <typename TP>
 static void sig_pairs_launch(hipStream_t s, const TP *P, long num_pairs, const long *tile_off, const int *tile_pair,
                              const int *tile_frame, int num_tiles, uint8_t *flag, int *sig_pair, int *sig_frame,

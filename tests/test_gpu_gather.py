@@ -170,6 +170,29 @@ def test_full_frames_tomogram_ranges(precision, part_frames):
     assert P.rel_err(out[0]['model2'], out[1]['model2']) <= (1e-9 if precision == 0 else 1e-4)
 
 
+def test_full_frames_sums_over_ranges_keep_precision():
+    """FP32 gathers, full frames in one and in 64 frame ranges: the sums pass from range to range without
+    a rounding, so a view differs by the roundings of the single range's sum and of the two views: 2^-24
+    each, whatever the number of ranges. Three orientations keep a voxel near one view's error."""
+    n = 64 * len(COUNTS[4:])
+    p = counted_problem(COUNTS[4:] * 64, 3)
+    p['fparams']['beta'] = np.full(n, 1e-3)  # every orientation counts for every frame
+    off, rq = np.arange(n + 1, dtype='i8'), np.full(n, -1, 'i4')
+    out = []
+    for part_frames in (12500, 20):
+        eng = P.engine_for(p)
+        eng.set_precision(3)
+        eng.set_option('sig_full_rows', 0)
+        eng.set_option('tomo_parts', 64)
+        eng.set_option('full_part_frames', part_frames)
+        eng.set_refine(1, np.zeros(3, 'i4'), off, rq)
+        out.append(P.run_engine(eng, dict(iteration=1))['model2'])
+        eng.close()
+    on = out[0] > 0.
+    assert on.sum() > 100 and np.array_equal(on, out[1] > 0.)
+    assert np.abs(out[1][on] / out[0][on] - 1.).max() <= 3. * 2. ** -24
+
+
 @pytest.mark.parametrize('precision', (0, 3))
 @pytest.mark.parametrize('repeat, buckets', ((1, 1), (8, 1), (8, 0)))
 @pytest.mark.parametrize('full', (False, True))
