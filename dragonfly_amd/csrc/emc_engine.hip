@@ -107,6 +107,8 @@ std::vector<int> morton_order(int num_pix, const double *qvals) {
     return perm;
 }
 
+// Device memory that lists which only serve speed leave free (of the 4 GB that the chunk width leaves)
+constexpr size_t kLeaveFree = (size_t)1 << 30;
 constexpr int kFusedPixPerGroup = 1024;  // of the persistent expand + likelihood
 // Pixels of one expand block: 64, a block's least (one compact patch): the blocks that an XCD holds at
 // once then read neighbouring patches of the same orientations, one region of the model, instead
@@ -701,7 +703,7 @@ int build_hot_lists(emc_engine *e) {
     for (size_t i = 0; i < num; ++i) slot[pix[i] = bright[i].second] = (int)i;
     int rc;
     e->hot_valid = false;
-    if (e->hot_mid.alloc(N) || e->hot_entry.alloc(std::max<size_t>(e->lik_pix.n, 1))) {
+    if (!e->hot_mid.alloc_spare(N, kLeaveFree) || !e->hot_entry.alloc_spare(std::max<size_t>(e->lik_pix.n, 1), kLeaveFree)) {
         e->hot_mid.release();  // no room: the plain gather
         e->hot_num = 0;
         e->hot_valid = true;
@@ -1760,7 +1762,7 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
                      HIP_TRY(hipMemcpyAsync(&total, e->bk_base.p + T, sizeof(long), hipMemcpyDeviceToHost, s));
                      HIP_TRY(hipStreamSynchronize(s));
                      // no room, or a tile too full: the blocks walk their tiles' pairs
-                     if (total < 0 || e->bk_photon.alloc((size_t)std::max(total, 1L))) return 0;
+                     if (total < 0 || !e->bk_photon.alloc_spare((size_t)std::max(total, 1L), kLeaveFree)) return 0;
                      emc::launch_pair_buckets(s, T, e->tile_off.p, e->sig_pair.p, e->sig_frame.p, e->sig_cnt.p, frows,
                                               e->fsort_off.p, e->fsort_pix.p, e->fsort_cnt.p, nr, e->bucket_bits, e->bk_loc.p, e->bk_tot.p, e->bk_base.p,
                                               e->bk_photon.p, 1);

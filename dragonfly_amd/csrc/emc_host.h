@@ -83,6 +83,18 @@ struct DevBuf {
         n = cap = count;
         return 0;
     }
+    // Memory that only serves speed: count elements if the device keeps `leave` bytes free beside them (the
+    // iteration and the calls after it allocate as well), else none and false.
+    bool alloc_spare(size_t count, size_t leave) {
+        if (p && count <= cap && count > 0) {
+            n = count;
+            return true;
+        }
+        release();
+        size_t freeb = 0, totalb = 0;
+        if (hipMemGetInfo(&freeb, &totalb) != hipSuccess) return (void)hipGetLastError(), false;
+        return freeb >= leave && count <= (freeb - leave) / sizeof(T) && alloc(count) == 0;
+    }
     int upload(const T *src, size_t count, hipStream_t s) {
         int rc = alloc(count);
         if (rc) return rc;

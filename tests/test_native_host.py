@@ -105,6 +105,7 @@ inline hipError_t hipHostMalloc(void **p, size_t n, int) { return hipMalloc(p, n
 inline hipError_t hipFree(void *p) { return free(p), hipSuccess; }
 inline hipError_t hipHostFree(void *p) { return hipFree(p); }
 inline hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, int, hipStream_t) { return memcpy(d, s, n), hipSuccess; }
+inline hipError_t hipMemGetInfo(size_t *f, size_t *t) { return *f = *t = most, hipSuccess; }
 inline hipError_t hipGetLastError() { const hipError_t e = last; return last = hipSuccess, e; }
 inline const char *hipGetErrorString(hipError_t) { return "out of memory"; }
 '''
@@ -136,5 +137,21 @@ int main() {
     // a bad argument asks the runtime nothing
     last = hipErrorOutOfMemory;
     if (emc::fail(EMC_E_ARG, "x") != EMC_E_ARG || hipGetLastError() != hipErrorOutOfMemory) return 9;
+    return 0;
+}''', '-I%s' % tmp_path)
+
+
+def test_lists_for_speed_leave_memory_free(run_cpp, tmp_path):
+    """alloc_spare takes memory only if `leave` bytes stay free beside it, keeps a large enough buffer, and
+    hands a smaller one back before it looks."""
+    (tmp_path / 'hip').mkdir()
+    (tmp_path / 'hip' / 'hip_runtime_api.h').write_text(FAKE_HIP)
+    run_cpp(r'''#include "emc_host.h"
+int main() {
+    emc::DevBuf<double> d;  // 1000 bytes free
+    if (!d.alloc_spare(100, 200) || d.n != 100 || d.cap != 100) return 1;
+    if (!d.alloc_spare(50, 100000) || d.n != 50 || d.cap != 100) return 2;
+    if (d.alloc_spare(101, 200) || d.p || d.cap) return 3;
+    if (d.alloc_spare(1, 1001) || d.alloc_spare((size_t)-1 / 8, 0) || hipGetLastError()) return 4;
     return 0;
 }''', '-I%s' % tmp_path)
