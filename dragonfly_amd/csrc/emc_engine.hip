@@ -2214,8 +2214,7 @@ int emc_set_model(emc_engine *e, long size, const double *model1) {
     HIP_TRY(hipSetDevice(e->device));
     const size_t vol = (size_t)size * size * size * e->num_modes;  // every mode's volume
     int rc;
-    // one spare element: the interpolation reads z edges of two voxels (slice_value)
-    if ((rc = e->model1.alloc(vol + 1)) || (rc = e->model1.upload(model1, vol, e->stream))) return rc;
+    if ((rc = e->model1.upload(model1, vol, e->stream))) return rc;
     if ((rc = e->model2.alloc(vol))) return rc;
     if ((rc = e->weight.alloc(vol))) return rc;
     emc::launch_fill(e->stream, e->model2.p, vol, 0.);
@@ -2238,7 +2237,7 @@ int emc_copy_model(emc_engine *dst, const emc_engine *src) {
     const long size = src->size;
     const size_t vol = (size_t)size * size * size * dst->num_modes;
     int rc;
-    if ((rc = dst->model1.alloc(vol + 1)) || (rc = dst->model2.alloc(vol)) || (rc = dst->weight.alloc(vol))) return rc;
+    if ((rc = dst->model1.alloc(vol)) || (rc = dst->model2.alloc(vol)) || (rc = dst->weight.alloc(vol))) return rc;
     // the source's model is complete on its own stream before the copy on the destination's
     HIP_TRY(hipStreamSynchronize(src->stream));
     HIP_TRY(hipMemcpyAsync(dst->model1.p, src->model1.p, vol * sizeof(double), hipMemcpyDeviceToDevice, dst->stream));

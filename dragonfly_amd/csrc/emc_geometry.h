@@ -44,15 +44,15 @@ typedef double VoxelPair __attribute__((ext_vector_type(2), aligned(8)));
 // DBL_MIN, so the loads of several calls can be in flight at once. The reference wraps the far
 // corner, (x + 1) % size, but cells stop at size - 2, so the wrap never happens: the far
 // corners are at fixed distances from the near one and the two corners of each z edge are one
-// 16-byte load. A 1^3 model has no cell: its (unused) loads stay at its one voxel and the spare
-// element that the engine allocates behind a model. Without the three 64-bit remainders and four of the eight loads the FP64
-// expand of 25,680 orientations x 66,820 pixels on 251^3 takes 16.0 ms instead of 19.4.
+// 16-byte load (models have 3 voxels an axis or more, so those of cell (0, 0, 0) are inside). Without
+// the three 64-bit remainders and four of the eight loads the FP64 expand of 25,680 orientations x 66,820
+// pixels on 251^3 took 16.0 ms instead of 19.4.
 __device__ __forceinline__ double slice_value(const double *__restrict__ model, long size,
                                               const double *rot, double q0, double q1, double q2,
                                               double corr, double center) {
     Cell c;
     const bool ok = locate(rot, q0, q1, q2, center, size, c);
-    const int sz = size < 2 ? 0 : (int)size;
+    const int sz = (int)size;
     const long at = (long)(int)((unsigned)c.x * (unsigned)sz + (unsigned)c.y) * sz + c.z;
     const double *__restrict__ m = model + (ok ? at : 0);
     const long s2 = (long)sz * sz;
