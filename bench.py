@@ -247,9 +247,9 @@ def roofline_learned(res, slots, num_pix, size, num_photons, num_frames, workloa
     expand: the FP32 model copy read (halo bricks, 512 B per 4^3 cells) and log W written
       (4 B per orientation x pixel);
     tomogram (full frames): their FP32 posterior read (4 B per frame x orientation), their
-      photon lists (int32 frame + f64 count) and the partial views written (4 B per
+      photon lists (int32 frame + f64 count) and their sums written (4 B per
       orientation x pixel);
-    reduce (pair tomogram): the partial views read, the photon lists of every frame, the
+    reduce (pair tomogram): those sums read, the photon lists of every frame, the
       nonzero masks (8 B per orientation x 64-pixel patch) and the nonzero view entries
       written (4 B each; the engine counts them);
     merge: the nonzero masks and nonzero view entries read and the merged volume read and

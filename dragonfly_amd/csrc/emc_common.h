@@ -36,7 +36,8 @@ constexpr int kUnitItems = 2048;
 constexpr int kPairRange = 64;
 
 // Tomogram rows (emc_tomogram.hip): bytes of one frame's row of a tile, and frames of one launch
-// (2 MB of rows, half an XCD's L2)
+// (2 MB of rows, half an XCD's L2; more where they would make more ranges than option tomo_parts, 8
+// by default, allows: past 131,072 frames)
 constexpr int kTomoRowBytes = 128;
 constexpr int kFramesPerTomoRange = 16384;
 constexpr int kTomoUnitEntries = 8192;  // photons of one block's pixels, about

@@ -113,9 +113,9 @@ constexpr int kFusedPixPerGroup = 1024;  // of the persistent expand + likelihoo
 // Pixels of one expand block: 64, a block's least (one compact patch): the blocks that an XCD holds at
 // once then read neighbouring patches of the same orientations, one region of the model, instead
 // of walking distant 1024-pixel groups side by side, and small detectors fill the chip. More, up to
-// 1024, only where the grid would pass 4 million blocks or 65,535 groups. 64, 128, 256 and 1024 pixels: 5.99, 6.45, 7.15
-// and 8.14 ms (10,880 orientations on 251^3), 2.68, 3.11, 3.32 and 3.69 with FP32 gathers, 0.43, 0.44, 0.47 and
-// 0.58 (3240 on 125^3), 12.7, 12.4, 13.5 and 14.5 (refinement subsets).
+// 1024, only where the grid would pass 4 million blocks or 65,535 groups. 64, 128, 256 and 1024 pixels: 4.54, 4.95, 5.21
+// and 5.74 ms (10,880 orientations on 251^3), 2.58, 3.16, 3.38 and 3.78 with FP32 gathers, 0.42, 0.44, 0.47 and
+// 0.58 (3240 on 125^3), 10.2, 9.9, 10.7 and 11.1 (refinement subsets).
 int pix_per_group(long num_pix, long C) {
     int n = 64;
     while (n < 1024 && ((num_pix + n - 1) / n > 65535 || (num_pix + n - 1) / n * (C / emc::kRTile) > 1L << 22)) n *= 2;
@@ -682,6 +682,12 @@ size_t round_up(size_t a, size_t b) { return (a + b - 1) / b * b; }
 // least kHotUses photons of a block's frames on average (fewer uses do not pay for the row's own
 // read), kHotRows at most. hot_num stays 0 where fewer than kLeastHotRows would, or without room for
 // the lists. Parts of 128 frames: with 512 the 30,000 frames took 21.0 ms instead of 19.1, 3000 0.34 and 0.30.
+// kHotUses matters for faint frames only. None, 1, 2, 3 and 6 uses, ms: 20,000 frames of 2 photons x 6300 0.75,
+// 0.71, 0.71, 0.71, 0.75; of 10 0.98, 1.01, 0.97, 0.94, 0.94; of 20 1.19, 1.18, 1.17, 1.14, 1.11; 15,000 frames x 6300 on
+// 66,820 pixels of 10 photons 0.91, 1.00, 0.93, 0.90, 0.91; of 20 1.14, 1.25, 1.21, 1.18, 1.13; from 60 photons on all
+// four alike (2.2, none 2.3). kLeastHotRows: none, 8, 16, 32, 64 rows and as many as fit: 2111 frames x 6480
+// 0.49, 0.51, 0.49, 0.45, 0.40, 0.37; 20,000 x 6300 3.80, 3.76, 3.59, 3.32, 2.92, 2.61; 15,000 x 6300 of 187 photons 6.44, 6.39,
+// 6.31, 6.19, 6.10, 5.90.
 constexpr int kHotUses = 3, kLeastHotRows = 32, kFramesPerHotPart = 128, kHotParts = 64;
 int build_hot_lists(emc_engine *e) {
     const int N = e->num_data, P = e->num_pix;
@@ -1729,7 +1735,7 @@ int maximize_subset(emc_engine *e, const emc_iter_opts *opts, emc_iter_stats *st
         }
         // the full frames' significant rows go to the pair tomogram directly when they average
         // at most sig_full_rows a tile (its blocks walk every row of their tile); else
-        // their tomogram is the plain path's, into partial views (also inside a graph, which
+        // their tomogram is the plain path's, into sums that the pair tomogram takes over (also in a graph, which
         // cannot read the count back)
         bool sig_full = false;
         if (nF > 0 && !device_weights) {

@@ -211,7 +211,7 @@ void launch_merge_bricks(hipStream_t s, const int4 *units, int num_units, const 
                          const double *corr, const uint8_t *mask, int num_pix, long size, int npatch, int nbx,
                          double *model2, double *weight, int do_model, int do_weight,
                          const int *gate = nullptr, const unsigned long long *nzmask = nullptr);
-// model-only merge with FP32 brick sums from an FP32 view (nzmask: as launch_merge_bricks')
+// model-only merge from an FP32 view (nzmask: as launch_merge_bricks')
 void launch_merge_model_f32(hipStream_t s, const int4 *units, int num_units, const int *list,
                             const unsigned long long *lmask, const double *rots, int r0, int num_rot,
                             const float *view, const double *psum_r, int all_on, const double *qvals,

@@ -1059,9 +1059,9 @@ __global__ void copy_brick_kernel(const double *__restrict__ in, long size, int 
 }
 
 // From 160^3: there a model passes the L2 of an XCD several times and the copy pays. Expand stage from
-// model1 and from the copy, ms: 10,880 orientations on 251^3 5.93, 4.94 (in FP16 rows 6.1, 5.5), 25,680 slots of
-// refinement subsets 12.6, 11.0, 10,880 on 185^3 2.69, 2.40; on 125^3 0.78, 0.78 (6300) and 0.43, 0.43 (3240), on 77^3
-// 0.27, 0.28. The copy of 251^3 (158 MB) takes 0.1 ms.
+// model1 and from the copy, ms: 10,880 orientations on 251^3 5.74, 4.54 (in FP16 rows 5.82, 5.17), 25,680 slots of
+// refinement subsets 12.1, 10.2, 10,880 on 185^3 2.64, 2.24; on 125^3 0.78, 0.78 (6300) and 0.43, 0.43 (3240), on 77^3
+// 0.27, 0.28 (the smaller sizes with an earlier logarithm). The copy of 251^3 (158 MB) takes 0.1 ms.
 size_t brick_copy_elems(long size, int modes) {
     const size_t n = size >= 160 ? BrickLayout(size).elems() : 0;
     return n < ((size_t)1 << 31) ? n * modes : 0;

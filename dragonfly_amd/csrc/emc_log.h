@@ -9,7 +9,8 @@
 // keeps its relative precision. log1p(r) is r plus its series, |r| < 2^-7; r joins the high part with its
 // rounding error kept, and everything small is added to that sum last: one rounding is left.
 // Against 80-bit logarithms of 30 million values: at most 0.51 ulp, 0.25 on average
-// (the device library's log: 0.64).
+// (the device library's log: 0.64). FP64 expand with the library's and with this, ms: 10,880 orientations x
+// 66,820 pixels 5.2, 4.5; 10,880 x 38,190 2.9, 2.2; 6300 x 22,801 0.93, 0.74; the same as FP16 rows, 10,880 x 66,820 5.8, 5.2.
 #pragma once
 
 #include <cmath>

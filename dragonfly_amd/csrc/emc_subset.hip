@@ -1066,8 +1066,9 @@ static void pair_tomogram_launch(hipStream_t s, const TP *P, const long *tile_of
                                  int ntiles, int num_pix, const PT *partial, VT *view,
                                  unsigned long long *nzmask, const SigFullRows &fr, const PairBuckets &bk) {
     if (ntiles <= 0) return;
-    // quarter patches where the lists are long enough to fill them (64 photons a block): with 190
-    // photons a quarter the stage takes 15.1 ms, 19.6 by whole patches; with 5, 2.0 against 1.8
+    // quarter patches where the lists are long enough to fill them (64 photons a block). The stage by
+    // quarters and by whole patches, ms: 119 photons a quarter 14.9, 19.7 (25,680 slots, 66,820 pixels); 60 8.3, 10.1;
+    // 29 5.0, 5.7; 12 3.2, 3.3 (FP32 gathers 3.6, 3.3); 5 2.0, 1.8. So the line is on the safe side of the crossing
     const bool quarter = bk.base && bk.sub == 4 && bk.per_tile >= 64L * bk.nr;
     const int nr = quarter ? bk.nr : nranges;
     // a block a (tile, range): 257,000 slots x 66,820 pixels in quarter patches are past a grid's 32 bits

@@ -18,8 +18,8 @@
 // Why: a pixel's frames are spread over the whole data set, so rows are only read at L2 speed
 // while the XCD's 4 MB L2 holds the tile's rows of every frame: 128 bytes a frame, where the
 // 64-orientation rows of the posterior itself need 512 (and 128-byte pieces of those would use a
-// quarter of the L2's sets). kFramesPerTomoRange bounds the frames of one launch; more frames
-// take several launches, each adding to the view of the one before. Equal pieces of a unit's list
+// quarter of the L2's sets). More than kFramesPerTomoRange frames take several launches, each adding to
+// the view of the one before (as many as option tomo_parts allows, then with more frames each). Equal pieces of a unit's list
 // and units of bounded photons, because pixels differ a thousandfold in photons (the 64 brightest
 // can hold a quarter of all): a block that takes several times a tile's time lets the XCD go on to
 // further tiles, whose rows then share its L2. Before, eight frame ranges wrote eight partial

@@ -77,7 +77,7 @@ def test_roofline_of_the_judged_iteration_units():
     st = out['stages']
     assert st['expand']['compulsory_bytes'] == 512 * 27 + 4 * 64 * 64
     assert st['expand']['frac'] == pytest.approx(60.416 / 8000., abs=1e-4)
-    # no fall-back frames: the pair tomogram reads no partial views
+    # no fall-back frames: the pair tomogram reads no sums
     assert st['reduce']['compulsory_bytes'] == 12 * 500 + 8 * 64 + 4 * 10 ** 9
     assert st['tomogram']['frac'] is None
 

@@ -187,7 +187,7 @@ def test_cfg4_geometry_fused_graph_equals_eager():
     with the persistent expand + likelihood kernel and captured as a HIP graph against the
     separate launches run eagerly, two iterations through the model update (the second replays
     the graph on the updated model and scales). Per-frame results equal; the merged and updated
-    volumes to the FP32 brick sums' order."""
+    volumes to the order of the brick sums."""
     from dragonfly_amd import _lib, synth
     print('case: cfg4 geometry, fused + graph, 3000 frames', flush=True)
     prob = synth.make_problem('cfg4', device='cuda', num_data=3000, batch=1024)

@@ -177,7 +177,7 @@ def test_fp32_gathers_refinement_subsets(variant, monkeypatch):
     (every cell) and an empty set, in 128-slot chunks (or one), against the oracle's refinement
     branch (tolerances of the FP32 gathers above); also with each kernel variant of the sparse
     M-step: the pair tomogram walking its tiles' pairs instead of per-(tile, range) buckets,
-    the full frames through partial views or read directly, merge units of 64 entries."""
+    the full frames through their own sums or read directly, merge units of 64 entries."""
     import os
     from oracle import core
     env = {'no-buckets': {'EMC_TOMO_BUCKETS': '0'}, 'full-parts': {'EMC_SIG_FULL_ROWS': '0'},

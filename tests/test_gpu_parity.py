@@ -242,7 +242,7 @@ def test_dense_integer_frames(tiny, zero_block):
 # kernel-variant options of the subset path's M-step (start values from EMC_<NAME>)
 SUBSET_VARIANTS = {
     'no-buckets': {'EMC_TOMO_BUCKETS': '0'},                # pair tomogram walks its tiles' pairs
-    'full-parts': {'EMC_SIG_FULL_ROWS': '0'},               # full frames through partial views
+    'full-parts': {'EMC_SIG_FULL_ROWS': '0'},               # full frames through their own sums
     'full-direct': {'EMC_SIG_FULL_ROWS': str(1 << 20)},     # full frames' rows read directly
     'full-parts-no-buckets': {'EMC_SIG_FULL_ROWS': '0', 'EMC_TOMO_BUCKETS': '0'},
     'small-units': {'EMC_UNIT_ITEMS': '64'},                # merge units of 64 list entries
