@@ -25,17 +25,17 @@ def tune(engine, iteration=1, need_scaling=0, known_scale=0, space=PLAIN_SPACE, 
     """Tune `engine` in place. Returns {option: chosen value} and the timings
     {option: {value: ms}}. Every candidate runs one full maximize (model2, inter_weight and
     the per-frame outputs are overwritten; scale factors are left alone). An option that the
-    kernels of the last iteration do not read is left as it is."""
+    kernels of its first candidate's run do not read stays at that candidate."""
     chosen, timings = {}, {}
     in_use = getattr(engine, 'option_in_use', lambda name: True)
     for name, values, stages in space:
-        if not in_use(name):
-            continue
         times = {}
         for v in values:
             engine.set_option(name, v)
             st = engine.maximize(iteration, need_scaling, 0, known_scale)
             times[v] = sum(st['stage_ms'][s] for s in stages)
+            if not in_use(name):
+                break
         best = min(times, key=times.get)
         engine.set_option(name, best)
         chosen[name] = best
