@@ -198,7 +198,8 @@ def likelihood_kernel(engine):
 
 def roofline(prob, itr, stage_tot, steps, nchunks, pairs, workload, lik_kernel, value_bytes=8):
     """HBM roofline of the dominant photon kernel (likelihood or tomogram gather, whichever
-    takes longer), timed with HIP events on the engine's stream.
+    takes longer), timed with HIP events on the engine's stream. A launch is the kernel's share of
+    one orientation chunk (the tomogram's launches, one a frame range, together).
 
     `achieved` counts compulsory bytes: every operand of one launch moved once -- for the
     likelihood (`lik_kernel`) the log W chunk (8 B per orientation x pixel), the frames' photon
